@@ -23,6 +23,7 @@
 // The whole kernel runs in round-toward-+inf (see vcphip_device.h).
 #include "vcphip_device.h"
 #include "vcphip_kernels.h"
+#include "vcphip_thin.h"
 
 namespace {
 
@@ -589,40 +590,94 @@ __global__ __launch_bounds__(NT, 2) void k_igemm_tiles(int ntiles, const VcphipR
   }
 }
 
-// row sums of |C| (upward, in column order: mats::norminf, vcp/mats.hpp:1583-1591)
-__global__ __launch_bounds__(256) void k_resid_rowsum(int nrows, const int* __restrict__ row_problem,
-                                                      const VcphipResidProblem* __restrict__ probs,
-                                                      double* __restrict__ rowsum) {
-  vcphip_mode_round_up();
-  const int g = blockIdx.x * 256 + threadIdx.x;
-  if (g >= nrows) return;
-  const int pi = row_problem[g];
-  const VcphipResidProblem p = probs[pi];
-  const int i = g - p.row_base;
-  const double* row = p.C + 2 * (long)i;
-  const long step = 2 * (long)p.ldc;
-  // the upward sum runs in column order, as the reference's; a thread per
-  // row is few waves per SIMD, so the loads of 32 columns are issued ahead of
-  // their additions
-  constexpr int U = 32;
-  double s = 0.0;
-  int j = 0;
-  for (; j + U <= p.n; j += U) {
-    double2 v[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) v[u] = *reinterpret_cast<const double2*>(row + step * (j + u));
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const double mag = fmax(__builtin_fabs(v[u].x), __builtin_fabs(v[u].y));
-      s = (j + u == 0) ? mag : s + mag;
+// ---------------------------------------------------------------------------
+// The single products with few columns, or too small to fill the device with
+// tiles: the row-serial form of vcphip_thin.h, one launch straight from the
+// AoS operands.
+// ---------------------------------------------------------------------------
+template <bool AI, bool BI>
+struct ThinProduct : VcphipThinDr<AI, BI> {
+  using Base = VcphipThinDr<AI, BI>;
+  double* __restrict__ C;
+  double* __restrict__ C2;
+  long ldc;
+  int accumulate, m, n;
+  VCPHIP_DEVINL void init(typename Base::Acc& c, int row, int col) const {
+    Base::init(c, row, col);
+    if (!AI && !BI && accumulate && row < m && col < n) {
+      c.up = C[row + ldc * col];
+      c.dn = -C2[row + ldc * col];
     }
   }
-  for (; j < p.n; ++j) {
-    const double2 v = *reinterpret_cast<const double2*>(row + step * j);
-    const double mag = fmax(__builtin_fabs(v.x), __builtin_fabs(v.y));
-    s = (j == 0) ? mag : s + mag;
+  VCPHIP_DEVINL void done(const typename Base::Acc& c, int row, int col) const {
+    if (AI || BI) {
+      *reinterpret_cast<double2*>(C + 2 * (row + ldc * col)) = this->result(c);
+    } else {
+      C[row + ldc * col] = c.up;
+      C2[row + ldc * col] = -c.dn;
+    }
   }
-  rowsum[g] = s;
+};
+
+template <bool AI, bool BI, int CW, int CPT>
+__global__ __launch_bounds__((VcphipThin<ThinProduct<AI, BI>, CW, CPT>::NT)) __attribute__((amdgpu_waves_per_eu(1, 2))) void k_drgemm_thin(int m, int n, int k, const double* __restrict__ A, long lda,
+                                                     const double* __restrict__ B, long ldb, double* __restrict__ C,
+                                                     long ldc, double* __restrict__ C2, int accumulate) {
+  vcphip_mode_round_up();
+  using T = VcphipThin<ThinProduct<AI, BI>, CW, CPT>;
+  __shared__ __attribute__((aligned(16))) typename T::Lds lds;
+  ThinProduct<AI, BI> op;
+  op.A = A;
+  op.B = B;
+  op.lda = lda;
+  op.ldb = ldb;
+  op.C = C;
+  op.C2 = C2;
+  op.ldc = ldc;
+  op.accumulate = accumulate;
+  op.m = m;
+  op.n = n;
+  const int rb = vcphip_xcd_remap(blockIdx.x, gridDim.x);
+  T::run(op, lds, m, n, k, rb * T::R, blockIdx.y * T::NC, (int)((blockIdx.x >> 8) % T::NW));
+}
+
+// row sums of |C| (upward, in column order: mats::norminf, vcp/mats.hpp:
+// 1583-1591) over 8-row blocks of the problems, in the row-serial form: each
+// C_p is read once at a cache line per row block and column (a thread per row
+// and wave-wide row blocks kept too few loads in flight: 153 against XX us
+// for 64 problems of n in [64, 1024])
+struct ResidRowSum {
+  static constexpr bool A2 = true, B2 = false, PAD16 = false;
+  static constexpr int AL = 1, BL = 0;
+  const double* A;
+  const double* B = nullptr;
+  long lda, ldb = 0;
+  double* out;
+  struct Acc {
+    double s;
+  };
+  VCPHIP_DEVINL double2 a(double2 v, int, int) const {
+    return make_double2(fmax(__builtin_fabs(v.x), __builtin_fabs(v.y)), 0.0);
+  }
+  VCPHIP_DEVINL double2 b(double2 v) const { return v; }
+  VCPHIP_DEVINL void init(Acc& c, int, int) const { c.s = 0.0; }
+  VCPHIP_DEVINL void step(Acc& c, double2 av, double2) const { c.s = c.s + av.x; }
+  VCPHIP_DEVINL void done(const Acc& c, int row, int) const { out[row] = c.s; }
+};
+
+__global__ __launch_bounds__((VcphipThin<ResidRowSum, 1>::NT)) __attribute__((amdgpu_waves_per_eu(1, 2)))
+void k_resid_rowsum(const VcphipResidTile* __restrict__ blocks, const VcphipResidProblem* __restrict__ probs,
+                    double* __restrict__ rowsum) {
+  vcphip_mode_round_up();
+  using T = VcphipThin<ResidRowSum, 1>;
+  __shared__ __attribute__((aligned(16))) typename T::Lds lds;
+  const VcphipResidTile tl = blocks[vcphip_xcd_remap(blockIdx.x, gridDim.x)];
+  const VcphipResidProblem p = probs[tl.problem];
+  ResidRowSum op;
+  op.A = p.C;
+  op.lda = p.ldc;
+  op.out = rowsum + p.row_base;
+  T::run(op, lds, p.n, 1, p.n, tl.row0, 0, (int)((blockIdx.x >> 8) % T::NW));
 }
 
 // ||C_p||_inf upper bound: the largest row sum (mats.hpp:1592-1598).  One
@@ -1090,6 +1145,42 @@ int vcphip_launch_drgemm(int kind, int m, int n, int k, const double* A, long ld
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
+int vcphip_launch_drgemm_thin(int kind, int m, int n, int k, const double* A, long lda, const double* B, long ldb,
+                              double* C, long ldc, double* C2, int accumulate, hipStream_t s) {
+  if (m <= 0 || n <= 0) return 0;
+  if (k <= 0) return -1;   // k = 0 takes the tile path
+  // columns of a workgroup: few right-hand sides take the narrow shapes; else
+  // the widest (64, the fewest LDS reads per multiply-add) that still gives
+  // about 150 workgroups (n = k = m = 300: 19 us with 64, 24 with 32, 30 with
+  // 8 columns; 96 x 80 x 160: 12, 8.5 and 6 us)
+  const long rb = ((long)m + VCPHIP_THIN_R - 1) / VCPHIP_THIN_R;
+  int nc = n <= 8 ? 8 : n <= 16 ? 16 : 64;
+  while (nc > 8 && n > 16 && rb * ((n + nc - 1) / nc) < 150) nc /= 2;
+  const long cg = ((long)n + nc - 1) / nc;
+  if (cg > 65535 || rb > 0x7FFFFFFF) return -7;
+  const dim3 grid((unsigned)rb, (unsigned)cg);
+#define VCPHIP_THIN_SHAPE(AI, BI, CW, CPT)                                                                        \
+  hipLaunchKernelGGL((k_drgemm_thin<AI, BI, CW, CPT>), grid, dim3((VcphipThin<ThinProduct<AI, BI>, CW, CPT>::NT)), \
+                     0, s, m, n, k, A, lda, B, ldb, C, ldc, C2, accumulate)
+#define VCPHIP_THIN_CASE(KIND, AI, BI)                    \
+  case KIND:                                              \
+    if (nc == 8) VCPHIP_THIN_SHAPE(AI, BI, 1, 1);         \
+    else if (nc == 16) VCPHIP_THIN_SHAPE(AI, BI, 2, 1);   \
+    else if (nc == 32) VCPHIP_THIN_SHAPE(AI, BI, 4, 1);   \
+    else VCPHIP_THIN_SHAPE(AI, BI, 4, 2);                 \
+    break;
+  switch (kind) {
+    VCPHIP_THIN_CASE(VCPHIP_DR_II, true, true)
+    VCPHIP_THIN_CASE(VCPHIP_DR_IP, true, false)
+    VCPHIP_THIN_CASE(VCPHIP_DR_PI, false, true)
+    VCPHIP_THIN_CASE(VCPHIP_DR_PP, false, false)
+    default: return -1;
+  }
+#undef VCPHIP_THIN_CASE
+#undef VCPHIP_THIN_SHAPE
+  return hipGetLastError() == hipSuccess ? 0 : -3;
+}
+
 int vcphip_launch_planes(int kind, int m, int n, int k, const double* A, long lda, const double* B, long ldb,
                          double* A0, double* A1, double* B0, double* B1, hipStream_t s) {
   const int mpad = (m + BM - 1) / BM * BM, npad = (n + BN - 1) / BN * BN, kpad = (k + BK - 1) / BK * BK;
@@ -1179,11 +1270,12 @@ int vcphip_launch_resid_tiles(int n64, int n32, const VcphipResidTile* tiles, co
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
-int vcphip_launch_resid(int n64, int n32, const VcphipResidTile* tiles, const VcphipResidProblem* probs, int nrows,
-                        const int* row_problem, double* rowsum, int count, double* normub, int grid64, int grid32,
-                        unsigned* queue, hipStream_t s) {
+int vcphip_launch_resid(int n64, int n32, const VcphipResidTile* tiles, const VcphipResidProblem* probs, int nblk,
+                        const VcphipResidTile* row_block, double* rowsum, int count, double* normub, int grid64,
+                        int grid32, unsigned* queue, hipStream_t s) {
   vcphip_launch_resid_tiles(n64, n32, tiles, probs, grid64, grid32, queue, s);
-  if (nrows > 0) hipLaunchKernelGGL(k_resid_rowsum, dim3((nrows + 255) / 256), dim3(256), 0, s, nrows, row_problem, probs, rowsum);
+  if (nblk > 0)
+    hipLaunchKernelGGL(k_resid_rowsum, dim3(nblk), dim3(VcphipThin<ResidRowSum, 1>::NT), 0, s, row_block, probs, rowsum);
   if (count > 0) hipLaunchKernelGGL(k_resid_max, dim3(count), dim3(256), 0, s, count, probs, rowsum, normub);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }

@@ -82,6 +82,13 @@ VCPHIP_DEVINL void vcphip_mode_round_up() {
   asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 4), 5" ::: "memory");
 }
 
+// back to round-to-nearest; what the code after it computes must come from
+// values loaded after it, and what it computed before it must be stored
+// before it (the memory clobber orders both)
+VCPHIP_DEVINL void vcphip_mode_nearest() {
+  asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 4), 0" ::: "memory");
+}
+
 // 2^e as a double for e in [-1022, 1023] (bit construction, exact)
 VCPHIP_DEVINL double vcphip_pow2(int e) {
   return __longlong_as_double((long long)(e + 1023) << 52);

@@ -49,7 +49,7 @@ struct vcphip_ctx {
   struct Resid {
     std::vector<VcphipResidProblem> probs;
     std::vector<VcphipResidTile> tiles;
-    std::vector<int> row_problem;
+    std::vector<VcphipResidTile> row_block;   // blocks of 8 rows, for the row sums
     double* normub = nullptr;
     hipStream_t stream = nullptr;
     hipGraph_t graph = nullptr;
@@ -57,11 +57,7 @@ struct vcphip_ctx {
     int n64 = 0, n32 = 0;       // tiles of each shape (64 x 64 first in the tile array)
     int grid = 0, grid32 = 0;   // persistent grids of the two tile launches
     // device descriptors of the cached set (for re-timing by the tuner)
-    const VcphipResidTile* dt = nullptr;
     const VcphipResidProblem* dp = nullptr;
-    const int* drp = nullptr;
-    double* drs = nullptr;
-    int nrows = 0;
   } resid;
   int num_cu = 0;
   // autotuner table: choices per product kind and size class (ceil(log2) of
@@ -834,6 +830,21 @@ int plane_rows(const vcphip_ctx* c, int kind, size_t mpad, size_t npad) {
   return (mpad / 64) * (npad / 64) <= per_cu * cus ? 32 : 64;
 }
 
+// Whether a single product takes the row-serial form (one launch, 8 rows per
+// workgroup) rather than planes and tiles: with few columns the tiles are
+// mostly padding (m = k = 4000, interval x point: 4 columns 77 against 470 us,
+// 32 columns 131 against 472 us, 64 columns 250 against 474 us, where tiles
+// start to pay once other work shares the device), and while the 8 x 64
+// blocks number at most one per CU the 32 x 64 tiles leave most CUs idle
+// (interval x interval, n = k = m = 96: 6 against 27 us, 300: 19 against 46,
+// 400: 38 against 62, but 512 at half the tiles' throughput when products on
+// several streams fill the device).  A forced plane shape takes the planes.
+bool thin_product(const vcphip_ctx* c, size_t m, size_t n) {
+  if (c->plane_rows) return false;
+  const size_t cus = c->num_cu > 0 ? (size_t)c->num_cu : 256;
+  return n <= 32 || ((m + 7) / 8) * ((n + 63) / 64) <= cus;
+}
+
 // A single product of kind VCPHIP_DR_*: the operand planes (midpoint and
 // radius of an interval operand, the point operand itself), padded and laid
 // out for whole k-slices, then the product from them.  k = 0 (an all-zero or,
@@ -844,6 +855,12 @@ int planes_product(vcphip_ctx* c, int kind, int m, int n, int k, const double* A
   if (k == 0) {
     const int rc =
         check_launch(vcphip_launch_drgemm(kind, m, n, k, A, lda, B, ldb, C, ldc, C2, accumulate, c->stream));
+    T.mark("drgemm");
+    return rc;
+  }
+  if (thin_product(c, (size_t)m, (size_t)n)) {
+    const int rc =
+        check_launch(vcphip_launch_drgemm_thin(kind, m, n, k, A, lda, B, ldb, C, ldc, C2, accumulate, c->stream));
     T.mark("drgemm");
     return rc;
   }
@@ -1360,12 +1377,13 @@ extern "C" int vcphip_residual_batched_dev(vcphip_ctx* c, int count, const int* 
     rs.grid = batch_grid(c, ts.t64.size(), c->resid_per_cu);
     rs.grid32 = batch_grid(c, ts.t32.size(), c->resid_per_cu);
     rs.tiles = tile_array(ts);
-    rs.row_problem.assign((size_t)nrows, 0);
+    rs.row_block.clear();
     for (int i = 0; i < count; ++i)
-      for (int r = 0; r < probs[i].n; ++r) rs.row_problem[(size_t)probs[i].row_base + r] = i;
+      for (int r = 0; r < probs[i].n; r += 8) rs.row_block.push_back(VcphipResidTile{i, r, 0, 0});
+    const int nblk = (int)rs.row_block.size();
     rs.probs = probs;
     const size_t bp = sizeof(VcphipResidProblem) * count, bt = sizeof(VcphipResidTile) * rs.tiles.size();
-    const size_t br = sizeof(int) * (size_t)nrows, bs = sizeof(double) * (size_t)nrows;
+    const size_t br = sizeof(VcphipResidTile) * (size_t)nblk, bs = sizeof(double) * (size_t)nrows;
     const size_t o_t = (bp + 255) & ~(size_t)255, o_r = o_t + ((bt + 255) & ~(size_t)255);
     const size_t o_s = o_r + ((br + 255) & ~(size_t)255), total = o_s + bs + 256;
     void* base;
@@ -1374,7 +1392,7 @@ extern "C" int vcphip_residual_batched_dev(vcphip_ctx* c, int count, const int* 
     char* b8 = (char*)base;
     if (hipMemcpyAsync(b8, rs.probs.data(), bp, hipMemcpyHostToDevice, c->stream) != hipSuccess ||
         (bt && hipMemcpyAsync(b8 + o_t, rs.tiles.data(), bt, hipMemcpyHostToDevice, c->stream) != hipSuccess) ||
-        (br && hipMemcpyAsync(b8 + o_r, rs.row_problem.data(), br, hipMemcpyHostToDevice, c->stream) != hipSuccess))
+        (br && hipMemcpyAsync(b8 + o_r, rs.row_block.data(), br, hipMemcpyHostToDevice, c->stream) != hipSuccess))
       return VCPHIP_ERR_DEVICE;
     if (rs.exec) { hipGraphExecDestroy(rs.exec); rs.exec = nullptr; }
     if (rs.graph) { hipGraphDestroy(rs.graph); rs.graph = nullptr; }
@@ -1383,13 +1401,9 @@ extern "C" int vcphip_residual_batched_dev(vcphip_ctx* c, int count, const int* 
     // capture the persistent launches and the norm kernels once; replays reuse them
     const VcphipResidTile* dt = (const VcphipResidTile*)(b8 + o_t);
     const VcphipResidProblem* dp = (const VcphipResidProblem*)b8;
-    const int* drp = (const int*)(b8 + o_r);
+    const VcphipResidTile* drp = (const VcphipResidTile*)(b8 + o_r);
     double* drs = (double*)(b8 + o_s);
-    rs.dt = dt;
     rs.dp = dp;
-    rs.drp = drp;
-    rs.drs = drs;
-    rs.nrows = nrows;
     unsigned* queue = batch_queue(c);
     if (!queue) {
       rs.probs.clear();
@@ -1397,11 +1411,11 @@ extern "C" int vcphip_residual_batched_dev(vcphip_ctx* c, int count, const int* 
     }
     bool captured = false;
     if (hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal) == hipSuccess) {
-      const int lrc = vcphip_launch_resid(rs.n64, rs.n32, dt, dp, nrows, drp, drs, count, normub_dev, rs.grid,
+      const int lrc = vcphip_launch_resid(rs.n64, rs.n32, dt, dp, nblk, drp, drs, count, normub_dev, rs.grid,
                                           rs.grid32, queue, c->stream);
       hipGraph_t g = nullptr;
       if (hipStreamEndCapture(c->stream, &g) == hipSuccess && lrc == 0 && g &&
-          graph_has_kernels(g, (size_t)vcphip_resid_kernels(rs.n64, rs.n32, nrows, count))) {
+          graph_has_kernels(g, (size_t)vcphip_resid_kernels(rs.n64, rs.n32, nblk, count))) {
         if (hipGraphInstantiate(&rs.exec, g, nullptr, nullptr, 0) == hipSuccess) {
           rs.graph = g;
           captured = true;
@@ -1418,7 +1432,7 @@ extern "C" int vcphip_residual_batched_dev(vcphip_ctx* c, int count, const int* 
       // a stream that cannot be captured (e.g. the legacy null stream) runs
       // the same kernels as direct launches
       StageTimer T(c);
-      const int lrc = vcphip_launch_resid(rs.n64, rs.n32, dt, dp, nrows, drp, drs, count, normub_dev, rs.grid,
+      const int lrc = vcphip_launch_resid(rs.n64, rs.n32, dt, dp, nblk, drp, drs, count, normub_dev, rs.grid,
                                           rs.grid32, queue, c->stream);
       T.mark("resid");
       rs.probs.clear();   // nothing cached to replay
@@ -1911,16 +1925,15 @@ extern "C" int vcphip_lss_dev(vcphip_ctx* c, int n, int nrhs, const double* IA, 
   hipStream_t s = c->stream;
   const size_t nr = (size_t)n * nrhs, al = 32;   // 256-byte alignment in doubles
   auto up = [&](size_t x) { return (x + al - 1) / al * al; };
-  const size_t o_mb = 0, o_mx = o_mb + up(nr), o_x = o_mx + up(nr), o_y = o_x + up(2 * nr), o_t = o_y + up(2 * nr);
-  const size_t o_w = o_t + up(2 * nr), o_c = o_w + up(2 * nr), o_r = o_c + up(2 * (size_t)n * n);
+  const size_t o_mx = 0, o_x = o_mx + up(nr), o_y = o_x + up(2 * nr), o_c = o_y + up(2 * nr);
+  const size_t o_r = o_c + up(2 * (size_t)n * n);
   const size_t np = (size_t)inv_order(n);
   const size_t o_s = o_r + up((size_t)n), o_ri = o_s + al, total = o_ri + (R ? 0 : up(inv_work_doubles(n)));
   void* base;
   const int wrc = ws_get(c, vcphip_ctx::WS_LSS, total * sizeof(double), &base);
   if (wrc) return wrc;
   double* w = (double*)base;
-  double *mb = w + o_mb, *mx = w + o_mx, *Xi = w + o_x, *Y = w + o_y, *Tm = w + o_t, *W = w + o_w, *C = w + o_c;
-  double *rows = w + o_r, *norms = w + o_s;   // norms: g, T, G lower, G upper
+  double *C = w + o_c, *rows = w + o_r, *norms = w + o_s;   // norms: g, T, G lower, G upper
   StageTimer T(c);
   // R = inv(mid(IA)) on the device when the caller gives none (:298-301)
   InvBatch inv;
@@ -1935,28 +1948,41 @@ extern "C" int vcphip_lss_dev(vcphip_ctx* c, int n, int nrhs, const double* IA, 
     ldr = (int)np;
     T.mark("lss_inv");
   }
+  VcphipLssProblem P = {};
+  P.A = IA;
+  P.b = Ib;
+  P.R = R;
+  P.X = X;
+  P.lda = lda;
+  P.ldb = ldb;
+  P.ldr = ldr;
+  P.ldx = ldx;
+  P.n = n;
+  P.nrhs = nrhs;
+  P.mx = w + o_mx;
+  P.xi = w + o_x;
+  P.y = w + o_y;
+  P.C = C;
+  P.norms = norms;
   int rc = 0;
-  // mx = R * mid(b), nearest rounding (:299-302)
-  rc |= vcphip_lss_launch_mid(n, nrhs, Ib, ldb, mb, n, s);
-  rc |= vcphip_lss_launch_gemv_rn(n, nrhs, n, R, ldr, mb, n, mx, n, s);
-  // y = R * (IA*mx - b) and |y| (:305-315)
-  rc |= vcphip_launch_drgemm(VCPHIP_DR_IP, n, nrhs, n, IA, lda, mx, n, Xi, n, nullptr, 0, s);
-  rc |= vcphip_lss_launch_sub(n, nrhs, Xi, n, Ib, ldb, s);
-  rc |= vcphip_launch_drgemm(VCPHIP_DR_PI, n, nrhs, n, R, ldr, Xi, n, Y, n, nullptr, 0, s);
-  rc |= vcphip_lss_launch_abs(n, nrhs, Y, n, s);
+  // mx = R * mid(b), nearest rounding (:299-302); y = |R * (IA*mx - b)| (:305-315)
+  rc |= vcphip_lss_launch_mx(P, s);
+  if (thin_product(c, (size_t)n, (size_t)nrhs)) {
+    rc |= vcphip_lss_launch_ax(P, s);
+    rc |= vcphip_lss_launch_ry(P, s);
+  } else {   // many right-hand sides: the tiled products and elementwise steps
+    rc |= planes_product(c, VCPHIP_DR_IP, n, nrhs, n, IA, lda, P.mx, n, P.xi, n) ? 1 : 0;   // on s, the context stream
+    rc |= vcphip_lss_launch_sub(n, nrhs, P.xi, n, Ib, ldb, s);
+    rc |= planes_product(c, VCPHIP_DR_PI, n, nrhs, n, R, ldr, P.xi, n, P.y, n) ? 1 : 0;
+    rc |= vcphip_lss_launch_abs(n, nrhs, P.y, n, s);
+  }
   T.mark("lss_rhs");
-  // R*IA - I and g = ||R*IA - I||_inf (:318-329)
-  rc |= planes_product(c, VCPHIP_DR_PI, n, n, n, R, ldr, IA, lda, C, n) ? 1 : 0;   // on s, the context stream
-  rc |= vcphip_lss_launch_diag(n, C, n, s);
-  rc |= vcphip_lss_launch_norm(n, n, C, n, rows, norms, s);
+  // R*IA (:318); the diagonal is taken off where it is read
+  rc |= planes_product(c, VCPHIP_DR_PI, n, n, n, R, ldr, IA, lda, C, n) ? 1 : 0;
   T.mark("lss_resid");
-  // T = ||y||_inf, G = T / (1 - g), |R*IA - I| * G (:334-350)
-  rc |= vcphip_lss_launch_norm(n, nrhs, Y, n, rows, norms + 1, s);
-  rc |= vcphip_lss_launch_abs(n, n, C, n, s);
-  rc |= vcphip_lss_launch_fill_g(n, nrhs, norms, Tm, n, norms + 2, s);
-  rc |= vcphip_launch_drgemm(VCPHIP_DR_II, n, nrhs, n, C, n, Tm, n, W, n, nullptr, 0, s);
-  // X = mx + [-u, u], u = |y| + W (:352-361)
-  rc |= vcphip_lss_launch_final(n, nrhs, Y, W, mx, X, ldx, s);
+  // g = ||R*IA - I||_inf, T = ||y||_inf, G = T / (1 - g) (:319-341), then
+  // X = mx + [-u, u], u = |y| + |R*IA - I| * G (:343-361)
+  rc |= vcphip_lss_launch_bound(P, rows, s);
   T.mark("lss_bound");
   if (rc) {
     hipStreamSynchronize(s);
@@ -1977,7 +2003,7 @@ extern "C" int vcphip_lss_dev(vcphip_ctx* c, int n, int nrhs, const double* IA, 
 
 // Many systems of uneven size: R_p IA_p - I and its norm through the batched
 // residual (its persistent launch and graph), the other steps as one launch
-// each over the (row, column) items of all problems.
+// each over the row blocks of all problems.
 extern "C" int vcphip_lss_batched_dev(vcphip_ctx* c, int count, const int* n, const int* nrhs,
                                       const double* const* IA, const int* lda, const double* const* Ib,
                                       const int* ldb, const double* const* R, const int* ldr, double* const* X,
@@ -1997,25 +2023,25 @@ extern "C" int vcphip_lss_batched_dev(vcphip_ctx* c, int count, const int* n, co
   }
   hipSetDevice(c->device);
   hipStream_t s = c->stream;
-  // workspace: descriptors, item offsets, g and norms, then per problem
-  // mb, mx, xi, y (n x nrhs) and C (n x n intervals); 256-byte aligned
+  // workspace: descriptors, block offsets, g and norms, then per problem
+  // mx, xi, y (n x nrhs) and C (n x n intervals); 256-byte aligned
   auto al = [](size_t bytes) { return (bytes + 255) & ~(size_t)255; };
   const size_t o_pb = al(sizeof(VcphipLssProblem) * count);
   const size_t o_g = o_pb + al(sizeof(long) * (count + 1));
   const size_t o_nm = o_g + al(sizeof(double) * count);
   size_t off = o_nm + al(sizeof(double) * 4 * (size_t)count);
   std::vector<size_t> o_prob((size_t)count);
-  std::vector<long> pb((size_t)count + 1, 0);
+  std::vector<long> wb((size_t)count + 1, 0);   // blocks of 8 rows x 8 right-hand sides
   std::vector<size_t> o_rinv((size_t)count, 0);
   for (int p = 0; p < count; ++p) {
     const size_t nr = (size_t)n[p] * nrhs[p];
     o_prob[p] = off;
-    off += al(8 * nr) * 2 + al(16 * nr) * 2 + al(16 * (size_t)n[p] * n[p]);
+    off += al(8 * nr) + al(16 * nr) * 2 + al(16 * (size_t)n[p] * n[p]);
     if (!has_r(p)) {
       o_rinv[p] = off;
       off += al(8 * inv_work_doubles(n[p]));
     }
-    pb[p + 1] = pb[p] + (long)nr;
+    wb[p + 1] = wb[p] + (((long)n[p] + 7) / 8) * (((long)nrhs[p] + 7) / 8);
   }
   void* base;
   const int wrc = ws_get(c, vcphip_ctx::WS_LSSB, off, &base);
@@ -2052,11 +2078,10 @@ extern "C" int vcphip_lss_batched_dev(vcphip_ctx* c, int count, const int* n, co
     P.ldx = ldx[p];
     P.n = n[p];
     P.nrhs = nrhs[p];
-    P.mb = (double*)q;
-    P.mx = (double*)(q + al(8 * nr));
-    P.xi = (double*)(q + 2 * al(8 * nr));
-    P.y = (double*)(q + 2 * al(8 * nr) + al(16 * nr));
-    Cp[p] = (double*)(q + 2 * al(8 * nr) + 2 * al(16 * nr));
+    P.mx = (double*)q;
+    P.xi = (double*)(q + al(8 * nr));
+    P.y = (double*)(q + al(8 * nr) + al(16 * nr));
+    Cp[p] = (double*)(q + al(8 * nr) + 2 * al(16 * nr));
     P.C = Cp[p];
     P.normub = gdev + p;
     P.norms = (double*)(b8 + o_nm) + 4 * (size_t)p;
@@ -2070,7 +2095,7 @@ extern "C" int vcphip_lss_batched_dev(vcphip_ctx* c, int count, const int* n, co
     return code;
   };
   if (hipMemcpyAsync(b8, probs.data(), sizeof(VcphipLssProblem) * count, hipMemcpyHostToDevice, s) != hipSuccess ||
-      hipMemcpyAsync(b8 + o_pb, pb.data(), sizeof(long) * (count + 1), hipMemcpyHostToDevice, s) != hipSuccess)
+      hipMemcpyAsync(b8 + o_pb, wb.data(), sizeof(long) * (count + 1), hipMemcpyHostToDevice, s) != hipSuccess)
     return fail(VCPHIP_ERR_DEVICE);
   if (!c->aux) {
     if (hipStreamCreateWithFlags(&c->aux, hipStreamNonBlocking) != hipSuccess ||
@@ -2090,7 +2115,7 @@ extern "C" int vcphip_lss_batched_dev(vcphip_ctx* c, int count, const int* n, co
   }
   // right-hand side on the second stream, after the descriptor upload
   if (hipEventRecord(c->ev_fork, s) != hipSuccess || hipStreamWaitEvent(c->aux, c->ev_fork, 0) != hipSuccess ||
-      vcphip_lss_launch_batched_rhs(count, pb[count], dpb, dprobs, c->aux) ||
+      vcphip_lss_launch_batched_rhs(count, wb[count], dpb, dprobs, c->aux) ||
       hipEventRecord(c->ev_join, c->aux) != hipSuccess)
     return fail(VCPHIP_ERR_DEVICE);
   // R_p IA_p - I and g_p (imats.hpp:318-329) meanwhile on the context stream
@@ -2098,7 +2123,7 @@ extern "C" int vcphip_lss_batched_dev(vcphip_ctx* c, int count, const int* n, co
   if (rc) return fail(rc);
   StageTimer T(c);
   if (hipStreamWaitEvent(s, c->ev_join, 0) != hipSuccess ||
-      vcphip_lss_launch_batched_bound(count, pb[count], dpb, dprobs, s))
+      vcphip_lss_launch_batched_bound(count, wb[count], dpb, dprobs, s))
     return fail(VCPHIP_ERR_DEVICE);
   T.mark("lss_batched");
   if (hipMemcpyAsync(normub, gdev, sizeof(double) * count, hipMemcpyDeviceToHost, s) != hipSuccess)

@@ -23,6 +23,9 @@ int vcphip_launch_planes(int kind, int m, int n, int k, const double* A, long ld
 int vcphip_launch_drgemm_planes(int kind, int m, int n, int k, const double* A0, const double* A1, const double* B0,
                                 const double* B1, double* C, long ldc, double* C2, int accumulate, int rows,
                                 hipStream_t s);
+// the single products in the row-serial form (few columns or small sizes), k > 0
+int vcphip_launch_drgemm_thin(int kind, int m, int n, int k, const double* A, long lda, const double* B, long ldb,
+                              double* C, long ldc, double* C2, int accumulate, hipStream_t s);
 // A^T A (interval or point, A k x n) from the planes of A (made here into
 // P0 / P1, each kpad x npad doubles; P1 unused for a point A); k > 0
 int vcphip_launch_drsyrk_planes(int interval, int k, int n, const double* A, long lda, double* P0, double* P1,
@@ -64,17 +67,18 @@ struct VcphipIgemmProblem {
 // first; one pair per stream of launches)
 int vcphip_launch_igemm_tiles(int n64, int n32, const VcphipResidTile* tiles, const VcphipIgemmProblem* probs,
                               int grid64, int grid32, unsigned* queue, hipStream_t s);
-int vcphip_launch_resid(int n64, int n32, const VcphipResidTile* tiles, const VcphipResidProblem* probs, int nrows,
-                        const int* row_problem, double* rowsum, int count, double* normub, int grid64, int grid32,
-                        unsigned* queue, hipStream_t s);
+// row_block: the problems' blocks of 8 rows {problem, first row}
+int vcphip_launch_resid(int n64, int n32, const VcphipResidTile* tiles, const VcphipResidProblem* probs, int nblk,
+                        const VcphipResidTile* row_block, double* rowsum, int count, double* normub, int grid64,
+                        int grid32, unsigned* queue, hipStream_t s);
 // the tile launches alone (the tuner times them)
 int vcphip_launch_resid_tiles(int n64, int n32, const VcphipResidTile* tiles, const VcphipResidProblem* probs,
                               int grid64, int grid32, unsigned* queue, hipStream_t s);
 // the number of kernels vcphip_launch_resid / vcphip_launch_igemm_tiles
 // enqueue for these sizes
 inline int vcphip_igemm_tile_kernels(int n64, int n32) { return (n64 > 0 || n32 > 0) + (n64 > 0) + (n32 > 0); }
-inline int vcphip_resid_kernels(int n64, int n32, int nrows, int count) {
-  return vcphip_igemm_tile_kernels(n64, n32) + (nrows > 0) + (count > 0);
+inline int vcphip_resid_kernels(int n64, int n32, int nblk, int count) {
+  return vcphip_igemm_tile_kernels(n64, n32) + (nblk > 0) + (count > 0);
 }
 // p[0..n) = v by a kernel
 int vcphip_fill_f64(double* p, long n, double v, hipStream_t s);
@@ -220,25 +224,15 @@ int vcphip_gather_rows(const double* A, long lda, int m, int k, int s, double* o
 int vcphip_ratio_max(const double* X, const double* Y, long total, double* part, int nblocks, hipStream_t st);
 int vcphip_fill_random(void* p, size_t bytes, uint32_t seed, hipStream_t st);
 
-// verified linear solve: elementwise and scalar steps (kern_lss.hip)
-int vcphip_lss_launch_mid(int n, int ncol, const double* b, long ldb, double* mb, long ldm, hipStream_t s);
+// verified linear solve (kern_lss.hip)
 // approximate inverse: midpoint matrix bordered by the identity to order npad,
-// and the copy of its leading n x n block out (kern_lss.hip)
+// and the copy of its leading n x n block out
 int vcphip_inv_launch_pad(int n, int npad, const double* IA, long lda, double* P, hipStream_t s);
 int vcphip_inv_launch_copy(int n, const double* P, long ldp, double* R, long ldr, hipStream_t s);
-int vcphip_lss_launch_gemv_rn(int m, int ncol, int k, const double* A, long lda, const double* B, long ldb, double* C,
-                              long ldc, hipStream_t s);
 int vcphip_lss_launch_sub(int n, int ncol, double* X, long ldx, const double* b, long ldb, hipStream_t s);
 int vcphip_lss_launch_abs(int rows, int cols, double* X, long ldx, hipStream_t s);
-int vcphip_lss_launch_diag(int n, double* C, long ldc, hipStream_t s);
-int vcphip_lss_launch_norm(int rows, int cols, const double* X, long ldx, double* rowbuf, double* out,
-                           hipStream_t s);
-int vcphip_lss_launch_fill_g(int n, int ncol, const double* norms, double* Tm, long ldt, double* Gout,
-                             hipStream_t s);
-int vcphip_lss_launch_final(int n, int ncol, const double* Y, const double* W, const double* mx, double* X, long ldx,
-                            hipStream_t s);
 
-// batched verified solve: one problem's operands and its workspace
+// one system's operands and its workspace
 struct VcphipLssProblem {
   const double* A;    // n x n intervals
   const double* b;    // n x nrhs intervals
@@ -246,20 +240,25 @@ struct VcphipLssProblem {
   double* X;          // n x nrhs intervals (output)
   long lda, ldb, ldr, ldx;
   int n, nrhs;
-  double* mb;         // n x nrhs, packed: mid(b)
-  double* mx;         // n x nrhs: R mid(b)
+  double* mx;         // n x nrhs, packed: R mid(b)
   double* xi;         // n x nrhs intervals: IA mx - b
   double* y;          // n x nrhs intervals: |R (IA mx - b)|
-  const double* C;    // n x n intervals, ld n: R IA - I (from the batched residual)
-  const double* normub;   // g >= ||R IA - I||_inf (from the batched residual)
-  double* norms;      // [1] T = ||y||_inf, [2] [3] G
+  const double* C;    // n x n intervals, ld n: R IA (single) or R IA - I (from the batched residual)
+  const double* normub;   // g >= ||R IA - I||_inf (batched)
+  double* norms;      // [0] g (single), [1] T = ||y||_inf, [2] [3] G
 };
-// problem p's (row, column) items are [pb[p], pb[p + 1]), pb[count] = total.
-// rhs: mid(b), R mid(b), IA mx - b, |R (...)| and ||y||_inf (independent of
-// R IA - I); bound: G and the enclosure (needs R IA - I and its norm).
-int vcphip_lss_launch_batched_rhs(int count, long items, const long* pb, const VcphipLssProblem* probs,
+// mx = R mid(b); xi = IA mx - b; y = |R xi|; then, from C = R IA, the row
+// sums of |C - I| (rows: n doubles), g, T, G (norms) and the enclosure X
+int vcphip_lss_launch_mx(const VcphipLssProblem& P, hipStream_t s);
+int vcphip_lss_launch_ax(const VcphipLssProblem& P, hipStream_t s);
+int vcphip_lss_launch_ry(const VcphipLssProblem& P, hipStream_t s);
+int vcphip_lss_launch_bound(const VcphipLssProblem& P, double* rows, hipStream_t s);
+// batched: problem p's blocks of 8 rows x 8 right-hand sides are [wb[p],
+// wb[p + 1]), wb[count] = blocks.  rhs: mx, xi, y and ||y||_inf (independent
+// of R IA - I); bound: G and the enclosure (needs R IA - I and its norm).
+int vcphip_lss_launch_batched_rhs(int count, long blocks, const long* wb, const VcphipLssProblem* probs,
                                   hipStream_t s);
-int vcphip_lss_launch_batched_bound(int count, long items, const long* pb, const VcphipLssProblem* probs,
+int vcphip_lss_launch_batched_bound(int count, long blocks, const long* wb, const VcphipLssProblem* probs,
                                     hipStream_t s);
 
 // Galerkin matrix A(i, j) = sum_k ((w_k u_k) phi(i, k)) phi(j, k) in interval
