@@ -84,10 +84,12 @@ enum {
                                       problem: VCPHIP_BATCH_TILES_* (0 = tuned per
                                       size class, else 64 x 64) */
     VCPHIP_PARAM_PLANE_ROWS = 7    /* output rows per tile of the plain single
-                                      products: 64 or 32 (0 = 32 up to 4 64-row
-                                      tiles per CU for interval x interval, 3 for
-                                      the other forms, else 64); the bits of
-                                      every output are the same in both */
+                                      products: 64 or 32 (0 = 32 up to 3 64-row
+                                      tiles per CU, 5 for A^T A, else 64, and
+                                      row-serial blocks for few columns or
+                                      small sizes, which a forced value rules
+                                      out); the bits of every output are the
+                                      same in all */
 };
 
 /* tile shapes of the batched persistent launches (vcphip_igemm_batched*,

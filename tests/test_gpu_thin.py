@@ -7,13 +7,21 @@ the same kernel at the numbers of right-hand sides where its shape or route
 changes."""
 import numpy as np
 import pytest
+import torch
 
 import oracle_ffi as O
 import vcp_amd
 from vcp_amd import workloads as W
-from test_gpu_planes import PAD, SENTINEL, _dev_iv, _dev_pt, _ok, _out_iv, _read_iv, _wide
+from test_gpu_planes import PAD, SENTINEL, _dev_iv, _dev_pt, _ok, _read_iv, _wide
+from test_gpu_planes import _out_iv as _out_async
 
 pytestmark = pytest.mark.gpu
+
+
+def _out_iv(rows, cols, ld):
+    t = _out_async(rows, cols, ld)
+    torch.cuda.synchronize()   # the fill runs on torch's stream, the product on the context's
+    return t
 
 # columns per workgroup: 8 up to n = 8 and for small grids, 16 up to n = 16,
 # 32 at (640, 64), 64 at (1200, 17) and (1201, 65)
@@ -49,6 +57,7 @@ def test_thin_products_bitexact(ctx, m, n, k):
         dU, dD = _dev_pt(U0, ldc), _dev_pt(D0, ldc)
         dU[:, m:] = SENTINEL
         dD[:, m:] = SENTINEL
+        torch.cuda.synchronize()
         _ok(L.vcphip_gemm_rurd_dev(ctx._h, m, n, k, dA.data_ptr(), lda, dB.data_ptr(), ldb, dU.data_ptr(),
                                    dD.data_ptr(), ldc, acc), "gemm_rurd_dev")
         ctx.synchronize()

@@ -14,286 +14,216 @@
 //   r2  = RU chain of rad A*|mid B|                       (:281)
 // and the epilogue applies the reference's fix-ups in its order
 //   t = RU(r1 + r2); upper = RU(up + t); lower = RD(-dn - t) = -RU(dn + t).
-// Two implementations share these chains: k_drgemm_planes (the single
-// products), fed from midpoint-radius planes made once per operand, and the
-// tile function dr_tile (k_drgemm for the thin products, the batched
-// launches), which reads the AoS {inf, sup} operands and converts them to
-// midpoint-radius on their way into LDS (pidblas_assist::midrad, :43-60).
+// Three implementations share these chains: k_drgemm_planes (the single
+// products), fed from midpoint-radius planes made once per operand; the tile
+// function dr_tile (the batched launches, and k = 0), which reads the AoS
+// {inf, sup} operands and converts them to midpoint-radius on their way into
+// LDS (pidblas_assist::midrad, :43-60); and the row-serial k_drgemm_thin for
+// few columns and small sizes (vcphip_thin.h).  The two tiled ones carry them
+// as DPP multiply-adds (vcphip_dpp.h).
 //
 // The whole kernel runs in round-toward-+inf (see vcphip_device.h).
 #include "vcphip_device.h"
 #include "vcphip_kernels.h"
 #include "vcphip_thin.h"
+#include "vcphip_dpp.h"
 
 namespace {
 
 constexpr int BM = 64, BN = 64, BK = 16;
+constexpr int NT = 256;          // 4 waves
+// the k = 0 syrk and the inf-sup tiles: thread (tx, ty) of 16 x 16 holds rows
+// 4 ty .. 4 ty + 3 and columns tx + 16 j
 constexpr int TM = 4, TN = 4;
-constexpr int NT = 256;          // 16 x 16 threads, 4 waves
-// thread (tx, ty) holds rows 4 ty .. 4 ty + 3 of a tile and four of its
-// columns: 2 tx, 2 tx + 1, 2 tx + 32, 2 tx + 33 in dr_tile (dr_col), tx + 16 j
-// in the syrk and inf-sup tiles.  Either way a wave reads B from consecutive
-// LDS addresses (no bank conflicts) and A as a broadcast of four row
-// quadruples
 constexpr int PAD = 2;           // doubles of row padding (keeps 16-byte alignment)
 constexpr int LA = BM + PAD;     // LDS row length of an A k-slice
 constexpr int LB = BN + PAD;
 constexpr int A_PER_T = BM * BK / NT;   // 4 elements of A per thread per tile
 constexpr int B_PER_T = BK * BN / NT;   // 4 elements of B per thread per tile
 
-template <bool AI, bool BI, int APT>
-struct Stage {
-  // register staging of one global tile (prefetch)
-  double a0[APT], a1[APT];
-  double b0[B_PER_T], b1[B_PER_T];
-};
-
-// LDS of one k-slice: midpoints and radii of A (rows) and B (columns).  One
+// LDS of the tile kernels: two slices of BKT k of A (rows) and B (columns),
+// an element as its (mid, rad) pair (interval) or itself (point).  One
 // instance per kernel, shared by every tile shape the kernel runs; a tile of
-// 32 rows uses the first 32 (+ padding) doubles of each A row.
+// 32 rows uses the first 32 elements of each A row.  The odd row stride
+// spreads B's stores (16 lanes along k) over the banks.
 template <bool AI, bool BI>
 struct DrLds {
-  double Am[BK][LA];
-  double Ar[AI ? BK : 1][LA];
-  double Bm[BK][LB];
-  double Br[BI ? BK : 1][LB];
+  static constexpr int BKT = AI && BI ? 8 : 16;   // k per slice
+  static constexpr int AE = AI ? 2 : 1, BE = BI ? 2 : 1, LDR = BM + 1;
+  double a[2][BKT * LDR * AE];
+  double b[2][BKT * LDR * BE];
 };
-
-// column of output j (< 4) of thread column tx in a 64-wide tile: pairs
-// 2 tx, 2 tx + 1 and 2 tx + 32, 2 tx + 33, so a wave reads B as 16-byte
-// pieces at consecutive addresses
-__device__ __forceinline__ int dr_col(int tx, int j) { return 2 * tx + (j & 1) + 32 * (j >> 1); }
 
 // One (16 TMR) x BN output tile at (row0, col0): TMR = 4 gives the 64 x 64
 // tile, TMR = 2 the 32 x 64 tile of the batched launches' short problems and
 // edge rows (each output's chains are the same in both, so are its bits).
+// Operands straight from the AoS matrices, converted on their way into LDS;
+// four waves of 4 TMR x 2 rows x 32 columns in the layout of vcphip_dpp.h.
 // RESID: the batched residual form R*A - I, whose diagonal elements get the
 // interval subtraction of 1 (imats.hpp:324-326).  Runs in the caller's
 // round-up mode.
-template <bool AI, bool BI, bool RESID, int TMR = TM, class Lds = DrLds<AI, BI>>
+template <bool PAIR>
+__device__ __forceinline__ double2 dr_load(__amdgpu_buffer_rsrc_t g, unsigned off) {
+  if (PAIR) return __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(g, off, 0, 0));
+  return make_double2(__builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(g, off, 0, 0)), 0.0);
+}
+
+constexpr long DR_LDMAX = VCPHIP_TILE_LDMAX;
+
+template <bool AI, bool BI, bool RESID, int TMR = 4, bool BIG = false, class Lds = DrLds<AI, BI>>
 __device__ __forceinline__ void dr_tile(Lds& L, int m, int n, int k, const double* __restrict__ A,
                                         long lda, const double* __restrict__ B, long ldb, double* __restrict__ C,
                                         long ldc, double* __restrict__ C2, int accumulate, int row0, int col0) {
   constexpr bool II = AI && BI;
-  constexpr int TBM = 16 * TMR;              // tile rows
-  constexpr int APT = TBM * BK / NT;         // elements of A per thread per slice
-  constexpr int AKS = NT / TBM;              // k stride of a thread's A elements
+  constexpr int RPL = 4 * TMR, TBM = 4 * RPL;   // rows per lane, tile rows
+  constexpr int BKT = Lds::BKT, AE = Lds::AE, BE = Lds::BE, LDR = Lds::LDR;
+  constexpr int APT = TBM * BKT / NT;           // elements of A per thread per slice
+  constexpr int BPT = BN * BKT / NT;
+  constexpr int AKS = NT / TBM;                 // k stride of a thread's A elements
+  constexpr int BCS = NT / BKT;                 // column stride of its B elements
   static_assert(TMR == 4 || TMR == 2, "tile rows");
-  auto& sAm = L.Am;
-  auto& sAr = L.Ar;
-  auto& sBm = L.Bm;
-  auto& sBr = L.Br;
-
+  static_assert(APT >= 1 && AKS * APT == BKT, "slice shape");
   const int tid = threadIdx.x;
 
   // global-load mapping: A column-major, TBM consecutive rows per k column;
-  // B column-major, 16 consecutive k per column.
+  // B column-major, BKT consecutive k per column.
   const int a_row = tid % TBM, a_kc = tid / TBM;   // k column a_kc + AKS q
-  const int b_k = tid % BK, b_col = tid / BK;      // column b_col + 16q
-
-  Stage<AI, BI, APT> st;
-  // global loads of one k-slice; a slice whose rows, columns and k lie
-  // inside the operands (every slice of an interior tile but a partial last
-  // one) takes the unchecked path (the choice is uniform per workgroup).  The
-  // interval x point form keeps the checked path only: the second path makes
-  // it spill at three waves per SIMD.
+  const int b_k = tid % BKT, b_col = tid / BKT;    // column b_col + BCS q
+  double2 ra[APT], rb[BPT];
+  // global loads of one k-slice, zeros outside the operands: buffer loads
+  // from a uniform base at 32-bit lane offsets that stay the same over the
+  // slices.  The resource's size ends A after column k - 1 and B after column
+  // n - 1; a row of A past m, and B's rows past k in the last slice, take an
+  // offset past any size.  (Leading dimensions below DR_LDMAX keep every
+  // offset below 2^31; larger ones, BIG, take 64-bit addresses and checks.)
+  constexpr unsigned OUT = 1u << 31;
+  const unsigned a_off = row0 + a_row < m ? 8u * AE * ((unsigned)a_row + (unsigned)lda * a_kc) : OUT;
+  const unsigned a_step = 8u * AE * AKS * (unsigned)lda;
+  const unsigned b_off = 8u * BE * ((unsigned)b_k + (unsigned)ldb * b_col), b_step = 8u * BE * BCS * (unsigned)ldb;
   auto load_tile = [&](int k0) {
-    constexpr bool FAST = II || !AI;
-    const bool inside = FAST && row0 + TBM <= m && col0 + BN <= n && k0 + BK <= k;
-    if (inside) {
+    if (BIG) {
 #pragma unroll
       for (int q = 0; q < APT; ++q) {
         const int kk = k0 + a_kc + AKS * q, r = row0 + a_row;
-        if (AI) {
-          const double2 v = *reinterpret_cast<const double2*>(A + 2 * (r + lda * kk));
-          st.a0[q] = v.x;
-          st.a1[q] = v.y;
-        } else {
-          st.a0[q] = A[r + lda * kk];
-        }
+        const bool ok = (r < m) && (kk < k);
+        if (AI) ra[q] = ok ? *reinterpret_cast<const double2*>(A + 2 * (r + lda * kk)) : make_double2(0.0, 0.0);
+        else ra[q].x = ok ? A[r + lda * kk] : 0.0;
       }
 #pragma unroll
-      for (int q = 0; q < B_PER_T; ++q) {
-        const int kk = k0 + b_k, c = col0 + b_col + 16 * q;
-        if (BI) {
-          const double2 v = *reinterpret_cast<const double2*>(B + 2 * (kk + ldb * c));
-          st.b0[q] = v.x;
-          st.b1[q] = v.y;
-        } else {
-          st.b0[q] = B[kk + ldb * c];
-        }
+      for (int q = 0; q < BPT; ++q) {
+        const int kk = k0 + b_k, c = col0 + b_col + BCS * q;
+        const bool ok = (kk < k) && (c < n);
+        if (BI) rb[q] = ok ? *reinterpret_cast<const double2*>(B + 2 * (kk + ldb * c)) : make_double2(0.0, 0.0);
+        else rb[q].x = ok ? B[kk + ldb * c] : 0.0;
       }
       return;
     }
+    // the last slice may start past k (k is rounded up to 16): A is then empty
+    const long sa = 8 * AE * (lda * (long)(k > k0 ? k - k0 : 0)), sb = 8 * BE * (ldb * (long)(n - col0));
+    const __amdgpu_buffer_rsrc_t ga = vcphip_rsrc(A + AE * (row0 + lda * k0), (int)(sa < (long)OUT ? sa : (long)OUT));
+    const __amdgpu_buffer_rsrc_t gb = vcphip_rsrc(B + BE * (k0 + ldb * col0), (int)(sb < (long)OUT ? sb : (long)OUT));
+    const unsigned bo = k0 + b_k < k ? b_off : OUT;
 #pragma unroll
-    for (int q = 0; q < APT; ++q) {
-      const int kk = k0 + a_kc + AKS * q, r = row0 + a_row;
-      const bool ok = (r < m) && (kk < k);
-      if (AI) {
-        double2 v = ok ? *reinterpret_cast<const double2*>(A + 2 * (r + lda * kk)) : make_double2(0.0, 0.0);
-        st.a0[q] = v.x;
-        st.a1[q] = v.y;
-      } else {
-        st.a0[q] = ok ? A[r + lda * kk] : 0.0;
-      }
-    }
+    for (int q = 0; q < APT; ++q) ra[q] = dr_load<AI>(ga, a_off + q * a_step);
 #pragma unroll
-    for (int q = 0; q < B_PER_T; ++q) {
-      const int kk = k0 + b_k, c = col0 + b_col + 16 * q;
-      const bool ok = (kk < k) && (c < n);
-      if (BI) {
-        double2 v = ok ? *reinterpret_cast<const double2*>(B + 2 * (kk + ldb * c)) : make_double2(0.0, 0.0);
-        st.b0[q] = v.x;
-        st.b1[q] = v.y;
-      } else {
-        st.b0[q] = ok ? B[kk + ldb * c] : 0.0;
-      }
-    }
+    for (int q = 0; q < BPT; ++q) rb[q] = dr_load<BI>(gb, bo + q * b_step);
   };
-  auto store_tile = [&]() {
+  auto store_tile = [&](int buf) {
 #pragma unroll
     for (int q = 0; q < APT; ++q) {
+      double* d = &L.a[buf][((a_kc + AKS * q) * LDR + a_row) * AE];
       if (AI) {
         double mm, rr;
-        vcphip_midrad_ru(st.a0[q], st.a1[q], mm, rr);
-        sAm[a_kc + AKS * q][a_row] = mm;
-        sAr[a_kc + AKS * q][a_row] = rr;
+        vcphip_midrad_ru(ra[q].x, ra[q].y, mm, rr);
+        *reinterpret_cast<double2*>(d) = make_double2(mm, rr);
       } else {
-        sAm[a_kc + AKS * q][a_row] = st.a0[q];
+        *d = ra[q].x;
       }
     }
 #pragma unroll
-    for (int q = 0; q < B_PER_T; ++q) {
+    for (int q = 0; q < BPT; ++q) {
+      double* d = &L.b[buf][(b_k * LDR + b_col + BCS * q) * BE];
       if (BI) {
         double mm, rr;
-        vcphip_midrad_ru(st.b0[q], st.b1[q], mm, rr);
-        sBm[b_k][b_col + 16 * q] = mm;
-        sBr[b_k][b_col + 16 * q] = rr;
+        vcphip_midrad_ru(rb[q].x, rb[q].y, mm, rr);
+        *reinterpret_cast<double2*>(d) = make_double2(mm, rr);
       } else {
-        sBm[b_k][b_col + 16 * q] = st.b0[q];
+        *d = rb[q].x;
       }
     }
   };
 
-  const int tx = tid % 16, ty = tid / 16;
-  double up[TMR][TN], dn[TMR][TN], r1[TMR][TN], r2[TMR][TN];
+  const int lane = tid & 63, w = tid >> 6;
+  const int lrow = (w & 1) * 2 * RPL + (lane >> 5) * RPL, lcol = (w >> 1) * 32 + (lane & 31);
+  const int orow = row0 + lrow, ocol = col0 + lcol;
+  const int aoff = (lrow + (lane & (RPL - 1))) * AE, boff = lcol * BE;
+  double up[RPL], dn[RPL], r1[RPL], r2[RPL];
 #pragma unroll
-  for (int i = 0; i < TMR; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      up[i][j] = 0.0;
-      dn[i][j] = 0.0;
-      r1[i][j] = 0.0;
-      r2[i][j] = 0.0;
-    }
+  for (int i = 0; i < RPL; ++i) {
+    up[i] = 0.0;
+    dn[i] = 0.0;
+    r1[i] = 0.0;
+    r2[i] = 0.0;
+  }
 
   if (!AI && !BI && accumulate) {
     // udmatmul form: the chains continue from the values already in CU / CD
 #pragma unroll
-    for (int i = 0; i < TMR; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int r = row0 + ty * TMR + i, c = col0 + dr_col(tx, j);
-        if (r < m && c < n) {
-          up[i][j] = C[r + ldc * c];
-          dn[i][j] = -C2[r + ldc * c];
-        }
+    for (int i = 0; i < RPL; ++i)
+      if (orow + i < m && ocol < n) {
+        up[i] = C[orow + i + ldc * ocol];
+        dn[i] = -C2[orow + i + ldc * ocol];
       }
   }
 
-  const int ntiles = (k + BK - 1) / BK;
-  load_tile(0);
-  store_tile();
-  __syncthreads();
-  for (int t = 0; t < ntiles; ++t) {
-    if (t + 1 < ntiles) load_tile((t + 1) * BK);
-#pragma unroll 2
-    for (int kk = 0; kk < BK; ++kk) {
-      double am[TMR], ar[TMR], bm[TN], br[TN];
-      {
-#pragma unroll
-        for (int h = 0; h < TMR / 2; ++h) {
-          const double2 x = *reinterpret_cast<const double2*>(&sAm[kk][ty * TMR + 2 * h]);
-          am[2 * h] = x.x;
-          am[2 * h + 1] = x.y;
-        }
-        const double2 y0 = *reinterpret_cast<const double2*>(&sBm[kk][2 * tx]);
-        const double2 y1 = *reinterpret_cast<const double2*>(&sBm[kk][2 * tx + 32]);
-        bm[0] = y0.x; bm[1] = y0.y; bm[2] = y1.x; bm[3] = y1.y;
-      }
-      if (AI) {
-#pragma unroll
-        for (int h = 0; h < TMR / 2; ++h) {
-          const double2 x = *reinterpret_cast<const double2*>(&sAr[kk][ty * TMR + 2 * h]);
-          ar[2 * h] = x.x;
-          ar[2 * h + 1] = x.y;
-        }
-      }
-      if (BI) {
-        const double2 y0 = *reinterpret_cast<const double2*>(&sBr[kk][2 * tx]);
-        const double2 y1 = *reinterpret_cast<const double2*>(&sBr[kk][2 * tx + 32]);
-        br[0] = y0.x; br[1] = y0.y; br[2] = y1.x; br[3] = y1.y;
-      }
-#pragma unroll
-      for (int i = 0; i < TMR; ++i) {
-        // (|mA| + rA), RU (:277): an add per k and row, not a third LDS array,
-        // since the tile's LDS reads already match its FMA time
-        double as = 0.0;
-        if (II) as = __builtin_fabs(am[i]) + ar[i];
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          up[i][j] = __builtin_fma(am[i], bm[j], up[i][j]);
-          dn[i][j] = __builtin_fma(-am[i], bm[j], dn[i][j]);
-          if (II) {
-            r1[i][j] = __builtin_fma(as, br[j], r1[i][j]);   // (|mA| + rA) rB (:277-279)
-            r2[i][j] = __builtin_fma(ar[i], __builtin_fabs(bm[j]), r2[i][j]);
-          } else if (AI) {
-            r1[i][j] = __builtin_fma(ar[i], __builtin_fabs(bm[j]), r1[i][j]);   // rA*|B|  (:129)
-          } else if (BI) {
-            r1[i][j] = __builtin_fma(__builtin_fabs(am[i]), br[j], r1[i][j]);   // |B|*rA  (:185)
-          }
-        }
-      }
-    }
-    __syncthreads();
-    if (t + 1 < ntiles) {
-      store_tile();
-      __syncthreads();
-    }
+  // slices up to k rounded up to 16 (as the planes pad)
+  const int nt = (k + 15) / 16 * 16 / BKT;
+  if (nt > 0) {
+    load_tile(0);
+    store_tile(0);
+    if (nt > 1) load_tile(BKT);
+  }
+  for (int t = 0; t < nt; ++t) {
+    __syncthreads();   // slice t is in LDS; the reads of the other buffer (slice t - 1) are done
+    if (t + 1 < nt) store_tile((t + 1) & 1);
+    if (t + 2 < nt) load_tile((t + 2) * BKT);
+    const double* sa = L.a[t & 1] + aoff;
+    const double* sb = L.b[t & 1] + boff;
+    auto rd = [&](int kk, double2& a, double2& b) {
+      if (AI) a = *reinterpret_cast<const double2*>(sa + kk * LDR * AE);
+      else a.x = sa[kk * LDR];
+      if (BI) b = *reinterpret_cast<const double2*>(sb + kk * LDR * BE);
+      else b.x = sb[kk * LDR];
+    };
+    vcphip_dpp_slice<BKT>(rd, [&](double2 a, double2 b) {
+      vcphip_dpp_step<AI, BI>(a.x, a.y, b.x, b.y, up, dn, r1, r2);
+    });
   }
 
   // epilogue
+  if (ocol >= n) return;
 #pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int c = col0 + dr_col(tx, j);
-    if (c >= n) continue;
-#pragma unroll
-    for (int i = 0; i < TMR; ++i) {
-      const int r = row0 + ty * TMR + i;
-      if (r >= m) continue;
-      if (AI || BI) {
-        double t;
-        if (II) t = r1[i][j] + r2[i][j];    // temp = (|mA|+rA) rB + rA |mB|   (:283)
-        else t = r1[i][j];
-        double hi = up[i][j] + t;             // uC += temp, RU                  (:284)
-        double nlo = dn[i][j] + t;            // lC -= temp, RD = -(RU(-lC + t)) (:285-286)
-        if (RESID && r == c) {                // b(i,i) -= 1 in interval arithmetic
-          hi = hi - 1.0;
-          nlo = nlo + 1.0;
-        }
-        *reinterpret_cast<double2*>(C + 2 * (r + ldc * c)) = make_double2(-nlo, hi);
-      } else {
-        C[r + ldc * c] = up[i][j];
-        C2[r + ldc * c] = -dn[i][j];
+  for (int i = 0; i < RPL; ++i) {
+    const int r = orow + i;
+    if (r >= m) break;
+    if (AI || BI) {
+      const double t = II ? r1[i] + r2[i] : r1[i];   // temp = (|mA|+rA) rB + rA |mB|   (:283)
+      double hi = up[i] + t;                         // uC += temp, RU                  (:284)
+      double nlo = dn[i] + t;                        // lC -= temp, RD = -(RU(-lC + t)) (:285-286)
+      if (RESID && r == ocol) {                      // b(i,i) -= 1 in interval arithmetic
+        hi = hi - 1.0;
+        nlo = nlo + 1.0;
       }
+      *reinterpret_cast<double2*>(C + 2 * (r + ldc * ocol)) = make_double2(-nlo, hi);
+    } else {
+      C[r + ldc * ocol] = up[i];
+      C2[r + ldc * ocol] = -dn[i];
     }
   }
 }
 
 template <bool AI, bool BI>
-// interval x interval tiles hold four chains per output (2 waves per SIMD);
-// the other forms fit in 168 VGPRs (3 waves per SIMD)
-__global__ __launch_bounds__(NT, (AI && BI) ? 2 : 3) void k_drgemm(int m, int n, int k, const double* __restrict__ A, long lda,
+__global__ __launch_bounds__(NT, 2) void k_drgemm(int m, int n, int k, const double* __restrict__ A, long lda,
                                                    const double* __restrict__ B, long ldb, double* __restrict__ C,
                                                    long ldc, double* __restrict__ C2, int accumulate) {
   vcphip_mode_round_up();
@@ -302,54 +232,61 @@ __global__ __launch_bounds__(NT, (AI && BI) ? 2 : 3) void k_drgemm(int m, int n,
   int tm, tn;
   vcphip_tile_coords(tile, ntm, ntn, 16, tm, tn);
   __shared__ __attribute__((aligned(16))) DrLds<AI, BI> lds;
-  dr_tile<AI, BI, false>(lds, m, n, k, A, lda, B, ldb, C, ldc, C2, accumulate, tm * BM, tn * BN);
+  dr_tile<AI, BI, false, 4, true>(lds, m, n, k, A, lda, B, ldb, C, ldc, C2, accumulate, tm * BM, tn * BN);
 }
 
 // ---------------------------------------------------------------------------
 // The single products from operand planes.
 //
-// pidblas_assist::midrad (:43-60) is taken once per operand element by two
-// small kernels instead of once per element and tile inside the product, and
+// pidblas_assist::midrad (:43-60) is taken once per operand element by one
+// small kernel instead of once per element and tile inside the product, and
 // both operands are laid out for whole, contiguous k-slices:
-//   A (m x k, column-major) -> mid(A), rad(A) (interval) or A (point),
-//                              mpad x kpad, column-major (ld mpad)
-//   B (k x n, column-major) -> mid(B), rad(B) or B, kpad x npad, row-major
-//                              (ld npad)
+//   A (m x k, column-major) -> (mid, rad) pairs (interval) or A (point),
+//                              kpad x mpad, rows contiguous (ld mpad)
+//   B (k x n, column-major) -> pairs or B, kpad x npad, columns contiguous
 // zero beyond m, n and k (mpad, npad multiples of 64, kpad of 16).  Every
-// k-slice of a tile (16 k x 64 of each plane) then lies in 16 runs of 512
-// contiguous bytes, which the product loads straight into LDS with no bounds
-// tests, no conversions and no register staging.  The chains and their order
-// are those of dr_tile, so are the results' bits (padding adds the same zero
-// terms the checked loads of dr_tile add past k).
+// k-slice of a tile then lies in runs of 256 to 1024 contiguous bytes, which
+// the product loads straight into LDS with no bounds tests, no conversions
+// and no register staging, and an element's pair is one 16-byte LDS read.
+// The chains and their order are those of dr_tile, so are the results' bits
+// (padding adds the same zero terms the checked loads of dr_tile add past k).
 // ---------------------------------------------------------------------------
-template <bool AI>
-__global__ __launch_bounds__(256) void k_planes_a(int m, int k, int mpad, const double* __restrict__ A, long lda,
-                                                  double* __restrict__ P0, double* __restrict__ P1) {
-  vcphip_mode_round_up();
-  const int r = blockIdx.x * 256 + threadIdx.x, kk = blockIdx.y;
-  if (r >= mpad) return;
-  const long o = (long)kk * mpad + r;
-  const bool in = r < m && kk < k;
-  if (AI) {
-    double mm = 0.0, rr = 0.0;
-    if (in) {
-      const double2 v = *reinterpret_cast<const double2*>(A + 2 * (r + lda * (long)kk));
-      vcphip_midrad_ru(v.x, v.y, mm, rr);
-    }
-    P0[o] = mm;
-    P1[o] = rr;
-  } else {
-    P0[o] = in ? A[r + lda * (long)kk] : 0.0;
-  }
-}
-
-// B through a 32 x 32 LDS tile: read along k (B's columns), write along n
-template <bool BI>
-__global__ __launch_bounds__(256) void k_planes_bt(int k, int n, int kpad, int npad, const double* __restrict__ B,
-                                                   long ldb, double* __restrict__ P0, double* __restrict__ P1) {
+// blocks [0, na): A, 64 rows x 16 k each; the rest: B, 32 x 32 tiles through
+// LDS (read along k, written along n), 32-column blocks inside 32-k blocks
+template <bool AI, bool BI>
+__global__ __launch_bounds__(256) void k_planes(int m, int n, int k, int mpad, int npad, int kpad, unsigned na,
+                                                const double* __restrict__ A, long lda, const double* __restrict__ B,
+                                                long ldb, double* __restrict__ PA, double* __restrict__ PB) {
   vcphip_mode_round_up();
   __shared__ double2 s[32][33];
-  const int k0 = blockIdx.x * 32, j0 = blockIdx.y * 32;
+  if (blockIdx.x < na) {
+    const unsigned rb = blockIdx.x % (unsigned)(mpad / 64), kb = blockIdx.x / (unsigned)(mpad / 64);
+    const int r = (int)rb * 64 + (threadIdx.x & 63), k0 = (int)kb * 16 + (threadIdx.x >> 6);
+    double2 v[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int kk = k0 + 4 * q;
+      v[q] = make_double2(0.0, 0.0);
+      if (r < m && kk < k) {
+        if (AI) v[q] = *reinterpret_cast<const double2*>(A + 2 * (r + lda * (long)kk));
+        else v[q].x = A[r + lda * (long)kk];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const long o = (long)(k0 + 4 * q) * mpad + r;
+      if (AI) {
+        double mm, rr;
+        vcphip_midrad_ru(v[q].x, v[q].y, mm, rr);   // (0, 0) for the padding
+        *reinterpret_cast<double2*>(PA + 2 * o) = make_double2(mm, rr);
+      } else {
+        PA[o] = v[q].x;
+      }
+    }
+    return;
+  }
+  const unsigned bb = blockIdx.x - na, nj = (unsigned)(npad / 32);
+  const int k0 = (int)(bb / nj) * 32, j0 = (int)(bb % nj) * 32;
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;   // 32 x 8
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -370,163 +307,142 @@ __global__ __launch_bounds__(256) void k_planes_bt(int k, int n, int kpad, int n
     const long o = (long)kk * npad + j;
     if (BI) {
       double mm, rr;
-      vcphip_midrad_ru(v.x, v.y, mm, rr);   // (0, 0) for the padding
-      P0[o] = mm;
-      P1[o] = rr;
+      vcphip_midrad_ru(v.x, v.y, mm, rr);
+      *reinterpret_cast<double2*>(PB + 2 * o) = make_double2(mm, rr);
     } else {
-      P0[o] = v.x;
+      PB[o] = v.x;
     }
   }
 }
 
-// Tiles of 16 TMR x 64 outputs: TMR = 4 (64 rows) for grids that fill the
-// device, TMR = 2 (32 rows) for small ones, which would leave most CUs one
-// workgroup (one wave per SIMD) or idle.  Interval x interval tiles hold four
-// chains per output, point x point two, the mixed forms three; the waves per
-// SIMD follow (64 rows: 2 / 4 / 3, 32 rows: 3 / 4 / 4).
-template <bool AI, bool BI, int TMR>
-__global__ __launch_bounds__(NT, TMR == 4 ? ((AI && BI) ? 2 : (AI || BI) ? 3 : 4) : ((AI && BI) ? 3 : 4))
-void k_drgemm_planes(int m, int n, int mpad, int npad, int kpad, const double* __restrict__ A0,
-                     const double* __restrict__ A1, const double* __restrict__ B0, const double* __restrict__ B1,
-                     double* __restrict__ C, long ldc, double* __restrict__ C2, int accumulate) {
+// The k-slices of a (4 RPL) x 64 tile in LDS and their loads: a stage is BKS
+// k of A's rows, then of B's columns, elements of AE / BE doubles.  A
+// wave-wide load moves 1 KB: 1024 / (row bytes) k-rows; the workgroup's four
+// waves take the stage's 1 KB pieces in turn, G each (a piece past the last
+// repeats the last one).  Two stages: the next one's loads are in flight
+// under the multiply-adds of the current one.  8 k for 64-row tiles, so that
+// three workgroups' stages fit a CU; 16 k for 32-row ones, whose 8 k take
+// about a load's latency.  (Three or four stages of 8 k measured 0 - 3% slower
+// at n = 1024 to 3072, 8 k for 32 rows 1 - 7% slower at 512 and 1024.)
+template <int RPL, int AE, int BE>
+struct PlaneStage {
+  static constexpr int BKS = RPL == 16 ? 8 : 16, NST = 2;
+  static constexpr int ROWS = 4 * RPL, ARB = ROWS * AE * 8, BRB = 64 * BE * 8;   // bytes of a k-row
+  static constexpr int ABYTES = BKS * ARB, BBYTES = BKS * BRB, BYTES = ABYTES + BBYTES;
+  static constexpr int NA = ABYTES / 1024, NB = BBYTES / 1024, G = (NA + NB + 3) / 4;
+  static_assert(ABYTES % 1024 == 0 && BBYTES % 1024 == 0 && 16 % BKS == 0, "stage shape");
+  const char *a, *b;
+  long lda, ldb;   // bytes of a k-row of the planes
+  uint32_t lds;
+  int w;
+  VCPHIP_DEVINL PlaneStage(const double* PA, long mpad, int row0, const double* PB, long npad, int col0, const void* L) {
+    const int lane = threadIdx.x & 63;
+    w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    lda = mpad * AE * 8;
+    ldb = npad * BE * 8;
+    a = (const char*)(PA + (long)row0 * AE) + (long)(16 * lane / ARB) * lda + 16 * lane % ARB;
+    b = (const char*)(PB + (long)col0 * BE) + (long)(16 * lane / BRB) * ldb + 16 * lane % BRB;
+    lds = vcphip_lds_addr(L);
+  }
+  VCPHIP_DEVINL void issue(int t) const {
+    const uint32_t d = lds + (uint32_t)(t % NST) * BYTES;
+    const char* ga = a + (long)t * BKS * lda;
+    const char* gb = b + (long)t * BKS * ldb;
+#pragma unroll
+    for (int q = 0; q < G; ++q) {
+      int c = 4 * q + w;   // wave-uniform
+      if (c > NA + NB - 1) c = NA + NB - 1;
+      if (c < NA) vcphip_lds_dma16(ga + (long)c * (1024 / ARB) * lda, d + (uint32_t)c * 1024);
+      else vcphip_lds_dma16(gb + (long)(c - NA) * (1024 / BRB) * ldb, d + (uint32_t)c * 1024);
+    }
+  }
+  // slice t has landed for every wave (only its loads are in flight), and
+  // every wave's reads of the other stage, slice t - 1, are done: that stage
+  // takes slice t + 1
+  VCPHIP_DEVINL void next(int t, int nt) const {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (t + 1 < nt) issue(t + 1);
+  }
+};
+
+// Tiles of 4 RPL x 64 outputs, four waves of 2 RPL rows x 32 columns, RPL
+// outputs of one column per lane (vcphip_dpp.h): RPL = 16 (64 rows) for grids
+// that fill the device, RPL = 8 (32 rows) for small ones.  Bound by the FP64
+// multiply-adds, at n = 4096 by the clock that they leave (61 TFLOP/s is 0.93
+// of the rate at 2.0 GHz).  Interval x interval, planes included, against 4 x 4
+// outputs per lane read from LDS: n = 1024 205 -> 203 us, 2048 1432 -> 1153,
+// 4096 11.0 -> 9.1 ms; point x interval at 4096 7.5 -> 6.5 - 7.2 ms.
+template <bool AI, bool BI, int RPL>
+__global__ __launch_bounds__(NT, RPL == 16 ? ((AI && BI) ? 3 : 4) : 4)
+void k_drgemm_planes(int m, int n, int mpad, int npad, int kpad, const double* __restrict__ PA,
+                     const double* __restrict__ PB, double* __restrict__ C, long ldc, double* __restrict__ C2,
+                     int accumulate) {
   constexpr bool II = AI && BI;
-  constexpr int TBM = 16 * TMR;                  // tile rows
-  constexpr int NA = AI ? 2 : 1, NB = BI ? 2 : 1, NP = NA + NB;
-  constexpr int ASL = BK * TBM, BSL = BK * BN;   // doubles of one plane's k-slice
-  constexpr int STAGE = NA * ASL + NB * BSL;
-  static_assert(TMR == 4 || TMR == 2, "tile rows");
-  static_assert(BN == 64 && BK == 16, "slice layout");
+  constexpr int AE = AI ? 2 : 1, BE = BI ? 2 : 1;
+  using Stage = PlaneStage<RPL, AE, BE>;
   vcphip_mode_round_up();
-  // [stage][A mid (or A), A rad: k x TBM][B mid (or B), B rad: k x 64]
-  __shared__ __attribute__((aligned(16))) double sL[2 * STAGE];
-  const int ntm = mpad / TBM, ntn = npad / BN;
+  __shared__ __attribute__((aligned(16))) char sL[Stage::NST * Stage::BYTES];
+  const int ntm = mpad / Stage::ROWS, ntn = npad / 64;
   const int tile = vcphip_xcd_remap(blockIdx.x, ntm * ntn);
   int tm, tn;
   vcphip_tile_coords(tile, ntm, ntn, 16, tm, tn);
-  const int row0 = tm * TBM, col0 = tn * BN;
-  const int tid = threadIdx.x, lane = tid & 63;
-  // wave w < NP loads plane w of every slice, one k-row of a plane slice
-  // per 2^lh lanes (two doubles a lane): a load instruction moves 1 KB, i.e.
-  // 64 / 2^lh k-rows, and a slice takes BK 2^lh / 64 of them
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const bool loader = w < NP;
-  const bool wa = w < NA;
-  const int lh = (wa && TBM == 32) ? 4 : 5;
-  const int nq = BK >> (6 - lh), rpi = 64 >> lh;
-  const double* plane = wa ? (w == 0 ? A0 : A1) : (w == NA ? B0 : B1);
-  const long ld = wa ? mpad : npad;
-  const double* src = plane + (long)(lane >> lh) * ld + (wa ? row0 : col0) + 2 * (lane & ((1 << lh) - 1));
-  const int poff = !loader ? 0 : wa ? w * ASL : NA * ASL + (w - NA) * BSL;
-  const uint32_t lds0 = vcphip_lds_addr(sL) + (uint32_t)poff * 8;
-  auto issue = [&](int stage, int t) {
-    if (!loader) return;
-    const double* g = src + (long)t * BK * ld;
-    const uint32_t d = lds0 + (uint32_t)stage * (STAGE * 8);
-    for (int q = 0; q < nq; ++q) vcphip_lds_dma16(g + (long)(rpi * q) * ld, d + (uint32_t)q * 1024);
-  };
+  const int row0 = tm * Stage::ROWS, col0 = tn * 64;
+  const Stage st(PA, mpad, row0, PB, npad, col0, sL);
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  // this lane's outputs: rows orow .. orow + RPL - 1 of column ocol; lane i
+  // of its DPP row of 16 holds A's row orow + i
+  const int lrow = (w & 1) * 2 * RPL + (lane >> 5) * RPL, lcol = (w >> 1) * 32 + (lane & 31);
+  const int orow = row0 + lrow, ocol = col0 + lcol;
+  const int aoff = (lrow + (lane & (RPL - 1))) * AE * 8, boff = Stage::ABYTES + lcol * BE * 8;
 
-  const int tx = tid % 16, ty = tid / 16;
-  double up[TMR][TN], dn[TMR][TN], r1[TMR][TN], r2[TMR][TN];
+  double up[RPL], dn[RPL], r1[RPL], r2[RPL];
 #pragma unroll
-  for (int i = 0; i < TMR; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      up[i][j] = 0.0;
-      dn[i][j] = 0.0;
-      r1[i][j] = 0.0;
-      r2[i][j] = 0.0;
-    }
+  for (int i = 0; i < RPL; ++i) {
+    up[i] = 0.0;
+    dn[i] = 0.0;
+    r1[i] = 0.0;
+    r2[i] = 0.0;
+  }
   if (!AI && !BI && accumulate) {
     // udmatmul form: the chains continue from the values already in CU / CD
 #pragma unroll
-    for (int i = 0; i < TMR; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int r = row0 + ty * TMR + i, c = col0 + dr_col(tx, j);
-        if (r < m && c < n) {
-          up[i][j] = C[r + ldc * c];
-          dn[i][j] = -C2[r + ldc * c];
-        }
+    for (int i = 0; i < RPL; ++i)
+      if (orow + i < m && ocol < n) {
+        up[i] = C[orow + i + ldc * ocol];
+        dn[i] = -C2[orow + i + ldc * ocol];
       }
   }
 
-  const int nt = kpad / BK;
-  issue(0, 0);
+  const int nt = kpad / Stage::BKS;
+  st.issue(0);
   for (int t = 0; t < nt; ++t) {
-    // only slice t's loads are in flight: wait for them, then for every wave
-    // (which also ends every wave's reads of the other stage, slice t - 1)
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (t + 1 < nt) issue((t + 1) & 1, t + 1);
-    const double* sAm = sL + (t & 1) * STAGE;
-    const double* sAr = sAm + (AI ? ASL : 0);
-    const double* sBm = sAm + NA * ASL;
-    const double* sBr = sBm + (BI ? BSL : 0);
-#pragma unroll 2
-    for (int kk = 0; kk < BK; ++kk) {
-      double am[TMR], ar[TMR], bm[TN], br[TN];
-#pragma unroll
-      for (int h = 0; h < TMR / 2; ++h) {
-        const double2 x = *reinterpret_cast<const double2*>(&sAm[kk * TBM + ty * TMR + 2 * h]);
-        am[2 * h] = x.x;
-        am[2 * h + 1] = x.y;
-      }
-      {
-        const double2 y0 = *reinterpret_cast<const double2*>(&sBm[kk * BN + 2 * tx]);
-        const double2 y1 = *reinterpret_cast<const double2*>(&sBm[kk * BN + 2 * tx + 32]);
-        bm[0] = y0.x; bm[1] = y0.y; bm[2] = y1.x; bm[3] = y1.y;
-      }
-      if (AI) {
-#pragma unroll
-        for (int h = 0; h < TMR / 2; ++h) {
-          const double2 z = *reinterpret_cast<const double2*>(&sAr[kk * TBM + ty * TMR + 2 * h]);
-          ar[2 * h] = z.x;
-          ar[2 * h + 1] = z.y;
-        }
-      }
-      if (BI) {
-        const double2 u0 = *reinterpret_cast<const double2*>(&sBr[kk * BN + 2 * tx]);
-        const double2 u1 = *reinterpret_cast<const double2*>(&sBr[kk * BN + 2 * tx + 32]);
-        br[0] = u0.x; br[1] = u0.y; br[2] = u1.x; br[3] = u1.y;
-      }
-#pragma unroll
-      for (int i = 0; i < TMR; ++i) {
-        double as = 0.0;
-        if (II) as = __builtin_fabs(am[i]) + ar[i];   // (|mA| + rA), RU (:277)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          up[i][j] = __builtin_fma(am[i], bm[j], up[i][j]);
-          dn[i][j] = __builtin_fma(-am[i], bm[j], dn[i][j]);
-          if (II) {
-            r1[i][j] = __builtin_fma(as, br[j], r1[i][j]);                    // (|mA| + rA) rB (:277-279)
-            r2[i][j] = __builtin_fma(ar[i], __builtin_fabs(bm[j]), r2[i][j]);  // rA |mB| (:281)
-          } else if (AI) {
-            r1[i][j] = __builtin_fma(ar[i], __builtin_fabs(bm[j]), r1[i][j]);  // rA*|B|  (:129)
-          } else if (BI) {
-            r1[i][j] = __builtin_fma(__builtin_fabs(am[i]), br[j], r1[i][j]);  // |B|*rA  (:185)
-          }
-        }
-      }
-    }
+    st.next(t, nt);
+    const char* s0 = sL + (t % Stage::NST) * Stage::BYTES;
+    auto rd = [&](int kk, double2& a, double2& b) {
+      if (AI) a = *reinterpret_cast<const double2*>(s0 + aoff + kk * Stage::ARB);
+      else a.x = *reinterpret_cast<const double*>(s0 + aoff + kk * Stage::ARB);
+      if (BI) b = *reinterpret_cast<const double2*>(s0 + boff + kk * Stage::BRB);
+      else b.x = *reinterpret_cast<const double*>(s0 + boff + kk * Stage::BRB);
+    };
+    vcphip_dpp_slice<Stage::BKS>(rd, [&](double2 a, double2 b) {
+      vcphip_dpp_step<AI, BI>(a.x, a.y, b.x, b.y, up, dn, r1, r2);
+    });
   }
 
+  if (ocol >= n) return;
 #pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int c = col0 + dr_col(tx, j);
-    if (c >= n) continue;
-#pragma unroll
-    for (int i = 0; i < TMR; ++i) {
-      const int r = row0 + ty * TMR + i;
-      if (r >= m) continue;
-      if (AI || BI) {
-        const double tt = II ? r1[i][j] + r2[i][j] : r1[i][j];   // temp (:283, :129, :185)
-        const double hi = up[i][j] + tt;                         // uC += temp, RU (:284)
-        const double nlo = dn[i][j] + tt;                        // lC -= temp, RD = -(RU(-lC + t)) (:285-286)
-        *reinterpret_cast<double2*>(C + 2 * (r + ldc * c)) = make_double2(-nlo, hi);
-      } else {
-        C[r + ldc * c] = up[i][j];
-        C2[r + ldc * c] = -dn[i][j];
-      }
+  for (int i = 0; i < RPL; ++i) {
+    const int r = orow + i;
+    if (r >= m) break;
+    if (AI || BI) {
+      const double tt = II ? r1[i] + r2[i] : r1[i];   // temp (:283, :129, :185)
+      const double hi = up[i] + tt;                   // uC += temp, RU (:284)
+      const double nlo = dn[i] + tt;                  // lC -= temp, RD = -(RU(-lC + t)) (:285-286)
+      *reinterpret_cast<double2*>(C + 2 * (r + ldc * ocol)) = make_double2(-nlo, hi);
+    } else {
+      C[r + ldc * ocol] = up[i];
+      C2[r + ldc * ocol] = -dn[i];
     }
   }
 }
@@ -548,15 +464,15 @@ __device__ __forceinline__ int next_tile(unsigned* __restrict__ queue, int& slot
   __syncthreads();   // every thread has read the previous index (and left the tile's LDS)
   if (threadIdx.x == 0) slot = (int)atomicAdd(queue, 1u);
   __syncthreads();
-  return slot;
+  return __builtin_amdgcn_readfirstlane(slot);   // uniform: the tile's descriptors are then scalar loads
 }
 
 __global__ __launch_bounds__(64) void k_queue_reset(unsigned* __restrict__ queue) {
   if (threadIdx.x < 2) queue[threadIdx.x] = 0u;
 }
 
-template <int TMR>
-__global__ __launch_bounds__(NT, 3) void k_resid_tiles(int ntiles, const VcphipResidTile* __restrict__ tiles,
+template <int TMR, bool BIG>
+__global__ __launch_bounds__(NT, BIG ? 2 : 3) void k_resid_tiles(int ntiles, const VcphipResidTile* __restrict__ tiles,
                                                         const VcphipResidProblem* __restrict__ probs,
                                                         unsigned* __restrict__ queue) {
   vcphip_mode_round_up();
@@ -565,7 +481,7 @@ __global__ __launch_bounds__(NT, 3) void k_resid_tiles(int ntiles, const VcphipR
   for (int t = next_tile(queue, slot); t < ntiles; t = next_tile(queue, slot)) {
     const VcphipResidTile tl = tiles[t];
     const VcphipResidProblem p = probs[tl.problem];
-    dr_tile<false, true, true, TMR>(lds, p.n, p.n, p.n, p.R, p.ldr, p.A, p.lda, p.C, p.ldc, nullptr, 0, tl.row0,
+    dr_tile<false, true, true, TMR, BIG>(lds, p.n, p.n, p.n, p.R, p.ldr, p.A, p.lda, p.C, p.ldc, nullptr, 0, tl.row0,
                                     tl.col0);
   }
 }
@@ -575,8 +491,8 @@ __global__ __launch_bounds__(NT, 3) void k_resid_tiles(int ntiles, const VcphipR
 // per problem): workgroups take the tiles of a list sorted by problem size
 // from a work queue, each tile the interval x interval form of k_drgemm, so
 // every C_p is bit-identical to the single product's.
-template <int TMR>
-__global__ __launch_bounds__(NT, 2) void k_igemm_tiles(int ntiles, const VcphipResidTile* __restrict__ tiles,
+template <int TMR, bool BIG>
+__global__ __launch_bounds__(NT, BIG ? 2 : 2) void k_igemm_tiles(int ntiles, const VcphipResidTile* __restrict__ tiles,
                                                         const VcphipIgemmProblem* __restrict__ probs,
                                                         unsigned* __restrict__ queue) {
   vcphip_mode_round_up();
@@ -585,7 +501,7 @@ __global__ __launch_bounds__(NT, 2) void k_igemm_tiles(int ntiles, const VcphipR
   for (int t = next_tile(queue, slot); t < ntiles; t = next_tile(queue, slot)) {
     const VcphipResidTile tl = tiles[t];
     const VcphipIgemmProblem p = probs[tl.problem];
-    dr_tile<true, true, false, TMR>(lds, p.m, p.n, p.k, p.A, p.lda, p.B, p.ldb, p.C, p.ldc, nullptr, 0, tl.row0,
+    dr_tile<true, true, false, TMR, BIG>(lds, p.m, p.n, p.k, p.A, p.lda, p.B, p.ldb, p.C, p.ldc, nullptr, 0, tl.row0,
                                     tl.col0);
   }
 }
@@ -643,9 +559,9 @@ __global__ __launch_bounds__((VcphipThin<ThinProduct<AI, BI>, CW, CPT>::NT)) __a
 
 // row sums of |C| (upward, in column order: mats::norminf, vcp/mats.hpp:
 // 1583-1591) over 8-row blocks of the problems, in the row-serial form: each
-// C_p is read once at a cache line per row block and column (a thread per row
-// and wave-wide row blocks kept too few loads in flight: 153 against XX us
-// for 64 problems of n in [64, 1024])
+// C_p is read once, at a cache line per row block and column (a thread per row,
+// 256 rows to a workgroup, had too few loads in flight: 153 against 98 us for
+// 64 problems of n in [64, 1024])
 struct ResidRowSum {
   static constexpr bool A2 = true, B2 = false, PAD16 = false;
   static constexpr int AL = 1, BL = 0;
@@ -831,118 +747,76 @@ __global__ __launch_bounds__(NT, 2) void k_drsyrk(int k, int n, const double* __
     }
 }
 
-// The same A^T A forms from the planes of A (k x n) made by k_planes_bt:
-// mid(A), rad(A) (or A) row-major kpad x npad, zero-padded.  Column i of A is
-// then the contiguous run at i of every k-row, so one plane set feeds both
-// operands: wave 0..3 load the slices of the row block (mid, rad) and of the
-// column block (mid, rad) straight into LDS, two stages.  The chains and
-// their order are k_drsyrk's.
-template <bool INTV>
-__global__ __launch_bounds__(NT, 2) void k_drsyrk_planes(int n, int npad, int kpad, const double* __restrict__ P0,
-                                                         const double* __restrict__ P1, double* __restrict__ C,
-                                                         long ldc) {
-  constexpr int NP = INTV ? 4 : 2;
+// The same A^T A forms from the planes of A (k x n) made by k_planes's B part:
+// (mid, rad) pairs (or A), kpad x npad, columns contiguous, zero-padded.
+// Column i of A is then the contiguous run at i of every k-row, so one plane
+// set feeds both operands.  Tiles of 4 RPL rows x 64 columns that meet the
+// upper triangle; the chains and their order are k_drsyrk's.
+template <bool INTV, int RPL>
+__global__ __launch_bounds__(NT, RPL == 16 ? (INTV ? 2 : 4) : 4) void k_drsyrk_planes(int n, int npad, int kpad,
+                                                                                      const double* __restrict__ P,
+                                                                                      double* __restrict__ C,
+                                                                                      long ldc) {
+  constexpr int E = INTV ? 2 : 1, H = 64 / (4 * RPL);   // row blocks per 64 rows
+  using Stage = PlaneStage<RPL, E, E>;
   vcphip_mode_round_up();
-  // [stage][plane: I mid, (I rad), J mid, (J rad)][k][64]
-  __shared__ __attribute__((aligned(16))) double sL[2][NP][BK][BM];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int nt = npad / BM;
-  int b = blockIdx.x, tm = 0;
-  while (b >= nt - tm) {
-    b -= nt - tm;
-    ++tm;
+  __shared__ __attribute__((aligned(16))) char sL[Stage::NST * Stage::BYTES];
+  int b = blockIdx.x, tn = 0;   // column block tn has H (tn + 1) row blocks
+  while (b >= H * (tn + 1)) {
+    b -= H * (tn + 1);
+    ++tn;
   }
-  const int tn = tm + b;
-  const int i0 = tm * BM, j0 = tn * BN;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const bool loader = w < NP;
-  // plane of wave w: I mid, I rad, J mid, J rad (interval); I, J (point)
-  const bool rad = INTV && (w & 1);
-  const bool jside = INTV ? (w >= 2) : (w == 1);
-  const double* src = (rad ? P1 : P0) + (long)(lane >> 5) * npad + (jside ? j0 : i0) + 2 * (lane & 31);
-  const uint32_t lds0 = vcphip_lds_addr(&sL[0][0][0][0]) + (uint32_t)(loader ? w : 0) * (BK * BM * 8);
-  auto issue = [&](int stage, int t) {
-    if (!loader) return;
-    const double* g = src + (long)t * BK * npad;
-    const uint32_t d = lds0 + (uint32_t)stage * (NP * BK * BM * 8);
+  const int i0 = b * Stage::ROWS, j0 = tn * 64;
+  const Stage st(P, npad, i0, P, npad, j0, sL);
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int lrow = (w & 1) * 2 * RPL + (lane >> 5) * RPL, lcol = (w >> 1) * 32 + (lane & 31);
+  const int aoff = (lrow + (lane & (RPL - 1))) * E * 8, boff = Stage::ABYTES + lcol * E * 8;
+  double up[RPL], dn[RPL], tij[RPL], tji[RPL], sij[RPL];
 #pragma unroll
-    for (int q = 0; q < BK / 2; ++q) vcphip_lds_dma16(g + (long)(2 * q) * npad, d + (uint32_t)q * (2 * BM * 8));
-  };
-
-  const int tx = tid % 16, ty = tid / 16;
-  double up[TM][TN], dn[TM][TN], tij[TM][TN], tji[TM][TN], sij[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      up[i][j] = 0.0;
-      dn[i][j] = 0.0;
-      tij[i][j] = 0.0;
-      tji[i][j] = 0.0;
-      sij[i][j] = 0.0;
-    }
-
-  const int ns = kpad / BK;
-  issue(0, 0);
-  for (int t = 0; t < ns; ++t) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (t + 1 < ns) issue((t + 1) & 1, t + 1);
-    const double(*sIm)[BM] = sL[t & 1][0];
-    const double(*sIr)[BM] = sL[t & 1][INTV ? 1 : 0];
-    const double(*sJm)[BM] = sL[t & 1][INTV ? 2 : 1];
-    const double(*sJr)[BM] = sL[t & 1][INTV ? 3 : 1];
-#pragma unroll(INTV ? 1 : 2)
-    for (int kk = 0; kk < BK; ++kk) {
-      double a[TM], ar[TM], bb[TN], br[TN];
-      {
-        const double2 x0 = *reinterpret_cast<const double2*>(&sIm[kk][ty * TM]);
-        const double2 x1 = *reinterpret_cast<const double2*>(&sIm[kk][ty * TM + 2]);
-        a[0] = x0.x; a[1] = x0.y; a[2] = x1.x; a[3] = x1.y;
-        const double2 y0 = *reinterpret_cast<const double2*>(&sJm[kk][2 * tx]);
-        const double2 y1 = *reinterpret_cast<const double2*>(&sJm[kk][2 * tx + 32]);
-        bb[0] = y0.x; bb[1] = y0.y; bb[2] = y1.x; bb[3] = y1.y;
-      }
-      if (INTV) {
-        const double2 x0 = *reinterpret_cast<const double2*>(&sIr[kk][ty * TM]);
-        const double2 x1 = *reinterpret_cast<const double2*>(&sIr[kk][ty * TM + 2]);
-        ar[0] = x0.x; ar[1] = x0.y; ar[2] = x1.x; ar[3] = x1.y;
-        const double2 y0 = *reinterpret_cast<const double2*>(&sJr[kk][2 * tx]);
-        const double2 y1 = *reinterpret_cast<const double2*>(&sJr[kk][2 * tx + 32]);
-        br[0] = y0.x; br[1] = y0.y; br[2] = y1.x; br[3] = y1.y;
-      }
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          up[i][j] = __builtin_fma(a[i], bb[j], up[i][j]);
-          dn[i][j] = __builtin_fma(-a[i], bb[j], dn[i][j]);
-          if (INTV) {
-            tij[i][j] = __builtin_fma(__builtin_fabs(a[i]), br[j], tij[i][j]);
-            tji[i][j] = __builtin_fma(__builtin_fabs(bb[j]), ar[i], tji[i][j]);
-            sij[i][j] = __builtin_fma(ar[i], br[j], sij[i][j]);
-          }
-        }
-    }
+  for (int i = 0; i < RPL; ++i) {
+    up[i] = 0.0;
+    dn[i] = 0.0;
+    tij[i] = 0.0;
+    tji[i] = 0.0;
+    sij[i] = 0.0;
   }
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int r = i0 + ty * TM + i, c = j0 + dr_col(tx, j);
-      if (r >= n || c >= n || r > c) continue;
-      double lo, hi;
+  const int nt = kpad / Stage::BKS;
+  st.issue(0);
+  for (int t = 0; t < nt; ++t) {
+    st.next(t, nt);
+    const char* s0 = sL + (t % Stage::NST) * Stage::BYTES;
+    auto rd = [&](int kk, double2& x, double2& y) {
       if (INTV) {
-        const double T = tij[i][j] + (tji[i][j] + sij[i][j]);
-        hi = up[i][j] + T;
-        lo = -(dn[i][j] + T);
+        x = *reinterpret_cast<const double2*>(s0 + aoff + kk * Stage::ARB);
+        y = *reinterpret_cast<const double2*>(s0 + boff + kk * Stage::BRB);
       } else {
-        hi = up[i][j];
-        lo = -dn[i][j];
+        x.x = *reinterpret_cast<const double*>(s0 + aoff + kk * Stage::ARB);
+        y.x = *reinterpret_cast<const double*>(s0 + boff + kk * Stage::BRB);
       }
-      *reinterpret_cast<double2*>(C + 2 * (r + ldc * c)) = make_double2(lo, hi);
-      *reinterpret_cast<double2*>(C + 2 * (c + ldc * r)) = make_double2(lo, hi);
+    };
+    vcphip_dpp_slice<Stage::BKS>(rd, [&](double2 x, double2 y) {
+      if (INTV) vcphip_dpp_syrk_step(x.x, x.y, y.x, y.y, up, dn, tij, tji, sij);
+      else vcphip_dpp_step<false, false>(x.x, 0.0, y.x, 0.0, up, dn, tij, tji);
+    });
+  }
+  const int c = j0 + lcol;
+  if (c >= n) return;
+#pragma unroll
+  for (int i = 0; i < RPL; ++i) {
+    const int r = i0 + lrow + i;
+    if (r > c) break;
+    double lo, hi;
+    if (INTV) {
+      const double T = tij[i] + (tji[i] + sij[i]);
+      hi = up[i] + T;
+      lo = -(dn[i] + T);
+    } else {
+      hi = up[i];
+      lo = -dn[i];
     }
+    *reinterpret_cast<double2*>(C + 2 * (r + ldc * c)) = make_double2(lo, hi);
+    *reinterpret_cast<double2*>(C + 2 * (c + ldc * r)) = make_double2(lo, hi);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1182,33 +1056,16 @@ int vcphip_launch_drgemm_thin(int kind, int m, int n, int k, const double* A, lo
 }
 
 int vcphip_launch_planes(int kind, int m, int n, int k, const double* A, long lda, const double* B, long ldb,
-                         double* A0, double* A1, double* B0, double* B1, hipStream_t s) {
+                         double* PA, double* PB, hipStream_t s) {
   const int mpad = (m + BM - 1) / BM * BM, npad = (n + BN - 1) / BN * BN, kpad = (k + BK - 1) / BK * BK;
   if (m <= 0 || n <= 0 || kpad <= 0) return 0;
-  const bool ai = kind == VCPHIP_DR_II || kind == VCPHIP_DR_IP, bi = kind == VCPHIP_DR_II || kind == VCPHIP_DR_PI;
-  const dim3 ga(mpad / 256 + (mpad % 256 != 0), kpad), gb(kpad / 32 + (kpad % 32 != 0), npad / 32);
-  if (ai) hipLaunchKernelGGL(k_planes_a<true>, ga, dim3(256), 0, s, m, k, mpad, A, lda, A0, A1);
-  else hipLaunchKernelGGL(k_planes_a<false>, ga, dim3(256), 0, s, m, k, mpad, A, lda, A0, A1);
-  if (bi) hipLaunchKernelGGL(k_planes_bt<true>, gb, dim3(256), 0, s, k, n, kpad, npad, B, ldb, B0, B1);
-  else hipLaunchKernelGGL(k_planes_bt<false>, gb, dim3(256), 0, s, k, n, kpad, npad, B, ldb, B0, B1);
-  return hipGetLastError() == hipSuccess ? 0 : -3;
-}
-
-int vcphip_launch_drgemm_planes(int kind, int m, int n, int k, const double* A0, const double* A1, const double* B0,
-                                const double* B1, double* C, long ldc, double* C2, int accumulate, int rows,
-                                hipStream_t s) {
-  const int mpad = (m + BM - 1) / BM * BM, npad = (n + BN - 1) / BN * BN, kpad = (k + BK - 1) / BK * BK;
-  if (m <= 0 || n <= 0) return 0;
-  if (kpad == 0 || (rows != 64 && rows != 32)) return -1;   // k = 0 takes the tile path
-  const dim3 grid((mpad / rows) * (npad / BN)), block(NT);
-#define VCPHIP_PLANES_CASE(KIND, AI, BI)                                                                          \
-  case KIND:                                                                                                     \
-    if (rows == 64)                                                                                              \
-      hipLaunchKernelGGL((k_drgemm_planes<AI, BI, 4>), grid, block, 0, s, m, n, mpad, npad, kpad, A0, A1, B0, B1, \
-                         C, ldc, C2, accumulate);                                                                \
-    else                                                                                                         \
-      hipLaunchKernelGGL((k_drgemm_planes<AI, BI, 2>), grid, block, 0, s, m, n, mpad, npad, kpad, A0, A1, B0, B1, \
-                         C, ldc, C2, accumulate);                                                                \
+  const size_t na = (size_t)(mpad / 64) * (kpad / 16), nb = (size_t)((kpad + 31) / 32) * (npad / 32);
+  if (na + nb > 0x7FFFFFFFu) return -7;
+  const dim3 grid((unsigned)(na + nb));
+#define VCPHIP_PLANES_CASE(KIND, AI, BI)                                                                             \
+  case KIND:                                                                                                         \
+    hipLaunchKernelGGL((k_planes<AI, BI>), grid, dim3(256), 0, s, m, n, k, mpad, npad, kpad, (unsigned)na, A, lda, B, \
+                       ldb, PA, PB);                                                                                 \
     break;
   switch (kind) {
     VCPHIP_PLANES_CASE(VCPHIP_DR_II, true, true)
@@ -1221,19 +1078,50 @@ int vcphip_launch_drgemm_planes(int kind, int m, int n, int k, const double* A0,
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
-int vcphip_launch_drsyrk_planes(int interval, int k, int n, const double* A, long lda, double* P0, double* P1,
-                                double* C, long ldc, hipStream_t s) {
+int vcphip_launch_drgemm_planes(int kind, int m, int n, int k, const double* PA, const double* PB, double* C, long ldc,
+                                double* C2, int accumulate, int rows, hipStream_t s) {
+  const int mpad = (m + BM - 1) / BM * BM, npad = (n + BN - 1) / BN * BN, kpad = (k + BK - 1) / BK * BK;
+  if (m <= 0 || n <= 0) return 0;
+  if (kpad == 0 || (rows != 64 && rows != 32)) return -1;   // k = 0 takes the tile path
+  const dim3 grid((mpad / rows) * (npad / BN)), block(NT);
+#define VCPHIP_PLANES_CASE(KIND, AI, BI)                                                                            \
+  case KIND:                                                                                                        \
+    if (rows == 64)                                                                                                 \
+      hipLaunchKernelGGL((k_drgemm_planes<AI, BI, 16>), grid, block, 0, s, m, n, mpad, npad, kpad, PA, PB, C, ldc, C2, \
+                         accumulate);                                                                               \
+    else                                                                                                            \
+      hipLaunchKernelGGL((k_drgemm_planes<AI, BI, 8>), grid, block, 0, s, m, n, mpad, npad, kpad, PA, PB, C, ldc, C2, \
+                         accumulate);                                                                               \
+    break;
+  switch (kind) {
+    VCPHIP_PLANES_CASE(VCPHIP_DR_II, true, true)
+    VCPHIP_PLANES_CASE(VCPHIP_DR_IP, true, false)
+    VCPHIP_PLANES_CASE(VCPHIP_DR_PI, false, true)
+    VCPHIP_PLANES_CASE(VCPHIP_DR_PP, false, false)
+    default: return -1;
+  }
+#undef VCPHIP_PLANES_CASE
+  return hipGetLastError() == hipSuccess ? 0 : -3;
+}
+
+int vcphip_launch_drsyrk_planes(int interval, int k, int n, const double* A, long lda, double* P, double* C, long ldc,
+                                int rows, hipStream_t s) {
   if (n <= 0) return 0;
   const int npad = (n + BN - 1) / BN * BN, kpad = (k + BK - 1) / BK * BK;
-  if (kpad == 0) return -1;   // k = 0 takes the tile path
-  const dim3 gb(kpad / 32 + (kpad % 32 != 0), npad / 32);
+  if (kpad == 0 || (rows != 64 && rows != 32)) return -1;   // k = 0 takes the tile path
+  const size_t nb = (size_t)((kpad + 31) / 32) * (npad / 32);
+  if (nb > 0x7FFFFFFFu) return -7;
+  const dim3 gb((unsigned)nb);
   const int nt = npad / BN;
+  const dim3 grid((unsigned)((64 / rows) * (nt * (nt + 1) / 2)));
   if (interval) {
-    hipLaunchKernelGGL(k_planes_bt<true>, gb, dim3(256), 0, s, k, n, kpad, npad, A, lda, P0, P1);
-    hipLaunchKernelGGL(k_drsyrk_planes<true>, dim3(nt * (nt + 1) / 2), dim3(NT), 0, s, n, npad, kpad, P0, P1, C, ldc);
+    hipLaunchKernelGGL((k_planes<true, true>), gb, dim3(256), 0, s, 0, n, k, 64, npad, kpad, 0u, A, lda, A, lda, P, P);
+    if (rows == 64) hipLaunchKernelGGL((k_drsyrk_planes<true, 16>), grid, dim3(NT), 0, s, n, npad, kpad, P, C, ldc);
+    else hipLaunchKernelGGL((k_drsyrk_planes<true, 8>), grid, dim3(NT), 0, s, n, npad, kpad, P, C, ldc);
   } else {
-    hipLaunchKernelGGL(k_planes_bt<false>, gb, dim3(256), 0, s, k, n, kpad, npad, A, lda, P0, P1);
-    hipLaunchKernelGGL(k_drsyrk_planes<false>, dim3(nt * (nt + 1) / 2), dim3(NT), 0, s, n, npad, kpad, P0, P1, C, ldc);
+    hipLaunchKernelGGL((k_planes<false, false>), gb, dim3(256), 0, s, 0, n, k, 64, npad, kpad, 0u, A, lda, A, lda, P, P);
+    if (rows == 64) hipLaunchKernelGGL((k_drsyrk_planes<false, 16>), grid, dim3(NT), 0, s, n, npad, kpad, P, C, ldc);
+    else hipLaunchKernelGGL((k_drsyrk_planes<false, 8>), grid, dim3(NT), 0, s, n, npad, kpad, P, C, ldc);
   }
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
@@ -1249,10 +1137,16 @@ int vcphip_launch_drsyrk(int interval, int k, int n, const double* A, long lda, 
 }
 
 int vcphip_launch_igemm_tiles(int n64, int n32, const VcphipResidTile* tiles, const VcphipIgemmProblem* probs,
-                              int grid64, int grid32, unsigned* queue, hipStream_t s) {
+                              int grid64, int grid32, bool big, unsigned* queue, hipStream_t s) {
   if (n64 > 0 || n32 > 0) hipLaunchKernelGGL(k_queue_reset, dim3(1), dim3(64), 0, s, queue);
-  if (n64 > 0) hipLaunchKernelGGL(k_igemm_tiles<4>, dim3(grid64), dim3(NT), 0, s, n64, tiles, probs, queue);
-  if (n32 > 0) hipLaunchKernelGGL(k_igemm_tiles<2>, dim3(grid32), dim3(NT), 0, s, n32, tiles + n64, probs, queue + 1);
+  if (n64 > 0) {
+    if (big) hipLaunchKernelGGL((k_igemm_tiles<4, true>), dim3(grid64), dim3(NT), 0, s, n64, tiles, probs, queue);
+    else hipLaunchKernelGGL((k_igemm_tiles<4, false>), dim3(grid64), dim3(NT), 0, s, n64, tiles, probs, queue);
+  }
+  if (n32 > 0) {
+    if (big) hipLaunchKernelGGL((k_igemm_tiles<2, true>), dim3(grid32), dim3(NT), 0, s, n32, tiles + n64, probs, queue + 1);
+    else hipLaunchKernelGGL((k_igemm_tiles<2, false>), dim3(grid32), dim3(NT), 0, s, n32, tiles + n64, probs, queue + 1);
+  }
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
@@ -1263,17 +1157,23 @@ int vcphip_fill_f64(double* p, long n, double v, hipStream_t s) {
 }
 
 int vcphip_launch_resid_tiles(int n64, int n32, const VcphipResidTile* tiles, const VcphipResidProblem* probs,
-                              int grid64, int grid32, unsigned* queue, hipStream_t s) {
+                              int grid64, int grid32, bool big, unsigned* queue, hipStream_t s) {
   if (n64 > 0 || n32 > 0) hipLaunchKernelGGL(k_queue_reset, dim3(1), dim3(64), 0, s, queue);
-  if (n64 > 0) hipLaunchKernelGGL(k_resid_tiles<4>, dim3(grid64), dim3(NT), 0, s, n64, tiles, probs, queue);
-  if (n32 > 0) hipLaunchKernelGGL(k_resid_tiles<2>, dim3(grid32), dim3(NT), 0, s, n32, tiles + n64, probs, queue + 1);
+  if (n64 > 0) {
+    if (big) hipLaunchKernelGGL((k_resid_tiles<4, true>), dim3(grid64), dim3(NT), 0, s, n64, tiles, probs, queue);
+    else hipLaunchKernelGGL((k_resid_tiles<4, false>), dim3(grid64), dim3(NT), 0, s, n64, tiles, probs, queue);
+  }
+  if (n32 > 0) {
+    if (big) hipLaunchKernelGGL((k_resid_tiles<2, true>), dim3(grid32), dim3(NT), 0, s, n32, tiles + n64, probs, queue + 1);
+    else hipLaunchKernelGGL((k_resid_tiles<2, false>), dim3(grid32), dim3(NT), 0, s, n32, tiles + n64, probs, queue + 1);
+  }
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
 int vcphip_launch_resid(int n64, int n32, const VcphipResidTile* tiles, const VcphipResidProblem* probs, int nblk,
                         const VcphipResidTile* row_block, double* rowsum, int count, double* normub, int grid64,
-                        int grid32, unsigned* queue, hipStream_t s) {
-  vcphip_launch_resid_tiles(n64, n32, tiles, probs, grid64, grid32, queue, s);
+                        int grid32, bool big, unsigned* queue, hipStream_t s) {
+  vcphip_launch_resid_tiles(n64, n32, tiles, probs, grid64, grid32, big, queue, s);
   if (nblk > 0)
     hipLaunchKernelGGL(k_resid_rowsum, dim3(nblk), dim3(VcphipThin<ResidRowSum, 1>::NT), 0, s, row_block, probs, rowsum);
   if (count > 0) hipLaunchKernelGGL(k_resid_max, dim3(count), dim3(256), 0, s, count, probs, rowsum, normub);

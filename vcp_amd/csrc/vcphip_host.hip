@@ -816,18 +816,27 @@ extern "C" int vcphip_igemm_ozaki_noalloc_dev(vcphip_ctx* c, int m, int n, int k
 
 namespace {
 
-// Tile rows of a plane-fed product.  The 32-row tiles give a CU more
-// resident waves (3 against 2 per SIMD for interval x interval, 4-6 against
-// 3-5 for the other forms) and a finer last round of tiles, at 1.5x the LDS
-// reads per FMA; measured on MI355X they are the faster choice up to about 4
-// (interval x interval) or 3 (the other forms) 64-row tiles per CU: n = 2048
-// interval x interval 1.43 against 1.55 ms, n = 1024 0.21 against 0.25 ms,
-// while from n = 3072 the 64-row tiles are 3-8% faster.
-int plane_rows(const vcphip_ctx* c, int kind, size_t mpad, size_t npad) {
+// Tile rows of a plane-fed product.  Both heights keep a wave's multiply-adds
+// at the same LDS reads per k; the 32-row tiles give twice the workgroups, the
+// 64-row ones twice the multiply-adds per read and barrier.  Measured on
+// MI355X (interval x interval / point RU-RD, 32 against 64 rows): n = 512 60
+// against 96 us / 58 against 80, 1024 204 against 203 / 129 against 161, 1536
+// 594 against 631 / 371 against 402, 2048 (4 64-row tiles per CU) 1218 against
+// 1153 / 708 against 689, 3072 4181 against 3900: 32 rows up to 3 per CU.
+int plane_rows(const vcphip_ctx* c, size_t mpad, size_t npad) {
   if (c->plane_rows) return (int)c->plane_rows;
   const size_t cus = c->num_cu > 0 ? (size_t)c->num_cu : 256;
-  const size_t per_cu = kind == VCPHIP_DR_II ? 4 : 3;
-  return (mpad / 64) * (npad / 64) <= per_cu * cus ? 32 : 64;
+  return (mpad / 64) * (npad / 64) <= 3 * cus ? 32 : 64;
+}
+
+// the same choice for the upper-triangle tiles of A^T A, whose 64-row interval
+// form holds five chains (192 registers, two waves per SIMD, against three
+// waves with 32 rows): n = 1500 775 against 952 us, 3000 (4.4 64-row tiles per
+// CU) 1512 against 1641
+int syrk_rows(const vcphip_ctx* c, size_t npad) {
+  if (c->plane_rows) return (int)c->plane_rows;
+  const size_t cus = c->num_cu > 0 ? (size_t)c->num_cu : 256, nt = npad / 64;
+  return nt * (nt + 1) / 2 <= 5 * cus ? 32 : 64;
 }
 
 // Whether a single product takes the row-serial form (one launch, 8 rows per
@@ -870,16 +879,13 @@ int planes_product(vcphip_ctx* c, int kind, int m, int n, int k, const double* A
   void* base;
   int rc = ws_get(c, vcphip_ctx::WS_MR, sizeof(double) * (na + nb), &base);
   if (rc) return rc;
-  double* A0 = (double*)base;
-  double* A1 = A0 + mpad * kpad;   // rad(A) when A is an interval
-  double* B0 = A0 + na;
-  double* B1 = B0 + kpad * npad;   // rad(B) when B is an interval
-  rc = check_launch(vcphip_launch_planes(kind, m, n, k, A, lda, B, ldb, A0, ai ? A1 : nullptr, B0,
-                                         bi ? B1 : nullptr, c->stream));
+  double* PA = (double*)base;
+  double* PB = PA + na;
+  rc = check_launch(vcphip_launch_planes(kind, m, n, k, A, lda, B, ldb, PA, PB, c->stream));
   T.mark("planes");
   if (rc) return rc;
-  rc = check_launch(vcphip_launch_drgemm_planes(kind, m, n, k, A0, ai ? A1 : nullptr, B0, bi ? B1 : nullptr, C, ldc,
-                                                C2, accumulate, plane_rows(c, kind, mpad, npad), c->stream));
+  rc = check_launch(vcphip_launch_drgemm_planes(kind, m, n, k, PA, PB, C, ldc, C2, accumulate,
+                                                plane_rows(c, mpad, npad), c->stream));
   T.mark("drgemm");
   return rc;
 }
@@ -896,9 +902,8 @@ int syrk_planes(vcphip_ctx* c, int interval, int k, int n, const double* A, int 
   void* base;
   int rc = ws_get(c, vcphip_ctx::WS_MR, sizeof(double) * (interval ? 2 : 1) * kpad * npad, &base);
   if (rc) return rc;
-  double* P0 = (double*)base;
-  rc = check_launch(vcphip_launch_drsyrk_planes(interval, k, n, A, lda, P0, interval ? P0 + kpad * npad : nullptr, C,
-                                                ldc, c->stream));
+  rc = check_launch(vcphip_launch_drsyrk_planes(interval, k, n, A, lda, (double*)base, C, ldc, syrk_rows(c, npad),
+                                                c->stream));
   T.mark("drsyrk");
   return rc;
 }
@@ -1128,6 +1133,18 @@ std::vector<VcphipResidTile> tile_array(const TileSet& s) {
   return all;
 }
 
+// whether some operand of the set needs the tiles' 64-bit addresses
+bool big_lds(const std::vector<VcphipIgemmProblem>& probs) {
+  for (const auto& p : probs)
+    if (p.lda >= VCPHIP_TILE_LDMAX || p.ldb >= VCPHIP_TILE_LDMAX) return true;
+  return false;
+}
+bool big_lds(const std::vector<VcphipResidProblem>& probs) {
+  for (const auto& p : probs)
+    if (p.ldr >= VCPHIP_TILE_LDMAX || p.lda >= VCPHIP_TILE_LDMAX) return true;
+  return false;
+}
+
 TileSet igemm_tiles(const vcphip_ctx* c, const std::vector<VcphipIgemmProblem>& probs) {
   // problems with the most work first (longest-processing-time order)
   std::vector<int> order(probs.size());
@@ -1311,7 +1328,7 @@ extern "C" int vcphip_igemm_batched_dev(vcphip_ctx* c, int count, const int* m, 
       return VCPHIP_ERR_OOM;
     }
     auto launch = [&]() {
-      return vcphip_launch_igemm_tiles(g.n64, g.n32, dt, dp, g.grid, g.grid32, queue, c->stream);
+      return vcphip_launch_igemm_tiles(g.n64, g.n32, dt, dp, g.grid, g.grid32, big_lds(probs), queue, c->stream);
     };
     bool captured = false;
     if (hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal) == hipSuccess) {
@@ -1410,9 +1427,10 @@ extern "C" int vcphip_residual_batched_dev(vcphip_ctx* c, int count, const int* 
       return VCPHIP_ERR_OOM;
     }
     bool captured = false;
+    const bool big = big_lds(probs);
     if (hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal) == hipSuccess) {
       const int lrc = vcphip_launch_resid(rs.n64, rs.n32, dt, dp, nblk, drp, drs, count, normub_dev, rs.grid,
-                                          rs.grid32, queue, c->stream);
+                                          rs.grid32, big, queue, c->stream);
       hipGraph_t g = nullptr;
       if (hipStreamEndCapture(c->stream, &g) == hipSuccess && lrc == 0 && g &&
           graph_has_kernels(g, (size_t)vcphip_resid_kernels(rs.n64, rs.n32, nblk, count))) {
@@ -1433,7 +1451,7 @@ extern "C" int vcphip_residual_batched_dev(vcphip_ctx* c, int count, const int* 
       // the same kernels as direct launches
       StageTimer T(c);
       const int lrc = vcphip_launch_resid(rs.n64, rs.n32, dt, dp, nblk, drp, drs, count, normub_dev, rs.grid,
-                                          rs.grid32, queue, c->stream);
+                                          rs.grid32, big, queue, c->stream);
       T.mark("resid");
       rs.probs.clear();   // nothing cached to replay
       return check_launch(lrc);
@@ -2977,8 +2995,7 @@ extern "C" int vcphip_tune_igemm_moduli_dev(vcphip_ctx* c, int m, int n, int k, 
   double* Co = (double*)(b8 + o_o);
   double* part = (double*)(b8 + o_m);
   if ((rc = check_launch(vcphip_gather_rows(IA, lda, m, k, s, As, c->stream)))) return rc;
-  if ((rc = check_launch(vcphip_launch_drgemm(VCPHIP_DR_II, s, n, k, As, s, IB, ldb, Cp, s, nullptr, 0, c->stream))))
-    return rc;
+  if ((rc = planes_product(c, VCPHIP_DR_II, s, n, k, As, s, IB, ldb, Cp, s))) return rc;
   const long long saved = c->oz_nmod, saved_rad = c->oz_radius;
   const long long saved_timing = c->timing;
   c->timing = 0;
@@ -3052,6 +3069,7 @@ extern "C" int vcphip_tune_residual_dev(vcphip_ctx* c, int count, const int* n, 
   if (rs.probs.empty() || !rs.dp) return VCPHIP_ERR_UNSUPPORTED;
   const std::vector<VcphipResidProblem> probs = rs.probs;
   const VcphipResidProblem* dp = rs.dp;
+  const bool big = big_lds(probs);
   // the tile launches of the set under the current shape table and a grid of
   // `per` workgroups per CU, from a tile array of the tuner's own
   int per = c->resid_per_cu;
@@ -3070,8 +3088,8 @@ extern "C" int vcphip_tune_residual_dev(vcphip_ctx* c, int count, const int* n, 
     // time_runs synchronises the stream before `tiles` goes out of scope
     unsigned* queue = batch_queue(c);
     if (!queue) return VCPHIP_ERR_OOM;
-    return time_runs(c, [&]() { return vcphip_launch_resid_tiles(n64, n32, dt, dp, g64, g32, queue, c->stream); }, 5,
-                     t);
+    return time_runs(c, [&]() { return vcphip_launch_resid_tiles(n64, n32, dt, dp, g64, g32, big, queue, c->stream); },
+                     5, t);
   };
   std::vector<int> rows((size_t)count);
   std::vector<double> work((size_t)count);
@@ -3126,6 +3144,7 @@ extern "C" int vcphip_tune_igemm_batched_dev(vcphip_ctx* c, int count, const int
   if (g.probs.empty() || !g.dp) return VCPHIP_ERR_UNSUPPORTED;
   const std::vector<VcphipIgemmProblem> probs = g.probs;
   const VcphipIgemmProblem* dp = g.dp;
+  const bool big = big_lds(probs);
   auto time_set = [&](double* t) -> int {
     TileSet ts = igemm_tiles(c, probs);
     const int n64 = (int)ts.t64.size(), n32 = (int)ts.t32.size();
@@ -3140,8 +3159,8 @@ extern "C" int vcphip_tune_igemm_batched_dev(vcphip_ctx* c, int count, const int
       return VCPHIP_ERR_DEVICE;
     unsigned* queue = batch_queue(c);
     if (!queue) return VCPHIP_ERR_OOM;
-    return time_runs(c, [&]() { return vcphip_launch_igemm_tiles(n64, n32, dt, dp, g64, g32, queue, c->stream); }, 5,
-                     t);
+    return time_runs(c, [&]() { return vcphip_launch_igemm_tiles(n64, n32, dt, dp, g64, g32, big, queue, c->stream); },
+                     5, t);
   };
   std::vector<int> rows((size_t)count);
   std::vector<double> work((size_t)count);

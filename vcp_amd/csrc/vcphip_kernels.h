@@ -13,23 +13,22 @@ enum { VCPHIP_DR_II = 0, VCPHIP_DR_IP = 1, VCPHIP_DR_PI = 2, VCPHIP_DR_PP = 3 };
 // plain FP64 directed-rounding GEMM family (kern_drgemm.hip)
 int vcphip_launch_isgemm(int m, int n, int k, const double* A, long lda, const double* B, long ldb, double* C,
                          long ldc, hipStream_t s);
-// the single products in two steps: planes of A (column-major, mpad x kpad;
-// mid and rad of an interval A, or A itself) and of B (row-major, kpad x
-// npad; mid and rad, or B), zero-padded to mpad, npad = ceil64, kpad =
-// ceil16, then the product from them (k > 0) in tiles of `rows` (64 or 32)
-// x 64 outputs.  A1 / B1 are unused for a point operand.
+// the single products in two steps: planes of A (kpad x mpad, rows
+// contiguous; (mid, rad) pairs of an interval A, or A itself) and of B (kpad x
+// npad, columns contiguous; pairs, or B), zero-padded to mpad, npad = ceil64,
+// kpad = ceil16, then the product from them (k > 0) in tiles of `rows` (64 or
+// 32) x 64 outputs
 int vcphip_launch_planes(int kind, int m, int n, int k, const double* A, long lda, const double* B, long ldb,
-                         double* A0, double* A1, double* B0, double* B1, hipStream_t s);
-int vcphip_launch_drgemm_planes(int kind, int m, int n, int k, const double* A0, const double* A1, const double* B0,
-                                const double* B1, double* C, long ldc, double* C2, int accumulate, int rows,
-                                hipStream_t s);
+                         double* PA, double* PB, hipStream_t s);
+int vcphip_launch_drgemm_planes(int kind, int m, int n, int k, const double* PA, const double* PB, double* C, long ldc,
+                                double* C2, int accumulate, int rows, hipStream_t s);
 // the single products in the row-serial form (few columns or small sizes), k > 0
 int vcphip_launch_drgemm_thin(int kind, int m, int n, int k, const double* A, long lda, const double* B, long ldb,
                               double* C, long ldc, double* C2, int accumulate, hipStream_t s);
-// A^T A (interval or point, A k x n) from the planes of A (made here into
-// P0 / P1, each kpad x npad doubles; P1 unused for a point A); k > 0
-int vcphip_launch_drsyrk_planes(int interval, int k, int n, const double* A, long lda, double* P0, double* P1,
-                                double* C, long ldc, hipStream_t s);
+// A^T A (interval or point, A k x n) from the planes of A (made here into P:
+// kpad x npad pairs or doubles); k > 0, tiles of `rows` (64 or 32) x 64
+int vcphip_launch_drsyrk_planes(int interval, int k, int n, const double* A, long lda, double* P, double* C, long ldc,
+                                int rows, hipStream_t s);
 int vcphip_launch_drgemm(int kind, int m, int n, int k, const double* A, long lda, const double* B,
                          long ldb, double* C, long ldc, double* C2, int accumulate, hipStream_t s);
 // C = A^T A forms (pidblas::mulltmm / vmulmm), kern_drgemm.hip
@@ -64,16 +63,19 @@ struct VcphipIgemmProblem {
 // tiles[0, n64) are 64 x 64 tiles, tiles[n64, n64 + n32) 32 x 64 ones; each
 // shape's persistent grid takes its part's tiles from a work queue: queue[0]
 // and queue[1] (device counters, zeroed by a kernel these launchers enqueue
-// first; one pair per stream of launches)
+// first; one pair per stream of launches).  big: some operand's leading
+// dimension is VCPHIP_TILE_LDMAX or more (the tiles then address it with 64
+// bits; below, 16 bytes x 64 columns x the leading dimension stay within 2^31)
+#define VCPHIP_TILE_LDMAX (1 << 21)
 int vcphip_launch_igemm_tiles(int n64, int n32, const VcphipResidTile* tiles, const VcphipIgemmProblem* probs,
-                              int grid64, int grid32, unsigned* queue, hipStream_t s);
+                              int grid64, int grid32, bool big, unsigned* queue, hipStream_t s);
 // row_block: the problems' blocks of 8 rows {problem, first row}
 int vcphip_launch_resid(int n64, int n32, const VcphipResidTile* tiles, const VcphipResidProblem* probs, int nblk,
                         const VcphipResidTile* row_block, double* rowsum, int count, double* normub, int grid64,
-                        int grid32, unsigned* queue, hipStream_t s);
+                        int grid32, bool big, unsigned* queue, hipStream_t s);
 // the tile launches alone (the tuner times them)
 int vcphip_launch_resid_tiles(int n64, int n32, const VcphipResidTile* tiles, const VcphipResidProblem* probs,
-                              int grid64, int grid32, unsigned* queue, hipStream_t s);
+                              int grid64, int grid32, bool big, unsigned* queue, hipStream_t s);
 // the number of kernels vcphip_launch_resid / vcphip_launch_igemm_tiles
 // enqueue for these sizes
 inline int vcphip_igemm_tile_kernels(int n64, int n32) { return (n64 > 0 || n32 > 0) + (n64 > 0) + (n32 > 0); }
