@@ -204,6 +204,20 @@ VCPHIP_DEVINL void oz_pass_planes(const VcphipOzParams& P, int z, int nmod, int&
   pb1 = nmod + P.rpb[r][1];
 }
 
+// plane z and tile of workgroup bid of nwg (see k_oz_gemm5)
+VCPHIP_DEVINL void oz_tile_order(int bid, int nwg, int tiles, int nmod, int by_plane, int& z, int& local) {
+  const int rad = by_plane ? nwg - nmod * tiles : 0;   // workgroups of the radius outputs
+  if (by_plane && bid >= rad) {
+    const int seq = vcphip_xcd_remap(bid - rad, nmod * tiles);
+    z = seq / tiles;
+    local = seq - z * tiles;
+    return;
+  }
+  z = bid / tiles;
+  local = vcphip_xcd_remap(bid - z * tiles, tiles);
+  if (by_plane) z += nmod;
+}
+
 // x (|x| <= 2^62) as the eight bytes of x + 2^63 (its two's complement with
 // the sign bit flipped), held as two byte quads, low byte first
 struct Bytes8 {
@@ -746,8 +760,19 @@ __device__ __forceinline__ void oz_mfma_frag32(const OzFrag32<FM, FN>& f, v16i (
 // NW waves per workgroup in a 2 x (NW / 2) grid: with NW = 8 and 4 x 2
 // fragments (128 x 64 per wave, 128 accumulator registers) the same 256 x 256
 // workgroup tile runs two waves per SIMD, twice the loads in flight per CU.
+// With 2 x 2 fragments and four waves the tile is 128 x 128: 64 KB of LDS, two
+// workgroups per CU, for products that leave the 256 x 256 grid short.
+// by_plane: the residue planes' tiles run as one sequence cut into eight runs,
+// one per XCD, after the radius outputs (whose two-pass tiles are the longest,
+// so they come first), and an XCD's L2 holds one or two planes' operands
+// instead of a part of every plane's.  Otherwise each plane is cut over the
+// XCDs by itself, which keeps all of them on one plane's operands.  int8 stage
+// by plane against cut: n = 1000 44 against 54-61 us, 1500 107 against 114,
+// 2000 203 against 209-228, 4096 1335 against 1343 (a whole dd product 3.07
+// against 2.96 ms), 8192 10.89 against 10.44 ms: planes of up to one 256 x 256
+// tile per two CUs.
 template <int FM, int FN, int NST, int NW = 4>
-__global__ __launch_bounds__(64 * NW) void k_oz_gemm5(int mpad, int npad, int kpad, int nmod, int nz,
+__global__ __launch_bounds__(64 * NW) void k_oz_gemm5(int mpad, int npad, int kpad, int nmod, int by_plane,
                                                       const int8_t* __restrict__ Aplanes,
                                                       const int8_t* __restrict__ Bplanes, VcphipOzParams P,
                                                       uint8_t* __restrict__ U, int32_t* __restrict__ Z) {
@@ -764,8 +789,8 @@ __global__ __launch_bounds__(64 * NW) void k_oz_gemm5(int mpad, int npad, int kp
 
   const int ntm = mpad / TMB, ntn = npad / TNB;
   const int tiles = ntm * ntn;
-  const int z = blockIdx.x / tiles;
-  const int local = vcphip_xcd_remap(blockIdx.x - z * tiles, tiles);
+  int z, local;
+  oz_tile_order(blockIdx.x, gridDim.x, tiles, nmod, by_plane, z, local);
   int tm, tn;
   vcphip_tile_coords(local, ntm, ntn, 8, tm, tn);
   const int row0 = tm * TMB, col0 = tn * TNB;
@@ -1228,11 +1253,13 @@ int vcphip_oz_split_cols(const double* B, long ldb, int k, int n, int npad, int 
 // 8 / 9 / 10 = k_oz_gemm4 256 x 256 with 4 / 3 stages, 128 x 256 with 4;
 // 13 / 14 = k_oz_gemm4 256 x 256 with the refill loads spread over the
 // MFMAs (4 / 3 stages); 11 / 12 = k_oz_gemm5 (32 x 32 x 32 MFMA, 4 waves,
-// 4 / 3 stages); 15 / 16 = k_oz_gemm5 with 8 waves of 128 x 64 (4 / 3 stages)
+// 4 / 3 stages); 15 / 16 = k_oz_gemm5 with 8 waves of 128 x 64 (4 / 3 stages);
+// VCPHIP_OZ_TILE128 = k_oz_gemm5 128 x 128, four waves of 64 x 64
 int vcphip_oz_gemm(int mpad, int npad, int kpad, int nmod, int nrad, const int8_t* Aplanes,
                    const int8_t* Bplanes, const VcphipOzParams& P, uint8_t* U, int32_t* Z, int variant,
                    hipStream_t s) {
   const int nz = nmod + nrad;
+  const int by_plane = (long)(mpad / 128) * (npad / 128) <= 4 * 128;   // k_oz_gemm5
   switch (variant) {
     case 6:
     case 7: {
@@ -1281,10 +1308,10 @@ int vcphip_oz_gemm(int mpad, int npad, int kpad, int nmod, int nrad, const int8_
       if (kpad % 64) return -7;
       const int tiles = (mpad / 256) * (npad / 256);
       if (variant == 11)
-        hipLaunchKernelGGL((k_oz_gemm5<4, 4, 4>), dim3(tiles * nz), dim3(256), 0, s, mpad, npad, kpad, nmod, nz,
+        hipLaunchKernelGGL((k_oz_gemm5<4, 4, 4>), dim3(tiles * nz), dim3(256), 0, s, mpad, npad, kpad, nmod, by_plane,
                            Aplanes, Bplanes, P, U, Z);
       else
-        hipLaunchKernelGGL((k_oz_gemm5<4, 4, 3>), dim3(tiles * nz), dim3(256), 0, s, mpad, npad, kpad, nmod, nz,
+        hipLaunchKernelGGL((k_oz_gemm5<4, 4, 3>), dim3(tiles * nz), dim3(256), 0, s, mpad, npad, kpad, nmod, by_plane,
                            Aplanes, Bplanes, P, U, Z);
       break;
     }
@@ -1293,10 +1320,10 @@ int vcphip_oz_gemm(int mpad, int npad, int kpad, int nmod, int nrad, const int8_
       if (kpad % 64) return -7;
       const int tiles = (mpad / 256) * (npad / 256);
       if (variant == 15)
-        hipLaunchKernelGGL((k_oz_gemm5<4, 2, 4, 8>), dim3(tiles * nz), dim3(512), 0, s, mpad, npad, kpad, nmod, nz,
+        hipLaunchKernelGGL((k_oz_gemm5<4, 2, 4, 8>), dim3(tiles * nz), dim3(512), 0, s, mpad, npad, kpad, nmod, by_plane,
                            Aplanes, Bplanes, P, U, Z);
       else
-        hipLaunchKernelGGL((k_oz_gemm5<4, 2, 3, 8>), dim3(tiles * nz), dim3(512), 0, s, mpad, npad, kpad, nmod, nz,
+        hipLaunchKernelGGL((k_oz_gemm5<4, 2, 3, 8>), dim3(tiles * nz), dim3(512), 0, s, mpad, npad, kpad, nmod, by_plane,
                            Aplanes, Bplanes, P, U, Z);
       break;
     }
@@ -1310,6 +1337,13 @@ int vcphip_oz_gemm(int mpad, int npad, int kpad, int nmod, int nrad, const int8_
       else
         hipLaunchKernelGGL((k_oz_gemm6<2>), dim3(tiles * nz), dim3(512), 0, s, mpad, npad, kpad, nmod, nz, Aplanes,
                            Bplanes, P, U, Z);
+      break;
+    }
+    case VCPHIP_OZ_TILE128: {
+      if (kpad % 64 || mpad % 128 || npad % 128) return -7;
+      const int tiles = (mpad / 128) * (npad / 128);
+      hipLaunchKernelGGL((k_oz_gemm5<2, 2, 4>), dim3(tiles * nz), dim3(256), 0, s, mpad, npad, kpad, nmod, by_plane,
+                         Aplanes, Bplanes, P, U, Z);
       break;
     }
     default: return -7;

@@ -161,6 +161,29 @@ enum { TUNE_IGEMM = 1, TUNE_DDGEMM = 2 };
 // dd 2.03 against 2.10 ms)
 constexpr int DEFAULT_VARIANT = 15;
 
+// the tile an int8 product of nz planes runs, and the padded m and n it takes:
+// the set or tuned variant, else 256 x 256, or 128 x 128 where that grid is
+// short or mostly padding.  Two 128 x 128 workgroups share a CU and hide each
+// other's prologue, but read twice the operand bytes from LDS per product and
+// run at 0.83-0.87 of the rate once the chip is full (n = 4096 1.54 against
+// 1.34 ms).  int8 stage, 128 against 256 (interval form, 22 planes): n = 200
+// 10.3 against 15.4 us, 500 15.8 against 22.2, 800 32 against 39, 1000 (352
+// tiles of 256) 41 against 42, 1000 x 2000 x 2000 (704) 115 against 105; by
+// padding 1050 57 against 68, 1300 (0.84 of the padded area) 82 against 95,
+// 100 x 4000 x 1000 30 against 42.
+struct OzTile {
+  int variant = 0, mpad = 0, npad = 0;
+};
+OzTile oz_tile(const vcphip_ctx* c, int variant, int m, int n, int nz) {
+  const auto up = [](int x, int to) { return (int)(((long)x + to - 1) / to * to); };
+  OzTile t{variant ? variant : DEFAULT_VARIANT, up(m, VCPHIP_OZ_PADMN), up(n, VCPHIP_OZ_PADMN)};
+  if (variant) return t;
+  const long cus = c->num_cu > 0 ? c->num_cu : 256;
+  const OzTile h{VCPHIP_OZ_TILE128, up(m, 128), up(n, 128)};
+  const long area = (long)t.mpad * t.npad, harea = (long)h.mpad * h.npad;
+  return area / (256 * 256) * nz <= 2 * cus || 20 * harea <= 17 * area ? h : t;
+}
+
 int size_class(int x) {
   int l = 0;
   while (l < 31 && (1 << l) < x) ++l;
@@ -670,7 +693,8 @@ static int dims_ok(int m, int n, int k) { return m >= 0 && n >= 0 && k >= 0; }
 // interval Ozaki product in this context
 struct OzPlan {
   VcphipOzParams P;
-  int nmod = 0, nz = 0, variant = 0, mpad = 0, npad = 0, kpad = 0, nchunk = 0;
+  int nmod = 0, nz = 0, kpad = 0, nchunk = 0;
+  OzTile tile;
   size_t b_pa = 0, b_pb = 0, b_pu = 0, b_pz = 0, b_sa = 0, b_sb = 0;   // bytes of each workspace buffer
 };
 
@@ -682,15 +706,16 @@ static int oz_plan(vcphip_ctx* c, int m, int n, int k, OzPlan& p) {
   if (rc) return rc;
   oz_set_radius(&p.P, oz_radius_scheme(c, tuned, k));
   p.nz = p.P.rnz;
-  p.variant = c->oz_variant ? (int)c->oz_variant : (tuned && tuned->variant ? tuned->variant : DEFAULT_VARIANT);
-  p.mpad = (m + VCPHIP_OZ_PADMN - 1) / VCPHIP_OZ_PADMN * VCPHIP_OZ_PADMN;
-  p.npad = (n + VCPHIP_OZ_PADMN - 1) / VCPHIP_OZ_PADMN * VCPHIP_OZ_PADMN;
+  p.tile = oz_tile(c, c->oz_variant ? (int)c->oz_variant : (tuned ? tuned->variant : 0), m, n, p.nmod + p.nz);
+  // the buffers of the widest padding, whichever tile runs
+  const size_t mpad = ((size_t)m + VCPHIP_OZ_PADMN - 1) / VCPHIP_OZ_PADMN * VCPHIP_OZ_PADMN;
+  const size_t npad = ((size_t)n + VCPHIP_OZ_PADMN - 1) / VCPHIP_OZ_PADMN * VCPHIP_OZ_PADMN;
   p.kpad = k > 0 ? (k + VCPHIP_OZ_PADK - 1) / VCPHIP_OZ_PADK * VCPHIP_OZ_PADK : VCPHIP_OZ_PADK;
   p.nchunk = k > 0 ? (k + VCPHIP_OZ_CHUNK - 1) / VCPHIP_OZ_CHUNK : 0;
-  p.b_pa = ((size_t)p.nmod + VCPHIP_OZ_NDIGIT_A) * p.mpad * p.kpad;
-  p.b_pb = ((size_t)p.nmod + VCPHIP_OZ_NDIGIT_B) * p.npad * p.kpad;
-  p.b_pu = (size_t)p.nmod * p.mpad * p.npad;
-  p.b_pz = (size_t)p.nz * sizeof(int32_t) * (size_t)p.mpad * p.npad;
+  p.b_pa = ((size_t)p.nmod + VCPHIP_OZ_NDIGIT_A) * mpad * p.kpad;
+  p.b_pb = ((size_t)p.nmod + VCPHIP_OZ_NDIGIT_B) * npad * p.kpad;
+  p.b_pu = (size_t)p.nmod * mpad * npad;
+  p.b_pz = (size_t)p.nz * sizeof(int32_t) * (size_t)mpad * npad;
   auto side_bytes = [&](int rows) {
     return (size_t)rows * (4 * sizeof(int) + sizeof(double)) +
            sizeof(double) * 5 * (size_t)(p.nchunk > 0 ? p.nchunk : 1) * rows + 1024;
@@ -717,7 +742,7 @@ static int oz_run(vcphip_ctx* c, const OzPlan& p, int m, int n, int k, const dou
     return s;
   };
   const VcphipOzSide SA = carve(sa, m), SB = carve(sb, n);
-  const int mpad = p.mpad, npad = p.npad, kpad = p.kpad;
+  const int mpad = p.tile.mpad, npad = p.tile.npad, kpad = p.kpad;
   int rc;
   StageTimer T(c, timed);
   if ((rc = check_launch(vcphip_oz_stats(A, 1, lda, m, k, SA, c->stream)))) return rc;
@@ -727,7 +752,7 @@ static int oz_run(vcphip_ctx* c, const OzPlan& p, int m, int n, int k, const dou
   if ((rc = check_launch(vcphip_oz_split_cols(B, ldb, k, n, npad, kpad, p.P, SB, (int8_t*)pb, c->stream)))) return rc;
   T.mark("split");
   if ((rc = check_launch(vcphip_oz_gemm(mpad, npad, kpad, p.nmod, p.nz, (const int8_t*)pa, (const int8_t*)pb, p.P,
-                                        (uint8_t*)pu, (int32_t*)pz, p.variant, c->stream))))
+                                        (uint8_t*)pu, (int32_t*)pz, p.tile.variant, c->stream))))
     return rc;
   T.mark("gemm");
   if ((rc = check_launch(vcphip_oz_recon(m, n, k, mpad, npad, p.P, SA, SB, (const uint8_t*)pu,
@@ -985,8 +1010,9 @@ static int dd_gemm_dev(vcphip_ctx* c, bool tn, int m, int n, int k, const double
   VcphipOzParams P;
   int rc = dd_make_params(k, nmod, &P);
   if (rc) return rc;
-  const int mpad = (m + VCPHIP_OZ_PADMN - 1) / VCPHIP_OZ_PADMN * VCPHIP_OZ_PADMN;
-  const int npad = (n + VCPHIP_OZ_PADMN - 1) / VCPHIP_OZ_PADMN * VCPHIP_OZ_PADMN;
+  const vcphip_ctx::Tune* tuned = tune_find(c, TUNE_DDGEMM, m, n, k);
+  const OzTile tile = oz_tile(c, c->oz_variant ? (int)c->oz_variant : (tuned ? tuned->variant : 0), m, n, nmod);
+  const int mpad = tile.mpad, npad = tile.npad;
   const int kpad = k > 0 ? (k + VCPHIP_OZ_PADK - 1) / VCPHIP_OZ_PADK * VCPHIP_OZ_PADK : VCPHIP_OZ_PADK;
   const int nchunk = k > 0 ? (k + VCPHIP_DD_CHUNK - 1) / VCPHIP_DD_CHUNK : 1;
   void *pa = nullptr, *pb, *pu, *st;
@@ -1014,11 +1040,9 @@ static int dd_gemm_dev(vcphip_ctx* c, bool tn, int m, int n, int k, const double
     return rc;
   if ((rc = check_launch(vcphip_dd_split_cols(B, ldb, k, n, npad, kpad, P, eb, fb, (int8_t*)pb, c->stream)))) return rc;
   T.mark("split");
-  const vcphip_ctx::Tune* tuned = tune_find(c, TUNE_DDGEMM, m, n, k);
-  const int variant = c->oz_variant ? (int)c->oz_variant : (tuned && tuned->variant ? tuned->variant : DEFAULT_VARIANT);
   const int8_t* Aplanes = tn ? (const int8_t*)pb : (const int8_t*)pa;
   if ((rc = check_launch(vcphip_oz_gemm(mpad, npad, kpad, nmod, 0, Aplanes, (const int8_t*)pb, P, (uint8_t*)pu,
-                                        nullptr, variant, c->stream))))
+                                        nullptr, tile.variant, c->stream))))
     return rc;
   T.mark("gemm");
   if ((rc = check_launch(vcphip_dd_recon(m, n, mpad, npad, P, tn ? eb : ea, tn ? fb : fa, eb, fb, (const uint8_t*)pu,
