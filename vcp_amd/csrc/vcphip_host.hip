@@ -345,23 +345,12 @@ int oz_moduli(int nmod, int* out) {
   return cnt;
 }
 
-// CRT constants shared by the interval and dd forms; beta from the no-wrap
-// condition k (2^beta + slack)^2 < M/2, i.e. k 2^(2 beta + extra) < M
-int oz_fill_params(int k, int nmod, int extra, int beta_cap, VcphipOzParams* P) {
+// the CRT constants of nmod moduli (everything but beta, which depends on k)
+int oz_constants(int nmod, VcphipOzParams* P) {
   memset(P, 0, sizeof(*P));
   P->dmask_a = P->dmask_b = ~0;   // every digit plane until a radius scheme is set
-  if (nmod < 8 || nmod > VCPHIP_OZ_MAXMOD) return VCPHIP_ERR_ARGUMENT;
   if (oz_moduli(nmod, P->mod) != nmod) return VCPHIP_ERR_ARGUMENT;
   P->nmod = nmod;
-  {
-    double lm = 0.0;
-    for (int t = 0; t < nmod; ++t) lm += log2((double)P->mod[t]);
-    int lk = 0;
-    while ((1ll << lk) < (long long)(k > 1 ? k : 1)) ++lk;
-    const int beta = (int)floor((lm - (double)extra - (double)lk - 1e-6) / 2.0);
-    P->beta = beta > beta_cap ? beta_cap : beta;
-  }
-  if (P->beta < 8) return VCPHIP_ERR_UNSUPPORTED;
   for (int t = 0; t < nmod; ++t) {
     const int m = P->mod[t];
     if (m <= 32) return VCPHIP_ERR_UNSUPPORTED;   // the splits' 24-bit quotient needs r_magic < 2^24
@@ -441,6 +430,48 @@ int oz_fill_params(int k, int nmod, int extra, int beta_cap, VcphipOzParams* P) 
   return VCPHIP_OK;
 }
 
+// The constants of each moduli count, formed once per process: long divisions
+// of 256-bit numbers take 10 (16 moduli) to 25 us (32) on the host, and a dd
+// product used to form them for up to nine counts per call (about 100 of the
+// 117 us of a 600 x 600 one).
+struct OzConstants {
+  VcphipOzParams P;
+  double log2M = 0.0;
+  int rc = VCPHIP_ERR_ARGUMENT;
+};
+
+const OzConstants& oz_constants_of(int nmod) {   // 8 <= nmod <= VCPHIP_OZ_MAXMOD
+  static OzConstants table[VCPHIP_OZ_MAXMOD + 1];
+  static std::once_flag once[VCPHIP_OZ_MAXMOD + 1];
+  std::call_once(once[nmod], [nmod] {
+    OzConstants& c = table[nmod];
+    c.rc = oz_constants(nmod, &c.P);
+    for (int t = 0; t < nmod; ++t) c.log2M += log2((double)c.P.mod[t]);
+  });
+  return table[nmod];
+}
+
+// beta from the no-wrap condition k (2^beta + slack)^2 < M/2, i.e.
+// k 2^(2 beta + extra) < M
+int oz_beta(const OzConstants& c, int k, int extra, int beta_cap) {
+  int lk = 0;
+  while ((1ll << lk) < (long long)(k > 1 ? k : 1)) ++lk;
+  const int beta = (int)floor((c.log2M - (double)extra - (double)lk - 1e-6) / 2.0);
+  return beta > beta_cap ? beta_cap : beta;
+}
+
+// CRT constants shared by the interval and dd forms, with the beta of k
+int oz_fill_params(int k, int nmod, int extra, int beta_cap, VcphipOzParams* P) {
+  if (nmod < 8 || nmod > VCPHIP_OZ_MAXMOD) return VCPHIP_ERR_ARGUMENT;
+  const OzConstants& c = oz_constants_of(nmod);
+  const int beta = oz_beta(c, k, extra, beta_cap);
+  if (beta < 8) return VCPHIP_ERR_UNSUPPORTED;
+  if (c.rc) return c.rc;
+  *P = c.P;
+  P->beta = beta;
+  return VCPHIP_OK;
+}
+
 // interval form: |A'| <= 2^beta, k 2^(2 beta + 1) < M, beta <= 62 (int64)
 int oz_make_params(int k, int nmod, VcphipOzParams* P) {
   if (nmod > VCPHIP_OZ_MAXMOD_IV) return VCPHIP_ERR_ARGUMENT;
@@ -454,8 +485,8 @@ int default_dd_nmod(int k) {
   // smallest count giving beta >= 110 (a product accurate to ~2^-108 of the
   // row / column scales, the dd precision)
   for (int nmod = 24; nmod <= VCPHIP_OZ_MAXMOD; ++nmod) {
-    VcphipOzParams P;
-    if (dd_make_params(k, nmod, &P) == VCPHIP_OK && P.beta >= 110) return nmod;
+    const OzConstants& c = oz_constants_of(nmod);
+    if (c.rc == VCPHIP_OK && oz_beta(c, k, 2, 115) >= 110) return nmod;
   }
   return VCPHIP_OZ_MAXMOD;
 }
@@ -693,7 +724,7 @@ static int dims_ok(int m, int n, int k) { return m >= 0 && n >= 0 && k >= 0; }
 // interval Ozaki product in this context
 struct OzPlan {
   VcphipOzParams P;
-  int nmod = 0, nz = 0, kpad = 0, nchunk = 0;
+  int nmod = 0, nz = 0, kpad = 0;
   OzTile tile;
   size_t b_pa = 0, b_pb = 0, b_pu = 0, b_pz = 0, b_sa = 0, b_sb = 0;   // bytes of each workspace buffer
 };
@@ -711,15 +742,11 @@ static int oz_plan(vcphip_ctx* c, int m, int n, int k, OzPlan& p) {
   const size_t mpad = ((size_t)m + VCPHIP_OZ_PADMN - 1) / VCPHIP_OZ_PADMN * VCPHIP_OZ_PADMN;
   const size_t npad = ((size_t)n + VCPHIP_OZ_PADMN - 1) / VCPHIP_OZ_PADMN * VCPHIP_OZ_PADMN;
   p.kpad = k > 0 ? (k + VCPHIP_OZ_PADK - 1) / VCPHIP_OZ_PADK * VCPHIP_OZ_PADK : VCPHIP_OZ_PADK;
-  p.nchunk = k > 0 ? (k + VCPHIP_OZ_CHUNK - 1) / VCPHIP_OZ_CHUNK : 0;
   p.b_pa = ((size_t)p.nmod + VCPHIP_OZ_NDIGIT_A) * mpad * p.kpad;
   p.b_pb = ((size_t)p.nmod + VCPHIP_OZ_NDIGIT_B) * npad * p.kpad;
   p.b_pu = (size_t)p.nmod * mpad * npad;
-  p.b_pz = (size_t)p.nz * sizeof(int32_t) * (size_t)mpad * npad;
-  auto side_bytes = [&](int rows) {
-    return (size_t)rows * (4 * sizeof(int) + sizeof(double)) +
-           sizeof(double) * 5 * (size_t)(p.nchunk > 0 ? p.nchunk : 1) * rows + 1024;
-  };
+  p.b_pz = (size_t)p.nz * sizeof(int32_t) * mpad * npad;
+  auto side_bytes = [&](int rows) { return (size_t)rows * (4 * sizeof(int) + sizeof(double)); };
   p.b_sa = side_bytes(m);
   p.b_sb = side_bytes(n);
   return VCPHIP_OK;
@@ -734,7 +761,6 @@ static int oz_run(vcphip_ctx* c, const OzPlan& p, int m, int n, int k, const dou
     VcphipOzSide s;
     char* q = (char*)base;
     s.n1 = (double*)q; q += sizeof(double) * rows;
-    s.part = (double*)q; q += sizeof(double) * 5 * (size_t)(p.nchunk > 0 ? p.nchunk : 1) * rows;
     s.e = (int*)q; q += sizeof(int) * rows;
     s.g = (int*)q; q += sizeof(int) * rows;
     s.h = (int*)q; q += sizeof(int) * rows;
@@ -745,11 +771,11 @@ static int oz_run(vcphip_ctx* c, const OzPlan& p, int m, int n, int k, const dou
   const int mpad = p.tile.mpad, npad = p.tile.npad, kpad = p.kpad;
   int rc;
   StageTimer T(c, timed);
-  if ((rc = check_launch(vcphip_oz_stats(A, 1, lda, m, k, SA, c->stream)))) return rc;
-  if ((rc = check_launch(vcphip_oz_stats(B, ldb, 1, n, k, SB, c->stream)))) return rc;
+  if ((rc = check_launch(vcphip_oz_stats(A, lda, m, SA, B, ldb, n, SB, k, c->stream)))) return rc;
   T.mark("stats");
-  if ((rc = check_launch(vcphip_oz_split_rows(A, lda, m, k, mpad, kpad, p.P, SA, (int8_t*)pa, c->stream)))) return rc;
-  if ((rc = check_launch(vcphip_oz_split_cols(B, ldb, k, n, npad, kpad, p.P, SB, (int8_t*)pb, c->stream)))) return rc;
+  if ((rc = check_launch(vcphip_oz_split(A, lda, m, mpad, SA, (int8_t*)pa, B, ldb, n, npad, SB, (int8_t*)pb, k, kpad, p.P,
+                                         c->stream))))
+    return rc;
   T.mark("split");
   if ((rc = check_launch(vcphip_oz_gemm(mpad, npad, kpad, p.nmod, p.nz, (const int8_t*)pa, (const int8_t*)pb, p.P,
                                         (uint8_t*)pu, (int32_t*)pz, p.tile.variant, c->stream))))
@@ -830,8 +856,12 @@ extern "C" int vcphip_igemm_ozaki_noalloc_dev(vcphip_ctx* c, int m, int n, int k
   int rc = oz_plan(c, m, n, k, p);
   if (rc) return rc;
   const size_t o_pb = al256(p.b_pa), o_pu = o_pb + al256(p.b_pb), o_pz = o_pu + al256(p.b_pu);
-  const size_t o_sa = o_pz + al256(p.b_pz), o_sb = o_sa + al256(p.b_sa), total = o_sb + al256(p.b_sb);
-  if (total > VCPHIP_NOALLOC_SCRATCH_BYTES) return VCPHIP_ERR_SCRATCH;
+  const size_t o_sa = o_pz + al256(p.b_pz), o_sb = o_sa + al256(p.b_sa);
+  // the limit also counts five doubles per 256 k of each row and column (an
+  // earlier layout's partial norms), so that the sizes refused stay the same
+  const size_t nchunk = k > VCPHIP_OZ_CHUNK ? ((size_t)k + VCPHIP_OZ_CHUNK - 1) / VCPHIP_OZ_CHUNK : 1;
+  auto limit_bytes = [&](size_t side, size_t rows) { return al256(side + sizeof(double) * 5 * nchunk * rows + 1024); };
+  if (o_sa + limit_bytes(p.b_sa, m) + limit_bytes(p.b_sb, n) > VCPHIP_NOALLOC_SCRATCH_BYTES) return VCPHIP_ERR_SCRATCH;
   unsigned char* base = (unsigned char*)scratch_of(c->device);
   if (!base) return VCPHIP_ERR_DEVICE;
   hipSetDevice(c->device);
@@ -1014,31 +1044,23 @@ static int dd_gemm_dev(vcphip_ctx* c, bool tn, int m, int n, int k, const double
   const OzTile tile = oz_tile(c, c->oz_variant ? (int)c->oz_variant : (tuned ? tuned->variant : 0), m, n, nmod);
   const int mpad = tile.mpad, npad = tile.npad;
   const int kpad = k > 0 ? (k + VCPHIP_OZ_PADK - 1) / VCPHIP_OZ_PADK * VCPHIP_OZ_PADK : VCPHIP_OZ_PADK;
-  const int nchunk = k > 0 ? (k + VCPHIP_DD_CHUNK - 1) / VCPHIP_DD_CHUNK : 1;
   void *pa = nullptr, *pb, *pu, *st;
   if (!tn && (rc = ws_get(c, vcphip_ctx::WS_PA, (size_t)nmod * mpad * kpad, &pa))) return rc;
   if ((rc = ws_get(c, vcphip_ctx::WS_PB, (size_t)nmod * npad * kpad, &pb))) return rc;
   if ((rc = ws_get(c, vcphip_ctx::WS_U, (size_t)nmod * mpad * npad, &pu))) return rc;
   const size_t rows_all = (size_t)m + n;
-  if ((rc = ws_get(c, vcphip_ctx::WS_DD, sizeof(int) * (2 * rows_all + (size_t)nchunk * rows_all) + 1024, &st))) return rc;
+  if ((rc = ws_get(c, vcphip_ctx::WS_DD, sizeof(int) * 2 * rows_all, &st))) return rc;
   int* ea = (int*)st;
   int* fa = ea + m;
   int* eb = fa + m;
   int* fb = eb + n;
-  int* part = fb + n;
   StageTimer T(c);
-  if (!tn) {
-    if ((rc = check_launch(ta ? vcphip_dd_stats(A, lda, 1, m, k, ea, fa, part, c->stream)
-                              : vcphip_dd_stats(A, 1, lda, m, k, ea, fa, part, c->stream))))
-      return rc;
-  }
-  if ((rc = check_launch(vcphip_dd_stats(B, ldb, 1, n, k, eb, fb, part, c->stream)))) return rc;
+  const double* Aop = tn ? nullptr : A;   // A^T A: the columns of B = A serve both sides
+  if ((rc = check_launch(vcphip_dd_stats(Aop, lda, m, ta ? 1 : 0, ea, fa, B, ldb, n, eb, fb, k, c->stream)))) return rc;
   T.mark("stats");
-  if (!tn && (rc = check_launch(ta ? vcphip_dd_split_cols(A, lda, k, m, mpad, kpad, P, ea, fa, (int8_t*)pa, c->stream)
-                                   : vcphip_dd_split_rows(A, lda, m, k, mpad, kpad, P, ea, fa, (int8_t*)pa,
-                                                          c->stream))))
+  if ((rc = check_launch(vcphip_dd_split(Aop, lda, m, mpad, ta ? 1 : 0, ea, fa, (int8_t*)pa, B, ldb, n, npad, eb, fb,
+                                         (int8_t*)pb, k, kpad, P, c->stream))))
     return rc;
-  if ((rc = check_launch(vcphip_dd_split_cols(B, ldb, k, n, npad, kpad, P, eb, fb, (int8_t*)pb, c->stream)))) return rc;
   T.mark("split");
   const int8_t* Aplanes = tn ? (const int8_t*)pb : (const int8_t*)pa;
   if ((rc = check_launch(vcphip_oz_gemm(mpad, npad, kpad, nmod, 0, Aplanes, (const int8_t*)pb, P, (uint8_t*)pu,

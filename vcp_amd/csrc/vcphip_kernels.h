@@ -94,7 +94,6 @@ int vcphip_fill_f64(double* p, long n, double v, hipStream_t s);
 // against B's rounded-up digit: 4), ceil 2 (rounded-up digits: 2)
 #define VCPHIP_OZ_MAXRAD 6
 #define VCPHIP_OZ_CHUNK 256   // k-chunk of the upward 1-norm partial sums
-#define VCPHIP_DD_CHUNK 64    // k-chunk of the dd row maxima (a maximum: any split gives the same result)
 #define VCPHIP_OZ_PADMN 256   // m and n are padded to multiples of this (128 for VCPHIP_OZ_TILE128)
 #define VCPHIP_OZ_TILE128 19  // 128 x 128 int8 GEMM tiles (m and n padded to 128); not a settable variant
 #define VCPHIP_OZ_PADK 128    // k is padded to a multiple of this
@@ -171,18 +170,17 @@ struct VcphipOzSide {
   int* h;       // digit scale of rad
   int* flags;   // VCPHIP_OZ_*ZERO: mid / |mid|+rad / rad identically zero
   double* n1;   // upward 1-norm of |mid|
-  double* part; // partials [4][nchunk][rows]
 };
 
-int vcphip_oz_stats(const double* X, long rs, long cs, int rows, int len, VcphipOzSide side,
+// statistics of the rows of A (m x k) and the columns of B (k x n), one launch
+int vcphip_oz_stats(const double* A, long lda, int m, VcphipOzSide sa, const double* B, long ldb, int n,
+                    VcphipOzSide sb, int k, hipStream_t s);
+// planes of both operands, one launch: N residue planes followed by the
+// radius-digit planes (VCPHIP_OZ_NDIGIT_A for A, _B for B), each
+// [rows_pad][kpad] int8 with k contiguous
+int vcphip_oz_split(const double* A, long lda, int m, int mpad, VcphipOzSide sa, int8_t* pa, const double* B, long ldb,
+                    int n, int npad, VcphipOzSide sb, int8_t* pb, int k, int kpad, const VcphipOzParams& P,
                     hipStream_t s);
-// planes: N residue planes followed by the radius-digit planes
-// (VCPHIP_OZ_NDIGIT_A for A, _B for B), each [rows_pad][kpad] int8 with k
-// contiguous
-int vcphip_oz_split_rows(const double* A, long lda, int m, int k, int mpad, int kpad,
-                         const VcphipOzParams& P, VcphipOzSide side, int8_t* planes, hipStream_t s);
-int vcphip_oz_split_cols(const double* B, long ldb, int k, int n, int npad, int kpad,
-                         const VcphipOzParams& P, VcphipOzSide side, int8_t* planes, hipStream_t s);
 // nmod modular products (u8 residues U) plus nrad radius products (int32 Z)
 int vcphip_oz_gemm(int mpad, int npad, int kpad, int nmod, int nrad, const int8_t* Aplanes,
                    const int8_t* Bplanes, const VcphipOzParams& P, uint8_t* U, int32_t* Z, int variant,
@@ -193,13 +191,14 @@ int vcphip_oz_recon(int m, int n, int k, int mpad, int npad, const VcphipOzParam
                     hipStream_t s);
 
 // ---- double-double product, Ozaki scheme II (kern_dd.hip) -------------------
-// rows (rs, cs) of a dd operand: e[r] with max |hi|+|lo| < 2^e; flags bit0: zero
-int vcphip_dd_stats(const double* X, long rs, long cs, int rows, int len, int* e, int* flags, int* part,
-                    hipStream_t s);
-int vcphip_dd_split_rows(const double* A, long lda, int m, int k, int mpad, int kpad, const VcphipOzParams& P,
-                         const int* e, const int* flags, int8_t* planes, hipStream_t s);
-int vcphip_dd_split_cols(const double* B, long ldb, int k, int n, int npad, int kpad, const VcphipOzParams& P,
-                         const int* e, const int* flags, int8_t* planes, hipStream_t s);
+// rows of A (m x k; its columns if a_lines / a_cols: A^T with A k x m) and
+// columns of B (k x n): e with max |hi|+|lo| < 2^e; flags 1: zero, 2: not
+// finite; then the residue planes, each one launch.  A == nullptr: B alone
+int vcphip_dd_stats(const double* A, long lda, int m, int a_lines, int* ea, int* fa, const double* B, long ldb, int n,
+                    int* eb, int* fb, int k, hipStream_t s);
+int vcphip_dd_split(const double* A, long lda, int m, int mpad, int a_cols, const int* ea, const int* fa, int8_t* pa,
+                    const double* B, long ldb, int n, int npad, const int* eb, const int* fb, int8_t* pb, int k,
+                    int kpad, const VcphipOzParams& P, hipStream_t s);
 int vcphip_dd_recon(int m, int n, int mpad, int npad, const VcphipOzParams& P, const int* ea, const int* fa,
                     const int* eb, const int* fb, const uint8_t* U, double* C, long ldc, hipStream_t s);
 
