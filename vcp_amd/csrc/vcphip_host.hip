@@ -91,6 +91,15 @@ struct vcphip_ctx {
   // the host-pointer entry points, and the events of their last DMA
   void* pin[2] = {nullptr, nullptr};
   hipEvent_t pin_ev[2] = {nullptr, nullptr};
+  // the pinned buffer of the small copies: blocks are handed out in turn;
+  // while busy, copies from [0, used) may be in flight on `stream` and end by ev
+  struct Stage {
+    char* p = nullptr;
+    size_t cap = 0, used = 0;
+    hipEvent_t ev = nullptr;
+    hipStream_t stream = nullptr;
+    bool busy = false;
+  } stage;
   // batched interval products: descriptors of the last problem set and its graph
   struct Igb {
     std::vector<VcphipIgemmProblem> probs;
@@ -580,6 +589,9 @@ extern "C" int vcphip_ctx_destroy(vcphip_ctx* c) {
     if (c->pin_ev[h]) hipEventDestroy(c->pin_ev[h]);
     if (c->pin[h]) hipHostFree(c->pin[h]);
   }
+  if (c->stage.busy) hipEventSynchronize(c->stage.ev);
+  if (c->stage.ev) hipEventDestroy(c->stage.ev);
+  if (c->stage.p) hipHostFree(c->stage.p);
   if (c->igb.exec) hipGraphExecDestroy(c->igb.exec);
   if (c->igb.graph) hipGraphDestroy(c->igb.graph);
   hipStreamDestroy(c->own);
@@ -2229,7 +2241,11 @@ namespace {
 // the previous block runs from the other.  Copies from pageable memory run
 // at a fifth of the PCIe rate otherwise.
 constexpr size_t PIN_BYTES = (size_t)128 << 20;
-constexpr size_t PIN_MIN = (size_t)8 << 20;   // below this, one direct copy
+constexpr size_t PIN_MIN = (size_t)8 << 20;   // below this, through the small buffer
+// The small buffer: a strided copy straight from or to pageable memory runs as
+// one transfer per column, about 8 us each (a 96 x 96 product spent 2.7 of its
+// 2.77 ms in them); packed by the host into pinned memory it is one transfer.
+constexpr size_t STAGE_MAX = 3 * PIN_MIN;
 
 bool pin_ready(vcphip_ctx* c) {
   for (int h = 0; h < 2; ++h) {
@@ -2245,6 +2261,64 @@ bool pin_ready(vcphip_ctx* c) {
     }
   }
   return true;
+}
+
+// `bytes` (at most PIN_MIN) of the small pinned buffer, or false
+bool stage_get(vcphip_ctx* c, size_t bytes, char** out) {
+  auto& g = c->stage;
+  const size_t want = (bytes + 255) & ~(size_t)255;
+  if (!g.ev && hipEventCreateWithFlags(&g.ev, hipEventDisableTiming) != hipSuccess) {
+    hipGetLastError();
+    g.ev = nullptr;
+    return false;
+  }
+  size_t need = g.used + want;   // what this call has in flight, and the new block
+  if (g.busy && (g.stream != c->stream || need > g.cap)) {
+    if (hipEventSynchronize(g.ev) != hipSuccess) return false;
+    g.busy = false;
+  }
+  if (!g.busy) g.used = 0;
+  if (g.used + want > g.cap || (!g.busy && need > g.cap && need <= STAGE_MAX)) {
+    if (!g.cap) need = 3 * want;   // the operands and the result of a square product
+    if (g.p) hipHostFree(g.p);
+    g.p = nullptr;
+    g.cap = 0;
+    need = (std::min(std::max(need, want), STAGE_MAX) + 0xFFFFF) & ~(size_t)0xFFFFF;
+    if (hipHostMalloc((void**)&g.p, need, hipHostMallocDefault) != hipSuccess) {
+      hipGetLastError();
+      g.p = nullptr;
+      return false;
+    }
+    g.cap = need;
+  }
+  *out = g.p + g.used;
+  return true;
+}
+
+// the block at `blk` to the device; it stays in use until the copy has ended
+int stage_send(vcphip_ctx* c, void* dev, const char* blk, size_t bytes) {
+  auto& g = c->stage;
+  g.used = (size_t)(blk - g.p) + ((bytes + 255) & ~(size_t)255);
+  g.stream = c->stream;
+  if (hipMemcpyAsync(dev, blk, bytes, hipMemcpyHostToDevice, c->stream) != hipSuccess ||
+      hipEventRecord(g.ev, c->stream) != hipSuccess) {
+    hipStreamSynchronize(c->stream);
+    return VCPHIP_ERR_DEVICE;
+  }
+  g.busy = true;
+  return VCPHIP_OK;
+}
+
+// device memory to the block at `blk`, waited for (and with it every copy of
+// the small buffer, which are all on this stream)
+int stage_receive(vcphip_ctx* c, char* blk, const void* dev, size_t bytes) {
+  if (hipMemcpyAsync(blk, dev, bytes, hipMemcpyDeviceToHost, c->stream) != hipSuccess) {
+    hipStreamSynchronize(c->stream);
+    return VCPHIP_ERR_DEVICE;
+  }
+  if (hipStreamSynchronize(c->stream) != hipSuccess) return VCPHIP_ERR_DEVICE;
+  c->stage.busy = false;
+  return VCPHIP_OK;
 }
 
 // columns [0, ncols) of `rowb` bytes each, from stride `sld` to stride `dld`
@@ -2283,7 +2357,8 @@ void copy_cols(char* dst, size_t dld, const char* src, size_t sld, size_t rowb, 
 // points): piece q is ncols columns of rowb bytes at source stride sld, to be
 // stored dense at byte offset doff of `dev`.  Offsets increase with q and do
 // not overlap.  Large inputs are packed into the pinned buffers, a device
-// range at a time, one DMA per range; below PIN_MIN, one copy per piece.
+// range at a time, one DMA per range; below PIN_MIN, through the small buffer
+// in one.
 struct HostPiece {
   const char* src;
   size_t sld, rowb;
@@ -2331,6 +2406,16 @@ int pieces_to_dev(vcphip_ctx* c, char* dev, const std::vector<HostPiece>& pieces
   for (const auto& q : pieces) total += q.rowb * (size_t)q.ncols;
   bool pinned = total >= PIN_MIN && pin_ready(c);
   for (const auto& q : pieces) pinned = pinned && q.rowb * (size_t)q.ncols <= PIN_BYTES;
+  char* stg;
+  if (!pieces.empty() && total < PIN_MIN) {
+    const size_t start = pieces.front().doff;
+    const HostPiece& last = pieces.back();
+    const size_t bytes = last.doff + last.rowb * (size_t)last.ncols - start;
+    if (bytes > 0 && bytes <= PIN_MIN && stage_get(c, bytes, &stg)) {
+      copy_pieces(pieces, 0, pieces.size(), stg, start, true);
+      return stage_send(c, dev + start, stg, bytes);
+    }
+  }
   if (!pinned) {
     for (const auto& q : pieces)
       if (q.ncols > 0 && q.rowb > 0 &&
@@ -2368,6 +2453,17 @@ int pieces_to_host(vcphip_ctx* c, const char* dev, const std::vector<HostPiece>&
   for (const auto& q : pieces) total += q.rowb * (size_t)q.ncols;
   bool pinned = total >= PIN_MIN && pin_ready(c);
   for (const auto& q : pieces) pinned = pinned && q.rowb * (size_t)q.ncols <= PIN_BYTES;
+  char* stg;
+  if (!pieces.empty() && total < PIN_MIN) {
+    const size_t start = pieces.front().doff;
+    const HostPiece& last = pieces.back();
+    const size_t bytes = last.doff + last.rowb * (size_t)last.ncols - start;
+    if (bytes > 0 && bytes <= PIN_MIN && stage_get(c, bytes, &stg)) {
+      const int rc = stage_receive(c, stg, dev + start, bytes);
+      if (rc == VCPHIP_OK) copy_pieces(pieces, 0, pieces.size(), stg, start, false);
+      return rc;
+    }
+  }
   if (!pinned) {
     for (const auto& q : pieces)
       if (q.ncols > 0 && q.rowb > 0 &&
@@ -2418,6 +2514,11 @@ int to_dev(vcphip_ctx* c, int slot, const double* h, int ld, int rows, int cols,
   *d = (double*)p;
   if (rows <= 0 || cols <= 0) return VCPHIP_OK;
   const size_t rowb = esize * (size_t)rows;
+  char* blk;
+  if (bytes < PIN_MIN && stage_get(c, bytes, &blk)) {
+    copy_cols(blk, rowb, (const char*)h, esize * (size_t)ld, rowb, cols);
+    return stage_send(c, p, blk, bytes);
+  }
   if (bytes < PIN_MIN || rowb > PIN_BYTES || !pin_ready(c)) {
     if (hipMemcpy2DAsync(p, rowb, h, esize * ld, rowb, cols, hipMemcpyHostToDevice, c->stream) != hipSuccess)
       return VCPHIP_ERR_DEVICE;
@@ -2438,6 +2539,12 @@ int to_dev(vcphip_ctx* c, int slot, const double* h, int ld, int rows, int cols,
 int to_host(vcphip_ctx* c, const double* d, double* h, int ld, int rows, int cols, size_t esize) {
   if (rows > 0 && cols > 0) {
     const size_t rowb = esize * (size_t)rows, bytes = rowb * (size_t)cols;
+    char* blk;
+    if (bytes < PIN_MIN && stage_get(c, bytes, &blk)) {
+      const int rc = stage_receive(c, blk, d, bytes);
+      if (rc == VCPHIP_OK) copy_cols((char*)h, esize * (size_t)ld, blk, rowb, rowb, cols);
+      return rc;
+    }
     if (bytes < PIN_MIN || rowb > PIN_BYTES || !pin_ready(c)) {
       if (hipMemcpy2DAsync(h, esize * ld, d, rowb, rowb, cols, hipMemcpyDeviceToHost, c->stream) != hipSuccess)
         return VCPHIP_ERR_DEVICE;
@@ -2865,7 +2972,7 @@ extern "C" int vcphip_residual_batched(vcphip_ctx* c, int count, const int* n, c
   if (count < 0 || (count > 0 && (!n || !R || !ldr || !IA || !lda || !C || !ldc || !normub))) return VCPHIP_ERR_ARGUMENT;
   if (count == 0) return VCPHIP_OK;
   hipSetDevice(c->device);
-  // one staging buffer: R_i (8 n^2), A_i (16 n^2), C_i (16 n^2) packed, then normub
+  // one staging buffer: R_i (8 n^2), A_i (16 n^2) packed, then C_i (16 n^2), then normub
   std::vector<size_t> offR(count), offA(count), offC(count);
   size_t tot = 0;
   for (int i = 0; i < count; ++i) {
@@ -2874,7 +2981,10 @@ extern "C" int vcphip_residual_batched(vcphip_ctx* c, int count, const int* n, c
     const size_t nn = (size_t)n[i] * n[i];
     offR[i] = tot; tot += ((8 * nn + 255) & ~(size_t)255);
     offA[i] = tot; tot += ((16 * nn + 255) & ~(size_t)255);
-    offC[i] = tot; tot += ((16 * nn + 255) & ~(size_t)255);
+  }
+  for (int i = 0; i < count; ++i) {
+    offC[i] = tot;
+    tot += ((16 * (size_t)n[i] * n[i] + 255) & ~(size_t)255);
   }
   const size_t offN = tot;
   tot += sizeof(double) * count + 256;
@@ -2885,6 +2995,7 @@ extern "C" int vcphip_residual_batched(vcphip_ctx* c, int count, const int* n, c
   std::vector<const double*> dR(count), dA(count);
   std::vector<double*> dC(count);
   std::vector<int> ld(count);
+  std::vector<HostPiece> in, out;
   for (int i = 0; i < count; ++i) {
     const int ni = n[i];
     dR[i] = (const double*)(b8 + offR[i]);
@@ -2892,20 +3003,19 @@ extern "C" int vcphip_residual_batched(vcphip_ctx* c, int count, const int* n, c
     dC[i] = (double*)(b8 + offC[i]);
     ld[i] = ni > 1 ? ni : 1;
     if (ni > 0) {
-      if (hipMemcpy2DAsync(b8 + offR[i], 8 * ni, R[i], 8 * (size_t)ldr[i], 8 * ni, ni, hipMemcpyHostToDevice, c->stream) != hipSuccess ||
-          hipMemcpy2DAsync(b8 + offA[i], 16 * ni, IA[i], 16 * (size_t)lda[i], 16 * ni, ni, hipMemcpyHostToDevice, c->stream) != hipSuccess)
-        return VCPHIP_ERR_DEVICE;
+      const size_t rb = 8 * (size_t)ni;
+      in.push_back(HostPiece{(const char*)R[i], 8 * (size_t)ldr[i], rb, ni, offR[i]});
+      in.push_back(HostPiece{(const char*)IA[i], 16 * (size_t)lda[i], 2 * rb, ni, offA[i]});
+      out.push_back(HostPiece{(const char*)C[i], 16 * (size_t)ldc[i], 2 * rb, ni, offC[i]});
     }
   }
+  VCPHIP_TRY(pieces_to_dev(c, b8, in));
   rc = vcphip_residual_batched_dev(c, count, n, dR.data(), ld.data(), dA.data(), ld.data(), dC.data(), ld.data(),
                                    (double*)(b8 + offN));
   if (rc) return rc;
-  for (int i = 0; i < count; ++i)
-    if (n[i] > 0 && hipMemcpy2DAsync(C[i], 16 * (size_t)ldc[i], dC[i], 16 * n[i], 16 * n[i], n[i], hipMemcpyDeviceToHost, c->stream) != hipSuccess)
-      return VCPHIP_ERR_DEVICE;
   if (hipMemcpyAsync(normub, b8 + offN, sizeof(double) * count, hipMemcpyDeviceToHost, c->stream) != hipSuccess)
     return VCPHIP_ERR_DEVICE;
-  return hipStreamSynchronize(c->stream) == hipSuccess ? VCPHIP_OK : VCPHIP_ERR_DEVICE;
+  return pieces_to_host(c, b8, out);
 }
 
 // ===========================================================================
