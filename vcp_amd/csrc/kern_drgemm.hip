@@ -536,7 +536,7 @@ struct ThinProduct : VcphipThinDr<AI, BI> {
 };
 
 template <bool AI, bool BI, int CW, int CPT>
-__global__ __launch_bounds__((VcphipThin<ThinProduct<AI, BI>, CW, CPT>::NT)) __attribute__((amdgpu_waves_per_eu(1, 2))) void k_drgemm_thin(int m, int n, int k, const double* __restrict__ A, long lda,
+__global__ __launch_bounds__((VcphipThin<ThinProduct<AI, BI>, CW, CPT>::NT)) VCPHIP_THIN_WAVES void k_drgemm_thin(int m, int n, int k, const double* __restrict__ A, long lda,
                                                      const double* __restrict__ B, long ldb, double* __restrict__ C,
                                                      long ldc, double* __restrict__ C2, int accumulate) {
   vcphip_mode_round_up();
@@ -581,7 +581,7 @@ struct ResidRowSum {
   VCPHIP_DEVINL void done(const Acc& c, int row, int) const { out[row] = c.s; }
 };
 
-__global__ __launch_bounds__((VcphipThin<ResidRowSum, 1>::NT)) __attribute__((amdgpu_waves_per_eu(1, 2)))
+__global__ __launch_bounds__((VcphipThin<ResidRowSum, 1>::NT)) VCPHIP_THIN_WAVES
 void k_resid_rowsum(const VcphipResidTile* __restrict__ blocks, const VcphipResidProblem* __restrict__ probs,
                     double* __restrict__ rowsum) {
   vcphip_mode_round_up();

@@ -321,7 +321,7 @@ VCPHIP_DEVINL double lss_ynorm(const VcphipLssProblem& P, double* red, double* f
 
 // ---- one system ---------------------------------------------------------------
 template <class Op, int CW, int CPT, bool UP>
-__global__ __launch_bounds__((VcphipThin<Op, CW, CPT>::NT)) __attribute__((amdgpu_waves_per_eu(1, 2)))
+__global__ __launch_bounds__((VcphipThin<Op, CW, CPT>::NT)) VCPHIP_THIN_WAVES
 void k_lss_step(VcphipLssProblem P) {
   if (UP) vcphip_mode_round_up();
   using T = VcphipThin<Op, CW, CPT>;
@@ -331,7 +331,7 @@ void k_lss_step(VcphipLssProblem P) {
   T::run(op, lds, P.n, P.nrhs, P.n, rb * T::R, blockIdx.y * T::NC, (int)((blockIdx.x >> 8) % T::NW));
 }
 
-__global__ __launch_bounds__((VcphipThin<LssRowSum, 1>::NT)) __attribute__((amdgpu_waves_per_eu(1, 2)))
+__global__ __launch_bounds__((VcphipThin<LssRowSum, 1>::NT)) VCPHIP_THIN_WAVES
 void k_lss_rowsum(VcphipLssProblem P, double* __restrict__ rows) {
   vcphip_mode_round_up();
   using T = VcphipThin<LssRowSum, 1>;
@@ -372,7 +372,7 @@ __global__ __launch_bounds__(NT) void k_lss_g(VcphipLssProblem P, const double* 
 }
 
 template <bool DIAG>
-__global__ __launch_bounds__((VcphipThin<LssFinal<DIAG>, 1>::NT)) __attribute__((amdgpu_waves_per_eu(1, 2)))
+__global__ __launch_bounds__((VcphipThin<LssFinal<DIAG>, 1>::NT)) VCPHIP_THIN_WAVES
 void k_lss_final(VcphipLssProblem P) {
   vcphip_mode_round_up();
   using T = VcphipThin<LssFinal<DIAG>, 1>;
@@ -395,7 +395,7 @@ VCPHIP_DEVINL int find_problem(const long* __restrict__ wb, int count, long blk)
 }
 
 template <class Op, bool UP>
-__global__ __launch_bounds__((VcphipThin<Op, 1>::NT)) __attribute__((amdgpu_waves_per_eu(1, 2)))
+__global__ __launch_bounds__((VcphipThin<Op, 1>::NT)) VCPHIP_THIN_WAVES
 void k_lssb_step(int count, const long* __restrict__ wb, const VcphipLssProblem* __restrict__ probs) {
   if (UP) vcphip_mode_round_up();
   using T = VcphipThin<Op, 1>;
@@ -427,7 +427,7 @@ __global__ __launch_bounds__(NT) void k_lssb_g(int count, const VcphipLssProblem
   P.norms[3] = G.y;
 }
 
-__global__ __launch_bounds__((VcphipThin<LssFinal<false>, 1>::NT)) __attribute__((amdgpu_waves_per_eu(1, 2)))
+__global__ __launch_bounds__((VcphipThin<LssFinal<false>, 1>::NT)) VCPHIP_THIN_WAVES
 void k_lssb_final(int count, const long* __restrict__ wb, const VcphipLssProblem* __restrict__ probs) {
   vcphip_mode_round_up();
   using T = VcphipThin<LssFinal<false>, 1>;

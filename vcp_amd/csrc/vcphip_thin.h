@@ -7,12 +7,14 @@
 // Such a product is bound by reading A once (16 or 8 bytes per element
 // against a few FMAs), or by the length of the chains.  So the split is by
 // rows: a workgroup takes 8 rows (128 contiguous bytes of an interval column,
-// one cache line), all four waves load and convert 8 x KB elements of A and
-// the KB x NC block of B into LDS, one stage ahead of the chains and with the
-// next stage's loads in flight, and one wave carries the chains: lane = row
-// (8) x column lane (8), CPT columns per lane.  m = 4000 rows give 500
-// workgroups, two per CU; consecutive row blocks run on one XCD, so that
-// cache lines that straddle two row blocks are fetched once per L2.
+// one cache line).  Loading waves (3 beside one chain wave, 2 beside two, 4
+// beside four) load and convert 8 x KB elements of A and the KB x NC block of
+// B into LDS, one stage ahead of the chains and with the next stage's loads in
+// flight; the chain waves carry the chains: lane = row (8) x column lane (8),
+// CPT columns per lane.  Loading by separate waves keeps conversions and
+// global waits out of the chains' way.  m = 4000 rows give 500 workgroups, two
+// per CU; consecutive row blocks run on one XCD, so that cache lines that
+// straddle two row blocks are fetched once per L2.
 //
 // The operation is a policy Op:
 //   A2, B2      global elements of A / B are pairs (else doubles)
@@ -25,6 +27,15 @@
 #pragma once
 
 #include "vcphip_device.h"
+
+// Register target of the kernels built on this: up to four waves per SIMD.  The
+// upper limit is also the most a SIMD will hold (the compiler reserves the
+// registers of that many), so a limit of two, enough for one row block's loads
+// in flight, kept the other workgroups of a batch, and those of other streams,
+// off the CU: a batch of 64 solves' row sums 100 against 49 us with four, its
+// bounds 88 against 66, R mid(b) 155 against 67, 4000 x 4000 times 4 vectors
+// in three streams 65 against 54.  Eight: as four.
+#define VCPHIP_THIN_WAVES __attribute__((amdgpu_waves_per_eu(1, 4)))
 
 constexpr int VCPHIP_THIN_R = 8;    // rows of a workgroup
 constexpr int VCPHIP_THIN_CL = 8;   // column lanes of the chain wave
