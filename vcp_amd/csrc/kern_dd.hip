@@ -340,38 +340,47 @@ __global__ __launch_bounds__(256) void k_dd_split(const double* __restrict__ A, 
 constexpr int NL = VCPHIP_OZ_NLIMB;
 static_assert(NL == vcphip_ddconv::NL, "limb count of the conversion");
 
-template <int N>
+template <int N, int EL>
 __global__ __launch_bounds__(256) void k_dd_recon(int m, int n, int mpad, int npad, VcphipOzParams P,
                                                   const int* __restrict__ ea, const int* __restrict__ fa,
                                                   const int* __restrict__ eb, const int* __restrict__ fb,
                                                   const uint8_t* __restrict__ U, double* __restrict__ C, long ldc) {
-  // threads follow the blocked 16 x 16 layout of the residue planes
-  // grid: x = 16-row block, y = 16-column block (the plane's block order)
-  // the block's planes from a uniform base plus the thread's offset o
-  // every lane runs through the CRT's matrix instructions; lanes past m or n
-  // (inside the padded planes) read row / column 0's tables and store nothing
-  const unsigned o = threadIdx.x;
-  const long bbase = ((long)blockIdx.y * (mpad >> 4) + blockIdx.x) * 256;
-  const unsigned i0 = blockIdx.x * 16 + 4 * (o >> 6) + (o & 3);
-  const unsigned j0 = blockIdx.y * 16 + ((o >> 2) & 15);
-  const bool live = i0 < (unsigned)m && j0 < (unsigned)n;
-  const unsigned i = live ? i0 : 0u, j = live ? j0 : 0u;
-  const long plane = (long)mpad * npad;
+  // a wave takes one 16 x 16 block of the residue planes, a lane four rows of
+  // one of its columns (see k_oz_recon); every lane runs through the CRT's
+  // matrix instructions, elements past m or n (inside the padded planes) read
+  // row / column 0's tables and are not stored
+  __shared__ VcphipBlockOut s_out[EL];
+  const unsigned lane = threadIdx.x & 63u;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int bi = EL == 4 ? blockIdx.x * 4 + wv : blockIdx.x, bj = blockIdx.y;
+  const int e0 = EL == 4 ? 0 : wv;   // this wave's elements are e0 .. e0 + EL - 1 of each lane's four
+  const long bbase = ((long)bj * (mpad >> 4) + bi) * 256;
+  const unsigned j0 = bj * 16 + (lane & 15);
+  const unsigned j = j0 < (unsigned)n ? j0 : 0u;
   VcphipCrtOps<N> T;
   vcphip_crt_ops_load<N>(P, T);
-  unsigned mag[NL];
-  const bool neg = vcphip_crt_symmetric<N, NL>(U + bbase, plane, o, T, P, mag);
-  const int flag = fa[i] | fb[j];
-  if (flag) {   // a zero row / column gives 0, a non-finite one NaN
-    const double v = (flag & 2) ? __builtin_nan("") : 0.0;
-    if (live) *reinterpret_cast<double2*>(C + 2 * (i + ldc * (long)j)) = make_double2(v, v);
-    return;
+  vcphip_v4i b[EL][VcphipCrtOps<N>::RH];
+  vcphip_crt_operands<N, EL>(U + bbase, (long)mpad * npad, lane, e0, b);
+  const int fj = fb[j], ej = eb[j];
+  double2 out[EL];
+#pragma unroll
+  for (int el = 0; el < EL; ++el) {
+    const unsigned i0 = bi * 16 + 4 * (lane >> 4) + e0 + el;
+    const unsigned i = i0 < (unsigned)m ? i0 : 0u;
+    unsigned mag[NL];
+    const bool neg = vcphip_crt_limbs<N, NL>(b[el], T, P, mag);
+    const int flag = fa[i] | fj;
+    if (flag) {   // a zero row / column gives 0, a non-finite one NaN
+      const double v = (flag & 2) ? __builtin_nan("") : 0.0;
+      out[el] = make_double2(v, v);
+    } else {
+      double hi, lo;
+      vcphip_dd_from_limbs(mag, ea[i] + ej - 2 * P.beta, hi, lo);
+      const double sgn = neg ? -1.0 : 1.0;
+      out[el] = make_double2(sgn * hi, sgn * lo);
+    }
   }
-  const int sc = ea[i] + eb[j] - 2 * P.beta;
-  double hi, lo;
-  vcphip_dd_from_limbs(mag, sc, hi, lo);
-  const double sgn = neg ? -1.0 : 1.0;
-  if (live) *reinterpret_cast<double2*>(C + 2 * (i + ldc * (long)j)) = make_double2(sgn * hi, sgn * lo);
+  vcphip_block_store<EL>(s_out[EL == 4 ? wv : 0], out, lane, e0, C, ldc, bi * 16, bj * 16, m, n);
 }
 
 // ---------------------------------------------------------------------------
@@ -790,10 +799,16 @@ int vcphip_dd_split(const double* A, long lda, int m, int mpad, int a_cols, cons
 int vcphip_dd_recon(int m, int n, int mpad, int npad, const VcphipOzParams& P, const int* ea, const int* fa,
                     const int* eb, const int* fb, const uint8_t* U, double* C, long ldc, hipStream_t s) {
   if (m <= 0 || n <= 0) return 0;
-  dim3 grid((unsigned)(mpad / 16), (unsigned)(npad / 16));
+  const bool split = (long)(mpad / 16) * (npad / 16) <= VCPHIP_CRT_SPLIT_BLOCKS;
+  const dim3 grid((unsigned)(split ? mpad / 16 : mpad / 64), (unsigned)(npad / 16));   // mpad: a multiple of 128
   switch (P.nmod) {
-#define VCPHIP_DD_CASE(NN) \
-  case NN: hipLaunchKernelGGL((k_dd_recon<NN>), grid, dim3(256), 0, s, m, n, mpad, npad, P, ea, fa, eb, fb, U, C, ldc); break;
+#define VCPHIP_DD_CASE(NN)                                                                                           \
+  case NN:                                                                                                           \
+    if (split)                                                                                                       \
+      hipLaunchKernelGGL((k_dd_recon<NN, 1>), grid, dim3(256), 0, s, m, n, mpad, npad, P, ea, fa, eb, fb, U, C, ldc); \
+    else                                                                                                             \
+      hipLaunchKernelGGL((k_dd_recon<NN, 4>), grid, dim3(256), 0, s, m, n, mpad, npad, P, ea, fa, eb, fb, U, C, ldc); \
+    break;
     VCPHIP_DD_CASE(24) VCPHIP_DD_CASE(25) VCPHIP_DD_CASE(26) VCPHIP_DD_CASE(27) VCPHIP_DD_CASE(28)
     VCPHIP_DD_CASE(29) VCPHIP_DD_CASE(30) VCPHIP_DD_CASE(31) VCPHIP_DD_CASE(32)
 #undef VCPHIP_DD_CASE

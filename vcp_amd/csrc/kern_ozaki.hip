@@ -1123,140 +1123,165 @@ constexpr int oz_limbs() {
   return (N + 3) / 4;
 }
 
-// |X| * 2^s rounded toward zero (tz) and away from zero (aw), exactly: both
-// come from one 64-bit window of the limbs and the sticky bit below it
+// |X| * 2^s rounded toward zero (tz) and away from zero (aw), exactly.  The
+// top limb is brought to the front by at most log2(NL) conditional moves of
+// all limbs, the 64 bits below X's top bit form W, and tail stands for any set
+// bit below W.  mant = W >> r is the kept part: r = 11 (53 bits), or more where
+// gradual underflow ends the significand at 2^-1074 (the shifted-out bits are
+// zero where |X| 2^s is representable).  With ex the exponent of mant's last
+// bit, (ex + 1074) 2^52 + mant is the double's bit pattern (a normal mant's
+// leading one counts as one in the exponent field), and away from zero is the
+// next pattern, infinity after the largest double.
 template <int NL>
 VCPHIP_DEVINL void conv_limbs2(const unsigned (&mag)[NL], int s, double& tz, double& aw) {
-  int top = -1;
+  unsigned x[NL];
 #pragma unroll
-  for (int l = NL - 1; l >= 0; --l)
-    if (top < 0 && mag[l] != 0) top = 32 * l + 31 - __builtin_clz(mag[l]);
-  if (top < 0) {
-    tz = aw = 0.0;
-    return;
-  }
-  int q = top - 52;
-  if (q < -1074 - s) q = -1074 - s;
-  unsigned long long mant;
-  bool rest = false;
-  if (q <= 0) {
-    mant = (unsigned long long)mag[0] | ((unsigned long long)mag[1] << 32);
-    q = 0;
-  } else {
-    // bits [q, q+64) and the sticky tail below q
-    const int ls = q >> 5, bs = q & 31;
-    unsigned w0 = 0, w1 = 0, w2 = 0;
-    bool tail = false;
+  for (int l = 0; l < NL; ++l) x[l] = mag[l];
+  int top = 32 * NL - 1;   // X's top bit, once x is normalised
 #pragma unroll
-    for (int l = 0; l < NL; ++l) {
-      if (l == ls) w0 = mag[l];
-      if (l == ls + 1) w1 = mag[l];
-      if (l == ls + 2) w2 = mag[l];
-      if (l < ls && mag[l] != 0) tail = true;
-    }
-    if (bs != 0 && (w0 & ((1u << bs) - 1u)) != 0) tail = true;
-    const unsigned long long lo = (unsigned long long)w0 | ((unsigned long long)w1 << 32);
-    mant = bs ? ((lo >> bs) | ((unsigned long long)w2 << (64 - bs))) : lo;
-    if (q >= 32 * NL) {
-      mant = 0;
-      tail = true;
-    }
-    rest = tail;
+  for (int h = NL > 4 ? 4 : NL > 2 ? 2 : 1; h > 0; h >>= 1) {
+    unsigned any = 0;
+#pragma unroll
+    for (int l = NL - h; l < NL; ++l) any |= x[l];
+    const bool mv = any == 0;
+#pragma unroll
+    for (int l = NL - 1; l >= 0; --l) x[l] = mv ? (l >= h ? x[l - h] : 0u) : x[l];
+    top -= mv ? 32 * h : 0;
   }
-  const int ex = q + s;
-  const unsigned long long mant_aw = mant + (rest ? 1ull : 0ull);
-  // mant < 2^53 except in the subnormal clamp (q <= 0), where both are exact
-  tz = (mant != 0 && ex + (64 - __builtin_clzll(mant)) > 1024) ? 1.7976931348623157e308 : __builtin_ldexp((double)mant, ex);
-  aw = (mant_aw != 0 && ex + (64 - __builtin_clzll(mant_aw)) > 1024) ? __builtin_inf() : __builtin_ldexp((double)mant_aw, ex);
+  const unsigned x0 = x[NL - 1], x1 = NL > 1 ? x[NL - 2] : 0u, x2 = NL > 2 ? x[NL - 3] : 0u;
+  const int z = x0 ? __builtin_clz(x0) : 0;
+  top -= z;
+  unsigned tail = x2 << z;
+#pragma unroll
+  for (int l = 0; l + 3 < NL; ++l) tail |= x[l];
+  const unsigned long long w =
+      ((((unsigned long long)x0 << 32) | x1) << z) | ((unsigned long long)x2 << z >> 32);
+  const int first = top - 63 + s;   // exponent of W's last bit
+  int r = first < -1074 - 11 ? -1074 - first : 11;
+  r = r > 63 ? 63 : r;   // r = 64 and above: W >> 63 = 1 is dropped below
+  unsigned long long mant = w >> r;
+  const bool none = first < -1074 - 63;
+  const bool rest = ((mant << r) != w) || tail != 0 || none;
+  mant = none ? 0ull : mant;
+  const int ex = none ? -1074 : first + r;
+  const unsigned long long bits = ((unsigned long long)(unsigned)(ex + 1074) << 52) + mant;
+  const bool big = ex > 971;   // |X| 2^s >= 2^1024
+  tz = __builtin_bit_cast(double, big ? 0x7FEFFFFFFFFFFFFFull : bits);
+  aw = __builtin_bit_cast(double, big ? 0x7FF0000000000000ull : bits + (rest ? 1ull : 0ull));
+  if (!x0) tz = aw = 0.0;
 }
 
-template <int N>
+template <int N, int EL>
 __global__ __launch_bounds__(256) void k_oz_recon(int m, int n, int k, int mpad, int npad, VcphipOzParams P,
                                                   VcphipOzSide sa, VcphipOzSide sb,
                                                   const uint8_t* __restrict__ U, const int32_t* __restrict__ Z,
                                                   double* __restrict__ C, long ldc) {
   vcphip_mode_round_up();
-  // threads follow the blocked 16 x 16 layout of the planes (coalesced
-  // residue reads): offset o in a block holds row 4 (o / 64) + o % 4 and
-  // column (o / 4) % 16 of that block
-  // grid: x = 16-row block, y = 16-column block (the plane's block order)
-  // the block's planes are addressed from a uniform base (Ub, Zb) plus the
-  // thread's offset o, and the row / column tables by unsigned indices
-  // every lane runs through the CRT's matrix instructions; lanes past m or n
-  // (inside the padded planes) read row / column 0's tables and store nothing
-  const unsigned o = threadIdx.x;
-  const long bbase = ((long)blockIdx.y * (mpad >> 4) + blockIdx.x) * 256;
-  const unsigned i0 = blockIdx.x * 16 + 4 * (o >> 6) + (o & 3);
-  const unsigned j0 = blockIdx.y * 16 + ((o >> 2) & 15);
-  const bool live = i0 < (unsigned)m && j0 < (unsigned)n;
-  const unsigned i = live ? i0 : 0u, j = live ? j0 : 0u;
+  // a wave takes one 16 x 16 block of the planes, a lane four rows of one of
+  // its columns: the block's planes are read a word (residues) or four (digit
+  // products) per lane and plane from a uniform base, and the weights, the
+  // column's tables and the scalar work are shared by four elements (EL = 4; in
+  // small products four waves share a block, EL = 1).  Bound by VALU and scalar
+  // issue, 367 and 198 instructions per 64 elements at 16 moduli (one element
+  // per lane, a byte load per plane and four 64-bit steps per limb took 464 and
+  // 364), and by HBM (40 bytes read per element at full radius, 16 written):
+  // n = 2000 78 -> 68 us, 8192 (15 moduli) 968 -> 812 us; dd 4096 318 -> 271.
+  // Every lane runs through the CRT's matrix instructions; elements past m or
+  // n (inside the padded planes) read row / column 0's tables and are not
+  // stored.
+  __shared__ VcphipBlockOut s_out[EL];
+  const unsigned lane = threadIdx.x & 63u;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int bi = EL == 4 ? blockIdx.x * 4 + wv : blockIdx.x, bj = blockIdx.y;
+  const int e0 = EL == 4 ? 0 : wv;   // this wave's elements are e0 .. e0 + EL - 1 of each lane's four
+  const long bbase = ((long)bj * (mpad >> 4) + bi) * 256;
+  const unsigned j0 = bj * 16 + (lane & 15);
+  const unsigned j = j0 < (unsigned)n ? j0 : 0u;
   const long plane = (long)mpad * npad;
   const int32_t* __restrict__ Zb = Z + bbase;
 
+  constexpr int NL = oz_limbs<N>();
   VcphipCrtOps<N> T;
   vcphip_crt_ops_load<N>(P, T);
-  constexpr int NL = oz_limbs<N>();
-  unsigned mag[NL];
-  const bool neg = vcphip_crt_symmetric<N, NL>(U + bbase, plane, o, T, P, mag);
-  const int fa = sa.flags[i], fb = sb.flags[j];
-  const bool zr = (fa & VCPHIP_OZ_MIDZERO) != 0, zc = (fb & VCPHIP_OZ_MIDZERO) != 0;
-  const int ei = sa.e[i], fj = sb.e[j];
-  const int sc = ei + fj - 2 * P.beta;
-  // RD and RU of the exact midpoint product
-  double tz, aw;
-  conv_limbs2(mag, sc, tz, aw);
-  const double lo_mid = neg ? -aw : tz, hi_mid = neg ? -tz : aw;
-  // radius term (|mA|+rA) rB + rA |mB| (pidblas :277-283) from the digit
-  // products.  With x1 <= (h1 + l1/127) 2^g1/127 <= H1 2^g1/127 (A, l1 >= 0)
-  // and x2 <= (H + L/127) 2^g2/127 <= H 2^g2/127 (B, L <= 0), per term
-  //   full    sum x1 x2 <= 2^(g1+g2)/127^2 (Zhh + Zmix/127 + Zll/127^2),
-  //           Zhh = sum h1 H, Zmix = sum h1 L + l1 H, Zll = sum l1 L <= 0;
-  //   folded  the same without Zll (<= 0, so the bound only rises);
-  //   half    (Zhh + Zlh/127) with Zlh = sum l1 H;
-  //   ceil    Zcc = sum H1 H.
-  // A quotient of a numerator of either sign is bounded above by the
-  // numerator times the RU or, when negative, the RD reciprocal.
-  double t1 = 0.0, t2 = 0.0;
+  vcphip_v4i b[EL][VcphipCrtOps<N>::RH];
+  vcphip_crt_operands<N, EL>(U + bbase, plane, lane, e0, b);
   const bool ceil_only = P.rscheme == VCPHIP_OZ_RADIUS_CEIL, full = P.rscheme == VCPHIP_OZ_RADIUS_FULL;
+  vcphip_v4i zd[VCPHIP_OZ_MAXRAD];   // the digit products of the four elements
+#pragma unroll
+  for (int z = 0; z < VCPHIP_OZ_MAXRAD; ++z) {
+    zd[z] = vcphip_v4i{0, 0, 0, 0};
+    if (z >= P.rnz) continue;
+    const auto rz = vcphip_rsrc(Zb + z * plane, 1024);
+    if (EL == 4) zd[z] = __builtin_bit_cast(vcphip_v4i, __builtin_amdgcn_raw_buffer_load_b128(rz, 16 * lane, 0, 0));
+    else zd[z][0] = (int)__builtin_amdgcn_raw_buffer_load_b32(rz, 16 * lane + 4 * e0, 0, 0);
+  }
+  const int fb = sb.flags[j], fj = sb.e[j], hj = sb.h[j];
+  const double n1j = sb.n1[j];
+  const bool zc = (fb & VCPHIP_OZ_MIDZERO) != 0;
   // the directed reciprocals as register values (a per-lane choice between
   // two parameter fields would otherwise become a per-lane load)
   const double c1 = vcphip_uniform(P.c1), c1dn = vcphip_uniform(P.c1dn);
   const double c127 = vcphip_uniform(P.c127), c127dn = vcphip_uniform(P.c127dn);
-  auto zload = [&](int z) {   // digit product z of this element
-    return (int)__builtin_amdgcn_raw_buffer_load_b32(vcphip_rsrc(Zb + z * plane, 1024), 4 * o, 0, 0);
-  };
-  auto digit_sum = [&](int zh, int zm, int zl) {
-    if (ceil_only) return (double)zload(zh);
-    const int mx = zload(zm);
-    double u = (double)zload(zh) + (double)mx * (mx >= 0 ? c1 : c1dn);
-    if (full) {
-      const int ll = zload(zl);
-      u = u + (double)ll * (ll >= 0 ? c127 : c127dn);
+  double2 out[EL];
+#pragma unroll
+  for (int el = 0; el < EL; ++el) {
+    const unsigned i0 = bi * 16 + 4 * (lane >> 4) + e0 + el;
+    const unsigned i = i0 < (unsigned)m ? i0 : 0u;
+    unsigned mag[NL];
+    const bool neg = vcphip_crt_limbs<N, NL>(b[el], T, P, mag);
+    const int fa = sa.flags[i];
+    const bool zr = (fa & VCPHIP_OZ_MIDZERO) != 0;
+    const int ei = sa.e[i];
+    const int sc = ei + fj - 2 * P.beta;
+    // RD and RU of the exact midpoint product
+    double tz, aw;
+    conv_limbs2(mag, sc, tz, aw);
+    const double lo_mid = neg ? -aw : tz, hi_mid = neg ? -tz : aw;
+    // radius term (|mA|+rA) rB + rA |mB| (pidblas :277-283) from the digit
+    // products.  With x1 <= (h1 + l1/127) 2^g1/127 <= H1 2^g1/127 (A, l1 >= 0)
+    // and x2 <= (H + L/127) 2^g2/127 <= H 2^g2/127 (B, L <= 0), per term
+    //   full    sum x1 x2 <= 2^(g1+g2)/127^2 (Zhh + Zmix/127 + Zll/127^2),
+    //           Zhh = sum h1 H, Zmix = sum h1 L + l1 H, Zll = sum l1 L <= 0;
+    //   folded  the same without Zll (<= 0, so the bound only rises);
+    //   half    (Zhh + Zlh/127) with Zlh = sum l1 H;
+    //   ceil    Zcc = sum H1 H.
+    // A quotient of a numerator of either sign is bounded above by the
+    // numerator times the RU or, when negative, the RD reciprocal.
+    double t1 = 0.0, t2 = 0.0;
+    auto digit_sum = [&](int zh, int zm, int zl) {
+      if (ceil_only) return (double)zd[zh][el];
+      const int mx = zd[zm][el];
+      double u = (double)zd[zh][el] + (double)mx * (mx >= 0 ? c1 : c1dn);
+      if (full) {
+        const int ll = zd[zl][el];
+        u = u + (double)ll * (ll >= 0 ? c127 : c127dn);
+      }
+      return u;
+    };
+    if (!((fa & VCPHIP_OZ_SUMZERO) || (fb & VCPHIP_OZ_RADZERO)))
+      t1 = vcphip_mulpow2(ceil_only ? digit_sum(0, 0, 0) : digit_sum(0, 1, 4), sa.g[i] + hj) * P.c127;
+    if (!((fa & VCPHIP_OZ_RADZERO) || zc))
+      t2 = vcphip_mulpow2(ceil_only ? digit_sum(1, 1, 1) : digit_sum(2, 3, 5), sa.h[i] + fj) * P.c127;
+    const double rt = t1 + t2;
+    // scaling error of the midpoint product
+    double E = 0.0;
+    if (!zr && !zc) {
+      const double ka = vcphip_mulpow2((double)k, ei - P.beta - 1);
+      const double e1 = vcphip_mulpow2(sa.n1[i] + ka, fj - P.beta - 1);
+      const double e2 = vcphip_mulpow2(n1j, ei - P.beta - 1);
+      E = e1 + e2;
     }
-    return u;
-  };
-  if (!((fa & VCPHIP_OZ_SUMZERO) || (fb & VCPHIP_OZ_RADZERO)))
-    t1 = vcphip_mulpow2(ceil_only ? digit_sum(0, 0, 0) : digit_sum(0, 1, 4), sa.g[i] + sb.h[j]) * P.c127;
-  if (!((fa & VCPHIP_OZ_RADZERO) || zc))
-    t2 = vcphip_mulpow2(ceil_only ? digit_sum(1, 1, 1) : digit_sum(2, 3, 5), sa.h[i] + fj) * P.c127;
-  const double rt = t1 + t2;
-  // scaling error of the midpoint product
-  double E = 0.0;
-  if (!zr && !zc) {
-    const double ka = vcphip_mulpow2((double)k, ei - P.beta - 1);
-    const double e1 = vcphip_mulpow2(sa.n1[i] + ka, fj - P.beta - 1);
-    const double e2 = vcphip_mulpow2(sb.n1[j], ei - P.beta - 1);
-    E = e1 + e2;
+    const double rad = rt + E;
+    double hi = hi_mid + rad;
+    double lo = -(rad - lo_mid);
+    if ((fa | fb) & VCPHIP_OZ_NONFINITE) {   // a non-finite operand end in the row or column
+      const bool nan = ((fa | fb) & VCPHIP_OZ_HASNAN) != 0;
+      lo = nan ? __builtin_nan("") : -__builtin_inf();
+      hi = nan ? __builtin_nan("") : __builtin_inf();
+    }
+    out[el] = make_double2(lo, hi);
   }
-  const double rad = rt + E;
-  double hi = hi_mid + rad;
-  double lo = -(rad - lo_mid);
-  if ((fa | fb) & VCPHIP_OZ_NONFINITE) {   // a non-finite operand end in the row or column
-    const bool nan = ((fa | fb) & VCPHIP_OZ_HASNAN) != 0;
-    lo = nan ? __builtin_nan("") : -__builtin_inf();
-    hi = nan ? __builtin_nan("") : __builtin_inf();
-  }
-  if (live) *reinterpret_cast<double2*>(C + 2 * (i + ldc * (long)j)) = make_double2(lo, hi);
+  vcphip_block_store<EL>(s_out[EL == 4 ? wv : 0], out, lane, e0, C, ldc, bi * 16, bj * 16, m, n);
 }
 
 }  // namespace
@@ -1401,10 +1426,16 @@ int vcphip_oz_recon(int m, int n, int k, int mpad, int npad, const VcphipOzParam
                     hipStream_t s) {
   if (m <= 0 || n <= 0) return 0;
   if (P.rscheme < VCPHIP_OZ_RADIUS_FULL || P.rscheme > VCPHIP_OZ_RADIUS_CEIL) return -7;
-  dim3 grid((unsigned)(mpad / 16), (unsigned)(npad / 16));
+  const bool split = (long)(mpad / 16) * (npad / 16) <= VCPHIP_CRT_SPLIT_BLOCKS;
+  const dim3 grid((unsigned)(split ? mpad / 16 : mpad / 64), (unsigned)(npad / 16));   // mpad: a multiple of 128
   switch (P.nmod) {
-#define VCPHIP_RECON_CASE(NN) \
-  case NN: hipLaunchKernelGGL((k_oz_recon<NN>), grid, dim3(256), 0, s, m, n, k, mpad, npad, P, sa, sb, U, Z, C, ldc); break;
+#define VCPHIP_RECON_CASE(NN)                                                                                           \
+  case NN:                                                                                                              \
+    if (split)                                                                                                          \
+      hipLaunchKernelGGL((k_oz_recon<NN, 1>), grid, dim3(256), 0, s, m, n, k, mpad, npad, P, sa, sb, U, Z, C, ldc);     \
+    else                                                                                                                \
+      hipLaunchKernelGGL((k_oz_recon<NN, 4>), grid, dim3(256), 0, s, m, n, k, mpad, npad, P, sa, sb, U, Z, C, ldc);     \
+    break;
     VCPHIP_RECON_CASE(8) VCPHIP_RECON_CASE(9) VCPHIP_RECON_CASE(10) VCPHIP_RECON_CASE(11)
     VCPHIP_RECON_CASE(12) VCPHIP_RECON_CASE(13) VCPHIP_RECON_CASE(14) VCPHIP_RECON_CASE(15)
     VCPHIP_RECON_CASE(16) VCPHIP_RECON_CASE(17) VCPHIP_RECON_CASE(18) VCPHIP_RECON_CASE(19)

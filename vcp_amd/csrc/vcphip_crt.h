@@ -62,41 +62,80 @@ VCPHIP_DEVINL void vcphip_crt_ops_load(const VcphipOzParams& P, VcphipCrtOps<N>&
       T.a[ch][rh] = mine ? *reinterpret_cast<const vcphip_v4i*>(&P.crt_a[16 * ch + cl][4 * rh]) : vcphip_v4i{0, 0, 0, 0};
 }
 
-// From the residues u[t] (bytes) of this lane's X: returns the sign of X and
-// its magnitude in NL little-endian 32-bit limbs.
+// The B operands (centred residues) of elements e0 .. e0 + EL - 1 of the four
+// elements 4 lane .. 4 lane + 3 that this lane reads of a 16 x 16 plane block
+// (rows 4 (lane / 16) .. + 3 of column lane % 16): EL = 4 (e0 = 0), or EL = 1
+// with a wave-uniform e0.  One word per plane, from a scalar resource at the
+// lane's offset (U: the block's base in the first plane, wave-uniform), and
+// 4 x 4 byte transposes of four planes' words.
+template <int N, int EL>
+VCPHIP_DEVINL void vcphip_crt_operands(const uint8_t* __restrict__ U, long plane, unsigned lane, int e0,
+                                       vcphip_v4i (&b)[EL][VcphipCrtOps<N>::RH]) {
+  constexpr int RH = VcphipCrtOps<N>::RH;
+  static_assert(EL == 1 || EL == 4, "elements per lane");
+  unsigned w[16 * RH];
+#pragma unroll
+  for (int t = 0; t < 16 * RH; ++t)   // bytes past N meet zero weights
+    w[t] = t < N ? __builtin_amdgcn_raw_buffer_load_b32(vcphip_rsrc(U + (long)t * plane, 256), 4 * lane, 0, 0) : 0u;
+  constexpr unsigned LO = 0x05010400u, HI = 0x07030602u, EVEN = 0x05040100u, ODD = 0x07060302u;
+  const unsigned s1 = e0 & 2 ? HI : LO, s2 = e0 & 1 ? ODD : EVEN;   // EL = 1
+#pragma unroll
+  for (int t = 0; t < 16 * RH; t += 4) {
+    if (t >= N) {
+#pragma unroll
+      for (int e = 0; e < EL; ++e) b[e][t / 16][t % 16 / 4] = 0;
+      continue;
+    }
+    if (EL == 1) {
+      const unsigned x01 = __builtin_amdgcn_perm(w[t + 1], w[t], s1), x23 = __builtin_amdgcn_perm(w[t + 3], w[t + 2], s1);
+      b[0][t / 16][t % 16 / 4] = (int)(__builtin_amdgcn_perm(x23, x01, s2) ^ 0x80808080u);   // u - 128 as int8
+      continue;
+    }
+#pragma unroll
+    for (int y = 0; y < 4; ++y) w[t + y] ^= 0x80808080u;
+    const unsigned l01 = __builtin_amdgcn_perm(w[t + 1], w[t], LO), h01 = __builtin_amdgcn_perm(w[t + 1], w[t], HI);
+    const unsigned l23 = __builtin_amdgcn_perm(w[t + 3], w[t + 2], LO), h23 = __builtin_amdgcn_perm(w[t + 3], w[t + 2], HI);
+#pragma unroll
+    for (int e = 0; e < EL; ++e)
+      b[e][t / 16][t % 16 / 4] = (int)__builtin_amdgcn_perm(e < 2 ? l23 : h23, e < 2 ? l01 : h01, e & 1 ? ODD : EVEN);
+  }
+}
+
+// From the residues of this lane's X (its operands b): returns the sign of X
+// and its magnitude in NL little-endian 32-bit limbs.
 template <int N, int NL>
-VCPHIP_DEVINL bool vcphip_crt_from_residues(const unsigned (&u)[N], const VcphipCrtOps<N>& T, const VcphipOzParams& P,
-                                            unsigned (&mag)[NL]) {
+VCPHIP_DEVINL bool vcphip_crt_limbs(const vcphip_v4i (&b)[VcphipCrtOps<N>::RH], const VcphipCrtOps<N>& T,
+                                    const VcphipOzParams& P, unsigned (&mag)[NL]) {
   static_assert(N <= 4 * NL, "byte columns beyond the limbs");
   constexpr int CH = VcphipCrtOps<N>::CH, RH = VcphipCrtOps<N>::RH;
-  vcphip_v4i b[RH];
-#pragma unroll
-  for (int rh = 0; rh < RH; ++rh)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      unsigned x = 0;
-#pragma unroll
-      for (int y = 0; y < 4; ++y)
-        if (16 * rh + 4 * e + y < N) x |= u[16 * rh + 4 * e + y] << (8 * y);
-      b[rh][e] = (int)(x ^ 0x80808080u);   // u - 128 as int8 (bytes past N meet zero weights)
-    }
   // column group 0 first: its columns 0..6 are the quotient bytes and the
   // residue sum, so q is known before the weight columns (7 .. N + 6) of the
   // later groups are formed, and one group's accumulators are live at a time
   vcphip_v16i acc = vcphip_v16i{};
 #pragma unroll
   for (int rh = 0; rh < RH; ++rh) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(T.a[0][rh], b[rh], acc, 0, 0, 0);
-  const int s128 = 128 * (acc[6] + 128 * N);   // 128 sum_t u_t
-  unsigned long long Q = 1ull << 47;
-#pragma unroll
-  for (int c = 0; c < 6; ++c) Q += (unsigned long long)(unsigned)(acc[c] + s128 + P.crt_k[c]) << (8 * c);
-  const long long q = (long long)(Q >> 48);
+  const unsigned s128 = 128u * (unsigned)(acc[6] + 128 * N);   // 128 sum_t u_t
+  // two byte columns at a time: col_c + 2^8 col_(c+1) < 2^30, with the centring
+  // terms of both added at once
+  const unsigned s2 = s128 * 257u;
+  auto pair = [&](int g, int v) {
+    const unsigned kk = (unsigned)P.crt_k[16 * g + v] + ((unsigned)P.crt_k[16 * g + v + 1] << 8);
+    return (((unsigned)acc[v + 1] << 8) + (unsigned)acc[v]) + (s2 + kk);
+  };
+  // q = floor((sum_b fc_b 2^(8b) + 2^47) / 2^48)
+  const unsigned q = (pair(0, 4) + 0x8000u + ((pair(0, 2) + (pair(0, 0) >> 16)) >> 16)) >> 16;
+  // limb l = low pair + 2^16 high pair - q M_l
   long long limb[NL];
 #pragma unroll
-  for (int l = 0; l < NL; ++l) limb[l] = -q * (long long)P.Mlimb[l];
+  for (int l = 0; l < NL; ++l) limb[l] = -(long long)((unsigned long long)q * P.Mlimb[l]);
+  unsigned half[2 * NL];
+#pragma unroll
+  for (int h = 0; h < 2 * NL; ++h) half[h] = 0;
 #pragma unroll
   for (int ch = 0; ch < CH; ++ch) {
+    unsigned last = 0;   // the column that a pair split over two groups begins with
     if (ch > 0) {
+      last = (unsigned)acc[15] + s128 + (unsigned)P.crt_k[16 * ch - 1];
       acc = vcphip_v16i{};
 #pragma unroll
       for (int rh = 0; rh < RH; ++rh) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(T.a[ch][rh], b[rh], acc, 0, 0, 0);
@@ -105,9 +144,14 @@ VCPHIP_DEVINL bool vcphip_crt_from_residues(const unsigned (&u)[N], const Vcphip
     for (int v = 0; v < 16; ++v) {
       const int c = 16 * ch + v - 7;   // weight byte c
       if (c < 0 || c >= N) continue;
-      limb[c >> 2] += (long long)(unsigned)(acc[v] + s128 + P.crt_k[16 * ch + v]) << (8 * (c & 3));   // < 2^21
+      if (c % 2 == 0 && c + 1 < N && v + 1 < 16) half[c >> 1] = pair(ch, v);
+      else if (c % 2 == 0 && c + 1 >= N) half[c >> 1] = (unsigned)acc[v] + s128 + (unsigned)P.crt_k[16 * ch + v];
+      else if (c % 2 == 1 && v == 0) half[c >> 1] = last + (((unsigned)acc[v] + s128 + (unsigned)P.crt_k[16 * ch]) << 8);
     }
   }
+#pragma unroll
+  for (int l = 0; l < NL; ++l)
+    limb[l] += (long long)((unsigned long long)half[2 * l] + ((unsigned long long)half[2 * l + 1] << 16));
   long long carry = 0;
 #pragma unroll
   for (int l = 0; l < NL; ++l) {
@@ -128,15 +172,34 @@ VCPHIP_DEVINL bool vcphip_crt_from_residues(const unsigned (&u)[N], const Vcphip
   return neg;
 }
 
-// Residues of element o (< 256) of a 16 x 16 plane block from N planes of
-// `plane` bytes, U being the block's base in the first plane (workgroup-
-// uniform): one buffer load per plane, from a scalar resource at the lane's
-// offset.
-template <int N, int NL>
-VCPHIP_DEVINL bool vcphip_crt_symmetric(const uint8_t* __restrict__ U, long plane, unsigned o,
-                                        const VcphipCrtOps<N>& T, const VcphipOzParams& P, unsigned (&mag)[NL]) {
-  unsigned u[N];
+// A 16 x 16 block of results, EL of its four rows of a column per lane, to C
+// through the block's LDS copy: 256 contiguous bytes per column instead of 16
+// scattered ones per lane.  EL = 4: a wave's own block; EL = 1: the block of
+// the workgroup's four waves, wave e0 holding element e0 of each lane.
+struct VcphipBlockOut {
+  static constexpr int LD = 17;   // an odd column stride in 16-byte slots
+  double2 v[16 * LD];
+};
+template <int EL>
+VCPHIP_DEVINL void vcphip_block_store(VcphipBlockOut& L, const double2 (&v)[EL], unsigned lane, int e0,
+                                      double* __restrict__ C, long ldc, int i0, int j0, int m, int n) {
 #pragma unroll
-  for (int t = 0; t < N; ++t) u[t] = __builtin_amdgcn_raw_buffer_load_b8(vcphip_rsrc(U + (long)t * plane, 256), o, 0, 0);
-  return vcphip_crt_from_residues<N, NL>(u, T, P, mag);
+  for (int e = 0; e < EL; ++e) L.v[(lane & 15) * VcphipBlockOut::LD + 4 * (lane >> 4) + e0 + e] = v[e];
+  if (EL == 4) __builtin_amdgcn_wave_barrier();   // LDS operations of a wave stay in order
+  else __syncthreads();
+  const int i = i0 + (int)(lane & 15);
+#pragma unroll
+  for (int e = 0; e < EL; ++e) {
+    const int c = 4 * (e0 + e) + (int)(lane >> 4), j = j0 + c;
+    if (i < m && j < n)
+      *reinterpret_cast<double2*>(C + 2 * (i + ldc * (long)j)) = L.v[c * VcphipBlockOut::LD + (lane & 15)];
+  }
 }
+
+// Blocks up to which a reconstruction gives each block four waves (EL = 1)
+// instead of one.  One wave shares the weights, tables and scalar work of a
+// block's elements, four fill the chip and shorten the chain; interval / dd
+// form, one against four waves: n = 500 12.4 / 12.4 against 9.2 / 9.9 us, 1000
+// 20 / 24 against 18 / 19, 1300 (7744 blocks) 32 / 33 against 28 / 30, 2000
+// (16384) 68 / 71 against 73 / 75.
+constexpr long VCPHIP_CRT_SPLIT_BLOCKS = 8192;

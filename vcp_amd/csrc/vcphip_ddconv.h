@@ -142,28 +142,25 @@ VCPHIP_HD void limbs_hi_lo(const unsigned (&mag)[NL], int sc, double& hi, double
 // false otherwise, and then the limb path gives the result.  Where it
 // applies the two paths agree bit for bit.
 VCPHIP_HD bool window_hi_lo(const unsigned (&mag)[NL], int sc, double& hi, double& lo) {
-  int lt = -1;
+  // the top limb to the front, by conditional moves of 4, 2 and 1 limbs
+  unsigned x[NL];
 #pragma unroll
-  for (int l = 0; l < NL; ++l)
-    if (mag[l] != 0) lt = l;
-  if (lt < 0) {
+  for (int l = 0; l < NL; ++l) x[l] = mag[l];
+  int lt = NL - 1;
+#pragma unroll
+  for (int h = NL / 2; h > 0; h >>= 1) {
+    unsigned any = 0;
+#pragma unroll
+    for (int l = NL - h; l < NL; ++l) any |= x[l];
+    const bool mv = any == 0;
+#pragma unroll
+    for (int l = NL - 1; l >= 0; --l) x[l] = mv ? (l >= h ? x[l - h] : 0u) : x[l];
+    lt -= mv ? h : 0;
+  }
+  const unsigned w4 = x[7], w3 = x[6], w2 = x[5], w1 = x[4], w0 = x[3], below = x[2] | x[1] | x[0];
+  if (w4 == 0) {
     hi = lo = 0.0;
     return true;
-  }
-  unsigned orp[NL + 1];   // orp[l] = OR of limbs below l
-  orp[0] = 0;
-#pragma unroll
-  for (int l = 0; l < NL; ++l) orp[l + 1] = orp[l] | mag[l];
-  unsigned w4 = 0, w3 = 0, w2 = 0, w1 = 0, w0 = 0, below = 0;
-#pragma unroll
-  for (int l = 0; l < NL; ++l) {
-    const bool c = l == lt;
-    w4 = c ? mag[l] : w4;
-    w3 = c ? (l >= 1 ? mag[l - 1] : 0u) : w3;
-    w2 = c ? (l >= 2 ? mag[l - 2] : 0u) : w2;
-    w1 = c ? (l >= 3 ? mag[l - 3] : 0u) : w1;
-    w0 = c ? (l >= 4 ? mag[l - 4] : 0u) : w0;
-    below = c ? (l >= 5 ? orp[l - 4] : 0u) : below;
   }
   const bool s0 = below != 0;
   const int b = 31 - __builtin_clz(w4);
