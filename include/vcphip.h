@@ -22,10 +22,10 @@
  * allocate their handle's own.  A batch of inverses spreads its groups of
  * equal padded order over the context stream and three more streams of its
  * own (default priority), forked from and joined back to the context stream,
- * so the batch stays ordered on that stream.  Host-pointer copies above 8 MiB are staged
- * through two pinned host buffers of 128 MiB that the context allocates on
- * first use and holds until it is destroyed.  A context is used by one host
- * thread at a time.
+ * so the batch stays ordered on that stream.  Host-pointer copies are staged
+ * through pinned host memory that the context allocates on first use and holds
+ * until it is destroyed: two buffers of 128 MiB from 8 MiB on, one of at most
+ * 24 MiB below.  A context is used by one host thread at a time.
  *
  * Every function returns VCPHIP_OK (0) or a negative VCPHIP_ERR_* code;
  * vcphip_strerror() names it.  vcp/error.hpp:42-114 is the exception
