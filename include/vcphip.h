@@ -153,7 +153,9 @@ int vcphip_ozaki_config(int k, int nmod, int* beta, int* moduli, int max_moduli)
 /* ---- interval x interval: C = IA * IB ----------------------------------- */
 /* Replaces vcp::pidblas::mulmm (vcp/pidblas.hpp:239-294), i.e. the four
  * dgemm_ calls at :266,271,279,281 under kv::hwround and the n^2 fix-ups
- * (forms PLAIN and OZAKI), and vcp::pidblas_fma::mulmm (form INFSUP). */
+ * (forms PLAIN and OZAKI), and vcp::pidblas_fma::mulmm (form INFSUP).
+ * C may lie over an operand (A <- A B) in the forms PLAIN and OZAKI; so may
+ * the results of vcphip_igemm_ip, vcphip_igemm_pi and vcphip_gemm_rurd. */
 int vcphip_igemm(vcphip_ctx* ctx, int form, int m, int n, int k,
                  const double* IA, int lda, const double* IB, int ldb, double* C, int ldc);
 int vcphip_igemm_dev(vcphip_ctx* ctx, int form, int m, int n, int k,

@@ -921,10 +921,21 @@ bool thin_product(const vcphip_ctx* c, size_t m, size_t n) {
   return n <= 32 || ((m + 7) / 8) * ((n + 63) / 64) <= cus;
 }
 
+// the bytes from the first to the last element of a column-major rows x cols
+// matrix (rows, cols > 0) of e doubles per element
+struct Extent {
+  uintptr_t first, last;
+  Extent(const double* p, int e, int rows, int ld, int cols)
+      : first((uintptr_t)p), last(first + sizeof(double) * e * ((size_t)(cols - 1) * ld + rows) - 1) {}
+  bool meets(const Extent& o) const { return first <= o.last && o.first <= last; }
+};
+
 // A single product of kind VCPHIP_DR_*: the operand planes (midpoint and
 // radius of an interval operand, the point operand itself), padded and laid
 // out for whole k-slices, then the product from them.  k = 0 (an all-zero or,
-// accumulating, unchanged product) takes the tile kernel.
+// accumulating, unchanged product) takes the tile kernel.  The planes are
+// copies, so a result may lie over an operand (A <- A B, X <- R X); the
+// row-serial form reads the operands while it stores, and is not taken then.
 int planes_product(vcphip_ctx* c, int kind, int m, int n, int k, const double* A, int lda, const double* B, int ldb,
                    double* C, int ldc, double* C2 = nullptr, int accumulate = 0) {
   StageTimer T(c);
@@ -934,13 +945,17 @@ int planes_product(vcphip_ctx* c, int kind, int m, int n, int k, const double* A
     T.mark("drgemm");
     return rc;
   }
-  if (thin_product(c, (size_t)m, (size_t)n)) {
+  const bool ai = kind == VCPHIP_DR_II || kind == VCPHIP_DR_IP, bi = kind == VCPHIP_DR_II || kind == VCPHIP_DR_PI;
+  const auto over_operand = [&](const double* X) {
+    const Extent ex(X, ai || bi ? 2 : 1, m, ldc, n);
+    return ex.meets(Extent(A, ai ? 2 : 1, m, lda, k)) || ex.meets(Extent(B, bi ? 2 : 1, k, ldb, n));
+  };
+  if (thin_product(c, (size_t)m, (size_t)n) && !over_operand(C) && !(C2 && over_operand(C2))) {
     const int rc =
         check_launch(vcphip_launch_drgemm_thin(kind, m, n, k, A, lda, B, ldb, C, ldc, C2, accumulate, c->stream));
     T.mark("drgemm");
     return rc;
   }
-  const bool ai = kind == VCPHIP_DR_II || kind == VCPHIP_DR_IP, bi = kind == VCPHIP_DR_II || kind == VCPHIP_DR_PI;
   const size_t mpad = ((size_t)m + 63) / 64 * 64, npad = ((size_t)n + 63) / 64 * 64, kpad = ((size_t)k + 15) / 16 * 16;
   const size_t na = (ai ? 2 : 1) * mpad * kpad, nb = (bi ? 2 : 1) * kpad * npad;
   void* base;
