@@ -368,8 +368,8 @@ int vcphip_lss_dev(vcphip_ctx* ctx, int n, int nrhs, const double* IA, int lda, 
  * R (and ldr) may be NULL, or R[p] NULL for some p: those R_p = inv(mid(IA_p))
  * are formed on the device first, one rocSOLVER batched getrf + getrs per
  * group of equal order (orders bordered by the identity to a multiple of 64).  Returns VCPHIP_ERR_SINGULAR when any such R_p met a
- * zero pivot, else VCPHIP_ERR_VERIFICATION when any normub[p] >= 1 (the
- * other problems' X are valid; a failed problem's X is NaN). */
+ * zero pivot, else VCPHIP_ERR_VERIFICATION when any normub[p] >= 1 or is NaN
+ * (the other problems' X are valid; a failed problem's X is NaN). */
 int vcphip_lss_batched(vcphip_ctx* ctx, int count, const int* n, const int* nrhs,
                        const double* const* IA, const int* lda, const double* const* Ib, const int* ldb,
                        const double* const* R, const int* ldr, double* const* X, const int* ldx,

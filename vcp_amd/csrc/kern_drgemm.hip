@@ -596,25 +596,25 @@ void k_resid_rowsum(const VcphipResidTile* __restrict__ blocks, const VcphipResi
   T::run(op, lds, p.n, 1, p.n, tl.row0, 0, (int)((blockIdx.x >> 8) % T::NW));
 }
 
-// ||C_p||_inf upper bound: the largest row sum (mats.hpp:1592-1598).  One
-// workgroup per problem; the maximum is exact in any order.
+// ||C_p||_inf upper bound: the largest row sum (mats.hpp:1592-1598), by the
+// rule that the verified solve's norm follows; one workgroup per problem
 __global__ __launch_bounds__(256) void k_resid_max(int count, const VcphipResidProblem* __restrict__ probs,
                                                    const double* __restrict__ rowsum, double* __restrict__ normub) {
   __shared__ double red[256];
   const int pi = blockIdx.x;
   const VcphipResidProblem p = probs[pi];
-  double best = -1.0;   // row sums are >= 0
+  if (p.n <= 0) {
+    if (threadIdx.x == 0) normub[pi] = 0.0;
+    return;
+  }
+  const double* in = rowsum + p.row_base;
+  double best = -__builtin_inf();
   for (int i = threadIdx.x; i < p.n; i += 256) {
-    const double v = rowsum[p.row_base + i];
+    const double v = in[i];
     best = v > best ? v : best;
   }
-  red[threadIdx.x] = best;
-  __syncthreads();
-  for (int h = 128; h > 0; h >>= 1) {
-    if ((int)threadIdx.x < h) red[threadIdx.x] = red[threadIdx.x + h] > red[threadIdx.x] ? red[threadIdx.x + h] : red[threadIdx.x];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) normub[pi] = p.n > 0 ? red[0] : 0.0;
+  const double norm = vcphip_block_max<256>(best, in[0], red);
+  if (threadIdx.x == 0) normub[pi] = norm;
 }
 
 // ---------------------------------------------------------------------------

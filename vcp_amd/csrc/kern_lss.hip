@@ -284,24 +284,8 @@ struct LssFinal {
   }
 };
 
-// T = ||y||_inf (upward row sums over the columns, then mats.hpp:1593-1598's
-// maximum: best = in[0], then in[i] where in[i] > best, so NaN exactly when
-// in[0] is and otherwise the largest non-NaN), by one workgroup of NT threads
-VCPHIP_DEVINL double lss_block_max(double best, double first, double* red) {
-  red[threadIdx.x] = best;
-  __syncthreads();
-  for (int s = NT / 2; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) {
-      const double o = red[threadIdx.x + s];
-      red[threadIdx.x] = o > red[threadIdx.x] ? o : red[threadIdx.x];
-    }
-    __syncthreads();
-  }
-  const double r = red[0];
-  __syncthreads();
-  return __builtin_isnan(first) ? first : r;
-}
-
+// T = ||y||_inf: upward row sums over the columns, then their maximum, by one
+// workgroup of NT threads
 VCPHIP_DEVINL double lss_ynorm(const VcphipLssProblem& P, double* red, double* first) {   // round-up mode
   double best = -__builtin_inf();
   for (int i = threadIdx.x; i < P.n; i += NT) {
@@ -316,7 +300,7 @@ VCPHIP_DEVINL double lss_ynorm(const VcphipLssProblem& P, double* red, double* f
     best = s > best ? s : best;
   }
   __syncthreads();
-  return lss_block_max(best, *first, red);
+  return vcphip_block_max<NT>(best, *first, red);
 }
 
 // ---- one system ---------------------------------------------------------------
@@ -354,7 +338,7 @@ __global__ __launch_bounds__(NT) void k_lss_g(VcphipLssProblem P, const double* 
     const double v = rows[i];
     best = v > best ? v : best;
   }
-  const double g = lss_block_max(best, rows[0], red);
+  const double g = vcphip_block_max<NT>(best, rows[0], red);
   const double t = lss_ynorm(P, red, &first);
   if (threadIdx.x == 0) {
     sg = g;

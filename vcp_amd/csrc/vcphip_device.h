@@ -89,6 +89,26 @@ VCPHIP_DEVINL void vcphip_mode_nearest() {
   asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 4), 0" ::: "memory");
 }
 
+// The reference's maximum (vcp/mats.hpp:1593-1598) over a workgroup of NT
+// threads: best = in[0], then in[i] where in[i] > best, so NaN exactly when
+// in[0] is (first) and otherwise the largest non-NaN.  best: each thread's
+// largest, from -infinity; every thread gets the result.
+template <int NT>
+VCPHIP_DEVINL double vcphip_block_max(double best, double first, double* red) {
+  red[threadIdx.x] = best;
+  __syncthreads();
+  for (int s = NT / 2; s > 0; s >>= 1) {
+    if ((int)threadIdx.x < s) {
+      const double o = red[threadIdx.x + s];
+      red[threadIdx.x] = o > red[threadIdx.x] ? o : red[threadIdx.x];
+    }
+    __syncthreads();
+  }
+  const double r = red[0];
+  __syncthreads();
+  return __builtin_isnan(first) ? first : r;
+}
+
 // 2^e as a double for e in [-1022, 1023] (bit construction, exact)
 VCPHIP_DEVINL double vcphip_pow2(int e) {
   return __longlong_as_double((long long)(e + 1023) << 52);
