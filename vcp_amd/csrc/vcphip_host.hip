@@ -914,9 +914,11 @@ int syrk_rows(const vcphip_ctx* c, size_t npad) {
 // blocks number at most one per CU the 32 x 64 tiles leave most CUs idle
 // (interval x interval, n = k = m = 96: 6 against 27 us, 300: 19 against 46,
 // 400: 38 against 62, but 512 at half the tiles' throughput when products on
-// several streams fill the device).  A forced plane shape takes the planes.
+// several streams fill the device).  A forced plane shape takes the planes,
+// and so does m from 2^26 on: a launch holds fewer than 2^32 threads, and up
+// to 512 of them take 8 rows.
 bool thin_product(const vcphip_ctx* c, size_t m, size_t n) {
-  if (c->plane_rows) return false;
+  if (c->plane_rows || m >= (size_t)1 << 26) return false;
   const size_t cus = c->num_cu > 0 ? (size_t)c->num_cu : 256;
   return n <= 32 || ((m + 7) / 8) * ((n + 63) / 64) <= cus;
 }
