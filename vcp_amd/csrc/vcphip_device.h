@@ -109,6 +109,15 @@ VCPHIP_DEVINL double vcphip_block_max(double best, double first, double* red) {
   return __builtin_isnan(first) ? first : r;
 }
 
+// a wave's LDS writes before it are seen by its lanes' reads after it, and its
+// reads before it precede its writes after it (a wave's LDS operations stay in
+// order; this keeps the compiler to that order)
+VCPHIP_DEVINL void vcphip_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // 2^e as a double for e in [-1022, 1023] (bit construction, exact)
 VCPHIP_DEVINL double vcphip_pow2(int e) {
   return __longlong_as_double((long long)(e + 1023) << 52);
