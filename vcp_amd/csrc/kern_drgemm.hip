@@ -373,7 +373,7 @@ struct PlaneStage {
 // lines of the two result matrices an element at a time.  RU / RD product, one
 // context, element-wise against through LDS (results / results and accumulated
 // values): 2048 x 2048 x 64 148 against 36 us / 100 against 44, 4096 x 4096 x
-// 128 245 against 180 / 320 against 202, 2000 x 2000 x 2000 657 against 597 /
+// 128 245 against 180 / 320 against 202, 2000 x 2000 x 2000 616 against 597 /
 // 722 against 593.  In LDS a column's pairs of rows are exchanged by its index,
 // which spreads the accesses of both directions over the banks.
 template <int RPL, int D>
@@ -387,6 +387,7 @@ struct PointBlock {
     const double* l = reinterpret_cast<const double*>(L);
 #pragma unroll
     for (int c0 = 0; c0 < 32; c0 += NC) {
+      if (col0 + c0 >= n) break;   // wave-uniform
       if (lc / NC == c0 / NC) {
 #pragma unroll
         for (int i = 0; i < RPL; i += 2) L[pair(lc % NC, (h * RPL + i) / 2)] = make_double2(v[i], v[i + 1]);
@@ -468,6 +469,7 @@ void k_drgemm_planes(int m, int n, int mpad, int npad, int kpad, const double* _
     r2[i] = 0.0;
   }
   const int wrow = row0 + (w & 1) * 2 * RPL, wcol = col0 + (w >> 1) * 32;   // the wave's block
+  const bool work = __builtin_amdgcn_readfirstlane(wrow < m && wcol < n);   // else it only loads and waits
   const int nt = kpad / Stage::BKS;
   st.issue(0);
   if (!AI && !BI && accumulate) {
@@ -482,6 +484,7 @@ void k_drgemm_planes(int m, int n, int mpad, int npad, int kpad, const double* _
   }
   for (int t = 0; t < nt; ++t) {
     st.next(t, nt);
+    if (!work) continue;
     const char* s0 = sL + (t % Stage::NST) * Stage::BYTES;
     auto rd = [&](int kk, double2& a, double2& b) {
       if (AI) a = *reinterpret_cast<const double2*>(s0 + aoff + kk * Stage::ARB);
@@ -496,6 +499,7 @@ void k_drgemm_planes(int m, int n, int mpad, int npad, int kpad, const double* _
 
   if (!AI && !BI) {
     __syncthreads();   // every wave has read the last stage
+    if (!work) return;
     double2* L = reinterpret_cast<double2*>(sL) + 256 * w;
     PointBlock<RPL, 512>::store(L, up, lane, C, ldc, wrow, wcol, m, n);
 #pragma unroll

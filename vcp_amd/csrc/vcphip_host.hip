@@ -917,10 +917,23 @@ int syrk_rows(const vcphip_ctx* c, size_t npad) {
 // several streams fill the device).  A forced plane shape takes the planes,
 // and so does m from 2^26 on: a launch holds fewer than 2^32 threads, and up
 // to 512 of them take 8 rows.
-bool thin_product(const vcphip_ctx* c, size_t m, size_t n) {
+//
+// Few columns of many rows: a row block's start-up at short k, and with an
+// interval B (bi) the conversions of B in every block, cost more than the
+// tiles' padding once the row blocks fill the device.  Row-serial against
+// planes, three contexts in turn / one (us): 100000 x 8 x 16 35 / 37 against
+// 19 / 30 (ii), at k = 64 58 / 64 against 79 / 104; 100000 x 16 x 32 43 / 46
+// against 23 / 34 (pi), 51 / 53 against 39 / 51 (ii), at k = 64 54 / 63 against
+// 54 / 77 and 69 / 74 against 82 / 110; 100000 x 32 x 32 75 / 75 against
+// 49 / 55 (ii), 29 / 32 against 19 / 26 (pp, k = 16), at k = 128 118 / 121
+// against 136 / 190 (ip); 8000 x 32 x 512 41 / 45 against 26 / 49 (pi),
+// 54 / 55 against 44 / 70 (ii); 6000 x 32 x 6000 353 against 378 (pi).
+bool thin_product(const vcphip_ctx* c, size_t m, size_t n, size_t k, bool bi) {
   if (c->plane_rows || m >= (size_t)1 << 26) return false;
-  const size_t cus = c->num_cu > 0 ? (size_t)c->num_cu : 256;
-  return n <= 32 || ((m + 7) / 8) * ((n + 63) / 64) <= cus;
+  const size_t cus = c->num_cu > 0 ? (size_t)c->num_cu : 256, blocks = (m + 7) / 8;
+  if (n > 32) return blocks * ((n + 63) / 64) <= cus;
+  if (n > 16) return blocks <= (bi ? 3 : 16) * cus || (!bi && k >= 128);
+  return blocks <= (n > 8 ? 8 : 16) * cus || k >= 64;
 }
 
 // the bytes from the first to the last element of a column-major rows x cols
@@ -952,7 +965,7 @@ int planes_product(vcphip_ctx* c, int kind, int m, int n, int k, const double* A
     const Extent ex(X, ai || bi ? 2 : 1, m, ldc, n);
     return ex.meets(Extent(A, ai ? 2 : 1, m, lda, k)) || ex.meets(Extent(B, bi ? 2 : 1, k, ldb, n));
   };
-  if (thin_product(c, (size_t)m, (size_t)n) && !over_operand(C) && !(C2 && over_operand(C2))) {
+  if (thin_product(c, (size_t)m, (size_t)n, (size_t)k, bi) && !over_operand(C) && !(C2 && over_operand(C2))) {
     const int rc =
         check_launch(vcphip_launch_drgemm_thin(kind, m, n, k, A, lda, B, ldb, C, ldc, C2, accumulate, c->stream));
     T.mark("drgemm");
@@ -2060,7 +2073,7 @@ extern "C" int vcphip_lss_dev(vcphip_ctx* c, int n, int nrhs, const double* IA, 
   int rc = 0;
   // mx = R * mid(b), nearest rounding (:299-302); y = |R * (IA*mx - b)| (:305-315)
   rc |= vcphip_lss_launch_mx(P, s);
-  if (thin_product(c, (size_t)n, (size_t)nrhs)) {
+  if (thin_product(c, (size_t)n, (size_t)nrhs, (size_t)n, true)) {
     rc |= vcphip_lss_launch_ax(P, s);
     rc |= vcphip_lss_launch_ry(P, s);
   } else {   // many right-hand sides: the tiled products and elementwise steps
