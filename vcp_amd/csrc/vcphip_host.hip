@@ -5,6 +5,7 @@
 // entry points enqueue on the stream and return.  Parameters of the Ozaki
 // form (moduli, scale exponent, CRT constants) are derived here on the host.
 #include <fenv.h>
+#include <limits.h>
 #include <math.h>
 #include <stdio.h>
 #include <stdlib.h>
@@ -172,25 +173,40 @@ constexpr int DEFAULT_VARIANT = 15;
 
 // the tile an int8 product of nz planes runs, and the padded m and n it takes:
 // the set or tuned variant, else 256 x 256, or 128 x 128 where that grid is
-// short or mostly padding.  Two 128 x 128 workgroups share a CU and hide each
-// other's prologue, but read twice the operand bytes from LDS per product and
-// run at 0.83-0.87 of the rate once the chip is full (n = 4096 1.54 against
-// 1.34 ms).  int8 stage, 128 against 256 (interval form, 22 planes): n = 200
-// 10.3 against 15.4 us, 500 15.8 against 22.2, 800 32 against 39, 1000 (352
-// tiles of 256) 41 against 42, 1000 x 2000 x 2000 (704) 115 against 105; by
-// padding 1050 57 against 68, 1300 (0.84 of the padded area) 82 against 95,
-// 100 x 4000 x 1000 30 against 42.
+// short or mostly padding.  Two 128 x 128 workgroups share a CU, hide each
+// other's prologue and leave less of the last round idle, but read twice the
+// operand bytes per product: with the chip full they run at about the rate of
+// the 256 x 256 tile up to k = 1000, at 0.9 of it at 2000, 0.85 at 4500 and
+// 0.7 - 0.8 from 16384 on.  So both lines, the 256 x 256 tiles of all planes
+// per CU and the share of the padded area that 128 x 128 tiles need, fall with
+// k.  Times of whole products, 128 / 256, three contexts in turn and one, on
+// 256 CUs: 88 tiles (n = 500) 0.93, 0.80 at k = 1000, 0.94, 0.79 at 2000, 0.96,
+// 0.75 at 4500, 1.02, 0.77 at 8192, 1.10, 0.77 at 32768; 198 (n = 700) 0.97,
+// 0.94 at 1000, 1.09, 0.91 at 2000, 1.17, 0.86 at 4500; 352 (n = 1000) 0.97,
+// 0.95 at 300, 1.01, 1.00 at 1000, 1.10, 0.99 at 2000; 432 (dd 1000) 0.96, 0.98
+// at 300, 1.01, 1.04 at 1000.  By area: 0.84 (n = 1300) 0.97, 0.89 at 1000,
+// 1.03, 0.91 at 2000, 1.06, 0.92 at 3000; 0.81 (1100) 1.00, 0.92 at 3000, 1.06,
+// 0.90 at 4500; 0.75 (4000 x 300) 1.00, 0.97 at 4500, 1.07, 0.99 at 8192; 0.69
+// (600) 1.00, 0.74 at 8192, 1.09, 0.75 at 32768; 0.5 (100 x 4000) 0.91, 0.86 at
+// 32768.
 struct OzTile {
   int variant = 0, mpad = 0, npad = 0;
 };
-OzTile oz_tile(const vcphip_ctx* c, int variant, int m, int n, int nz) {
+OzTile oz_tile(const vcphip_ctx* c, int variant, int m, int n, int k, int nz) {
   const auto up = [](int x, int to) { return (int)(((long)x + to - 1) / to * to); };
   OzTile t{variant ? variant : DEFAULT_VARIANT, up(m, VCPHIP_OZ_PADMN), up(n, VCPHIP_OZ_PADMN)};
   if (variant) return t;
   const long cus = c->num_cu > 0 ? c->num_cu : 256;
   const OzTile h{VCPHIP_OZ_TILE128, up(m, 128), up(n, 128)};
   const long area = (long)t.mpad * t.npad, harea = (long)h.mpad * h.npad;
-  return area / (256 * 256) * nz <= 2 * cus || 20 * harea <= 17 * area ? h : t;
+  struct Line {
+    int k, eighths, percent;   // up to k: 256 x 256 tiles per CU (in eighths), padded area
+  };
+  constexpr Line lines[] = {{640, 16, 85},  {1280, 11, 85}, {2048, 4, 85}, {3072, 3, 82},
+                            {6144, 3, 76}, {16384, 3, 70}, {INT_MAX, 2, 60}};
+  const Line* l = lines;
+  while (k > l->k) ++l;
+  return 8 * (area / (256 * 256) * nz) <= l->eighths * cus || 100 * harea <= l->percent * area ? h : t;
 }
 
 int size_class(int x) {
@@ -749,7 +765,7 @@ static int oz_plan(vcphip_ctx* c, int m, int n, int k, OzPlan& p) {
   if (rc) return rc;
   oz_set_radius(&p.P, oz_radius_scheme(c, tuned, k));
   p.nz = p.P.rnz;
-  p.tile = oz_tile(c, c->oz_variant ? (int)c->oz_variant : (tuned ? tuned->variant : 0), m, n, p.nmod + p.nz);
+  p.tile = oz_tile(c, c->oz_variant ? (int)c->oz_variant : (tuned ? tuned->variant : 0), m, n, k, p.nmod + p.nz);
   // the buffers of the widest padding, whichever tile runs
   const size_t mpad = ((size_t)m + VCPHIP_OZ_PADMN - 1) / VCPHIP_OZ_PADMN * VCPHIP_OZ_PADMN;
   const size_t npad = ((size_t)n + VCPHIP_OZ_PADMN - 1) / VCPHIP_OZ_PADMN * VCPHIP_OZ_PADMN;
@@ -1083,7 +1099,7 @@ static int dd_gemm_dev(vcphip_ctx* c, bool tn, int m, int n, int k, const double
   int rc = dd_make_params(k, nmod, &P);
   if (rc) return rc;
   const vcphip_ctx::Tune* tuned = tune_find(c, TUNE_DDGEMM, m, n, k);
-  const OzTile tile = oz_tile(c, c->oz_variant ? (int)c->oz_variant : (tuned ? tuned->variant : 0), m, n, nmod);
+  const OzTile tile = oz_tile(c, c->oz_variant ? (int)c->oz_variant : (tuned ? tuned->variant : 0), m, n, k, nmod);
   const int mpad = tile.mpad, npad = tile.npad;
   const int kpad = k > 0 ? (k + VCPHIP_OZ_PADK - 1) / VCPHIP_OZ_PADK * VCPHIP_OZ_PADK : VCPHIP_OZ_PADK;
   void *pa = nullptr, *pb, *pu, *st;
