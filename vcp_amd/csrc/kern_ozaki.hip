@@ -1319,29 +1319,33 @@ int vcphip_oz_split(const double* A, long lda, int m, int mpad, VcphipOzSide sa,
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
-// tile variants (all bit-identical): 6 / 7 = k_oz_gemm3 256 x 256 / 128 x 256;
+// tile variants (all bit-identical): 6 = k_oz_gemm3 256 x 256; 7
+// (VCPHIP_OZ_TILE128) = k_oz_gemm5 128 x 128, four waves of 64 x 64;
 // 8 / 9 / 10 = k_oz_gemm4 256 x 256 with 4 / 3 stages, 128 x 256 with 4;
 // 13 / 14 = k_oz_gemm4 256 x 256 with the refill loads spread over the
 // MFMAs (4 / 3 stages); 11 / 12 = k_oz_gemm5 (32 x 32 x 32 MFMA, 4 waves,
 // 4 / 3 stages); 15 / 16 = k_oz_gemm5 with 8 waves of 128 x 64 (4 / 3 stages);
-// VCPHIP_OZ_TILE128 = k_oz_gemm5 128 x 128, four waves of 64 x 64
+// 17 / 18 = k_oz_gemm6 256 x 384 (3 / 2 stages).  (A 128 x 256 k_oz_gemm3 was
+// 7 before: over n = 500 to 2300 and k = 300 to 32768 it was never the faster
+// of itself, 128 x 128 and 15.)
 int vcphip_oz_gemm(int mpad, int npad, int kpad, int nmod, int nrad, const int8_t* Aplanes,
                    const int8_t* Bplanes, const VcphipOzParams& P, uint8_t* U, int32_t* Z, int variant,
                    hipStream_t s) {
   const int nz = nmod + nrad;
   const int by_plane = (long)(mpad / 128) * (npad / 128) <= 4 * 128;   // k_oz_gemm5
   switch (variant) {
-    case 6:
-    case 7: {
-      const int fm = variant == 6 ? 8 : 4, fn = variant == 6 ? 8 : 8;
+    case 6: {
       if (kpad % 64) return -7;
-      const int tiles = (mpad / (32 * fm)) * (npad / (32 * fn));
-      if (variant == 6)
-        hipLaunchKernelGGL((k_oz_gemm3<8, 8>), dim3(tiles * nz), dim3(256), 0, s, mpad, npad, kpad, nmod, nz, Aplanes,
-                           Bplanes, P, U, Z);
-      else
-        hipLaunchKernelGGL((k_oz_gemm3<4, 8>), dim3(tiles * nz), dim3(256), 0, s, mpad, npad, kpad, nmod, nz, Aplanes,
-                           Bplanes, P, U, Z);
+      const int tiles = (mpad / 256) * (npad / 256);
+      hipLaunchKernelGGL((k_oz_gemm3<8, 8>), dim3(tiles * nz), dim3(256), 0, s, mpad, npad, kpad, nmod, nz, Aplanes,
+                         Bplanes, P, U, Z);
+      break;
+    }
+    case VCPHIP_OZ_TILE128: {
+      if (kpad % 64 || mpad % 128 || npad % 128) return -7;
+      const int tiles = (mpad / 128) * (npad / 128);
+      hipLaunchKernelGGL((k_oz_gemm5<2, 2, 4>), dim3(tiles * nz), dim3(256), 0, s, mpad, npad, kpad, nmod, by_plane,
+                         Aplanes, Bplanes, P, U, Z);
       break;
     }
     case 8:
@@ -1407,13 +1411,6 @@ int vcphip_oz_gemm(int mpad, int npad, int kpad, int nmod, int nrad, const int8_
       else
         hipLaunchKernelGGL((k_oz_gemm6<2>), dim3(tiles * nz), dim3(512), 0, s, mpad, npad, kpad, nmod, nz, Aplanes,
                            Bplanes, P, U, Z);
-      break;
-    }
-    case VCPHIP_OZ_TILE128: {
-      if (kpad % 64 || mpad % 128 || npad % 128) return -7;
-      const int tiles = (mpad / 128) * (npad / 128);
-      hipLaunchKernelGGL((k_oz_gemm5<2, 2, 4>), dim3(tiles * nz), dim3(256), 0, s, mpad, npad, kpad, nmod, by_plane,
-                         Aplanes, Bplanes, P, U, Z);
       break;
     }
     default: return -7;

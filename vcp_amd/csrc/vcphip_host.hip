@@ -194,10 +194,10 @@ struct OzTile {
 };
 OzTile oz_tile(const vcphip_ctx* c, int variant, int m, int n, int k, int nz) {
   const auto up = [](int x, int to) { return (int)(((long)x + to - 1) / to * to); };
-  OzTile t{variant ? variant : DEFAULT_VARIANT, up(m, VCPHIP_OZ_PADMN), up(n, VCPHIP_OZ_PADMN)};
-  if (variant) return t;
-  const long cus = c->num_cu > 0 ? c->num_cu : 256;
+  const OzTile t{variant ? variant : DEFAULT_VARIANT, up(m, VCPHIP_OZ_PADMN), up(n, VCPHIP_OZ_PADMN)};
   const OzTile h{VCPHIP_OZ_TILE128, up(m, 128), up(n, 128)};
+  if (variant) return variant == VCPHIP_OZ_TILE128 ? h : t;
+  const long cus = c->num_cu > 0 ? c->num_cu : 256;
   const long area = (long)t.mpad * t.npad, harea = (long)h.mpad * h.npad;
   struct Line {
     int k, eighths, percent;   // up to k: 256 x 256 tiles per CU (in eighths), padded area
@@ -734,10 +734,12 @@ extern "C" int vcphip_ozaki_plan(vcphip_ctx* c, int m, int n, int k, int* nmod, 
   const vcphip_ctx::Tune* tuned = tune_find(c, TUNE_IGEMM, m, n, k);
   const int nm = c->oz_nmod ? (int)c->oz_nmod : (tuned && tuned->nmod ? tuned->nmod : default_nmod(k));
   const int rad = oz_radius_scheme(c, tuned, k);
-  const int var = c->oz_variant ? (int)c->oz_variant : (tuned && tuned->variant ? tuned->variant : DEFAULT_VARIANT);
+  VcphipOzParams P;
+  oz_set_radius(&P, rad);
+  const OzTile tile = oz_tile(c, c->oz_variant ? (int)c->oz_variant : (tuned ? tuned->variant : 0), m, n, k, nm + P.rnz);
   if (nmod) *nmod = nm;
   if (radius) *radius = rad;
-  if (variant) *variant = var;
+  if (variant) *variant = tile.variant;
   // residue products plus hi x hi, two mixed and (full) lo x lo per radius term
   if (products) *products = nm + oz_radius_products(rad);
   return VCPHIP_OK;
@@ -3118,9 +3120,10 @@ int tune_gemm_stage(vcphip_ctx* c, bool dd, int m, int n, int k, int* best_varia
   double best_t = 0.0;
   rc = VCPHIP_OK;
   for (int v : TUNE_VARIANTS) {
+    const OzTile tile = oz_tile(c, v, m, n, k, nmod + nrad);   // with the padding that a product with v takes
     auto launch = [&]() {
-      return vcphip_oz_gemm(mpad, npad, kpad, nmod, nrad, (const int8_t*)pa, (const int8_t*)pb, P, (uint8_t*)pu,
-                            (int32_t*)pz, v, c->stream);
+      return vcphip_oz_gemm(tile.mpad, tile.npad, kpad, nmod, nrad, (const int8_t*)pa, (const int8_t*)pb, P,
+                            (uint8_t*)pu, (int32_t*)pz, v, c->stream);
     };
     if (launch() != 0) {   // variant not applicable to this shape
       hipGetLastError();

@@ -95,7 +95,7 @@ int vcphip_fill_f64(double* p, long n, double v, hipStream_t s);
 #define VCPHIP_OZ_MAXRAD 6
 #define VCPHIP_OZ_CHUNK 256   // k-chunk of the upward 1-norm partial sums
 #define VCPHIP_OZ_PADMN 256   // m and n are padded to multiples of this (128 for VCPHIP_OZ_TILE128)
-#define VCPHIP_OZ_TILE128 19  // 128 x 128 int8 GEMM tiles (m and n padded to 128); not a settable variant
+#define VCPHIP_OZ_TILE128 7   // the variant with 128 x 128 int8 GEMM tiles (m and n padded to 128)
 #define VCPHIP_OZ_PADK 128    // k is padded to a multiple of this
 #define VCPHIP_OZ_NLIMB 8     // 32-bit limbs of M (M < 2^256)
 #define VCPHIP_OZ_CRTCOL 48   // CRT columns: N weight bytes, 6 quotient bytes, the residue sum (3 x 16)
