@@ -213,7 +213,8 @@ struct LssRy : VcphipThinDr<false, true> {
 
 // upper end of the row sums of |RA - I| (mats::norminf, vcp/mats.hpp:
 // 1587-1592): s = mag(c_i0), then s = RU(s + mag(c_ij)) for j = 1, 2, ...
-// C holds R A; the unit diagonal is subtracted on load
+// DIAG: C holds R A, and the unit diagonal is subtracted on load
+template <bool DIAG>
 struct LssRowSum {
   static constexpr bool A2 = true, B2 = false, PAD16 = false;
   static constexpr int AL = 1, BL = 0;
@@ -225,7 +226,7 @@ struct LssRowSum {
     double s;
   };
   VCPHIP_DEVINL double2 a(double2 v, int row, int kk) const {
-    if (row == kk) v = lss_minus_one(v);
+    if (DIAG && row == kk) v = lss_minus_one(v);
     const double p = __builtin_fabs(v.x), q = __builtin_fabs(v.y);
     return make_double2(p > q ? p : q, 0.0);
   }
@@ -238,8 +239,13 @@ struct LssRowSum {
 // W = |RA - I| G (the II product with the constant column G, one column for
 // all right-hand sides; its lower chain is not used) and X = mx + [-u, u],
 // u = RU(|y|u + Wu) (imats.hpp:343-361).  The eight column lanes carry the
-// same chain and share the right-hand sides.  DIAG: C holds R A, and the unit
-// diagonal is subtracted on load.
+// same chain and share a group of right-hand sides, a workgroup per row block
+// and group: one group for all of them left 8 rows x nrhs steps to one wave (a
+// whole solve of n = 64 with 4096 right-hand sides 1151 us; 118 with groups and
+// the row sums of |y| spread over workgroups, 2000 with 2000 11.4 and 4.2 ms).
+// DIAG: C holds R A, and the unit diagonal is subtracted on load.
+__host__ __device__ inline int lss_final_group(int n) { return n > 256 ? n / 4 / 8 * 8 : 64; }   // right-hand sides of a group
+
 template <bool DIAG>
 struct LssFinal {
   static constexpr bool A2 = true, B2 = false, PAD16 = false;
@@ -250,13 +256,15 @@ struct LssFinal {
   const double *y, *mx;
   double* X;
   long ldx;
-  int n, nrhs;
+  int n, j0, j1;
   double bm, br;
   struct Acc {
     double up, r1, r2;
   };
-  VCPHIP_DEVINL explicit LssFinal(const VcphipLssProblem& P)
-      : A(P.C), lda(P.n), y(P.y), mx(P.mx), X(P.X), ldx(P.ldx), n(P.n), nrhs(P.nrhs) {
+  VCPHIP_DEVINL LssFinal(const VcphipLssProblem& P, int group)
+      : A(P.C), lda(P.n), y(P.y), mx(P.mx), X(P.X), ldx(P.ldx), n(P.n), j0(group * lss_final_group(P.n)) {
+    const int left = P.nrhs - j0;
+    j1 = j0 + (left < lss_final_group(n) ? left : lss_final_group(n));
     vcphip_midrad_ru(P.norms[2], P.norms[3], bm, br);
   }
   VCPHIP_DEVINL double2 a(double2 v, int row, int kk) const {
@@ -276,16 +284,18 @@ struct LssFinal {
   }
   VCPHIP_DEVINL void done(const Acc& c, int row, int col) const {
     const double wu = c.up + (c.r1 + c.r2);
-    for (int j = col; j < nrhs; j += VCPHIP_THIN_CL) {
-      const long q = row + (long)n * j;
-      const double u = y[2 * q + 1] + wu, m = mx[q];
-      *reinterpret_cast<double2*>(X + 2 * (row + ldx * j)) = make_double2(-(u - m), u + m);
+    const double *__restrict__ yr = y + 2 * row + 1, *__restrict__ mr = mx + row;
+    double* __restrict__ xr = X + 2 * row;
+#pragma unroll 4
+    for (int j = j0 + col; j < j1; j += VCPHIP_THIN_CL) {
+      const double u = yr[2 * (long)n * j] + wu, m = mr[(long)n * j];
+      *reinterpret_cast<double2*>(xr + 2 * ldx * j) = make_double2(-(u - m), u + m);
     }
   }
 };
 
 // T = ||y||_inf: upward row sums over the columns, then their maximum, by one
-// workgroup of NT threads
+// workgroup of NT threads (batched form)
 VCPHIP_DEVINL double lss_ynorm(const VcphipLssProblem& P, double* red, double* first) {   // round-up mode
   double best = -__builtin_inf();
   for (int i = threadIdx.x; i < P.n; i += NT) {
@@ -315,41 +325,49 @@ void k_lss_step(VcphipLssProblem P) {
   T::run(op, lds, P.n, P.nrhs, P.n, rb * T::R, blockIdx.y * T::NC, (int)((blockIdx.x >> 8) % T::NW));
 }
 
-__global__ __launch_bounds__((VcphipThin<LssRowSum, 1>::NT)) VCPHIP_THIN_WAVES
+// the row sums of |RA - I| into rows[0, n) and those of |y| into rows[n, 2n),
+// row blocks of the one, then of the other
+__global__ __launch_bounds__((VcphipThin<LssRowSum<true>, 1>::NT)) VCPHIP_THIN_WAVES
 void k_lss_rowsum(VcphipLssProblem P, double* __restrict__ rows) {
   vcphip_mode_round_up();
-  using T = VcphipThin<LssRowSum, 1>;
+  using T = VcphipThin<LssRowSum<true>, 1>;
+  using Y = VcphipThin<LssRowSum<false>, 1>;
   __shared__ __attribute__((aligned(16))) typename T::Lds lds;
-  LssRowSum op;
-  op.A = P.C;
-  op.lda = P.n;
-  op.out = rows;
-  const int rb = vcphip_xcd_remap(blockIdx.x, gridDim.x);
-  T::run(op, lds, P.n, 1, P.n, rb * T::R, 0, (int)((blockIdx.x >> 8) % T::NW));
+  static_assert(sizeof(T::Lds) == sizeof(Y::Lds), "one buffer for both");
+  const int nrb = gridDim.x / 2, rot = (int)((blockIdx.x >> 8) % T::NW);
+  if ((int)blockIdx.x < nrb) {
+    LssRowSum<true> op;
+    op.A = P.C;
+    op.lda = P.n;
+    op.out = rows;
+    T::run(op, lds, P.n, 1, P.n, vcphip_xcd_remap(blockIdx.x, nrb) * T::R, 0, rot);
+  } else {
+    LssRowSum<false> op;
+    op.A = P.y;
+    op.lda = P.n;
+    op.out = rows + P.n;
+    Y::run(op, reinterpret_cast<typename Y::Lds&>(lds), P.n, 1, P.nrhs, ((int)blockIdx.x - nrb) * Y::R, 0, rot);
+  }
 }
 
-// g = ||RA - I||_inf from its row sums, T = ||y||_inf and G: norms[0 .. 3]
+// g = ||RA - I||_inf and T = ||y||_inf from their row sums, and G: norms[0 .. 3]
 __global__ __launch_bounds__(NT) void k_lss_g(VcphipLssProblem P, const double* __restrict__ rows) {
-  vcphip_mode_round_up();
   __shared__ double red[NT];
-  __shared__ double first, sg, st;
-  double best = -__builtin_inf();
-  for (int i = threadIdx.x; i < P.n; i += NT) {
-    const double v = rows[i];
-    best = v > best ? v : best;
+  double norm[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const double* in = rows + (long)h * P.n;
+    double best = -__builtin_inf();
+    for (int i = threadIdx.x; i < P.n; i += NT) {
+      const double v = in[i];
+      best = v > best ? v : best;
+    }
+    norm[h] = vcphip_block_max<NT>(best, in[0], red);
   }
-  const double g = vcphip_block_max<NT>(best, rows[0], red);
-  const double t = lss_ynorm(P, red, &first);
   if (threadIdx.x == 0) {
-    sg = g;
-    st = t;
-  }
-  __syncthreads();
-  vcphip_mode_nearest();
-  if (threadIdx.x == 0) {   // sg and st are read back after the mode switch
-    const double2 G = lss_bound_factor(sg, st);
-    P.norms[0] = sg;
-    P.norms[1] = st;
+    const double2 G = lss_bound_factor(norm[0], norm[1]);
+    P.norms[0] = norm[0];
+    P.norms[1] = norm[1];
     P.norms[2] = G.x;
     P.norms[3] = G.y;
   }
@@ -361,7 +379,7 @@ void k_lss_final(VcphipLssProblem P) {
   vcphip_mode_round_up();
   using T = VcphipThin<LssFinal<DIAG>, 1>;
   __shared__ __attribute__((aligned(16))) typename T::Lds lds;
-  LssFinal<DIAG> op(P);
+  LssFinal<DIAG> op(P, blockIdx.y);
   const int rb = vcphip_xcd_remap(blockIdx.x, gridDim.x);
   T::run(op, lds, P.n, VCPHIP_THIN_CL, P.n, rb * T::R, 0, (int)((blockIdx.x >> 8) % T::NW));
 }
@@ -420,9 +438,10 @@ void k_lssb_final(int count, const long* __restrict__ wb, const VcphipLssProblem
   const int p = find_problem(wb, count, blk);
   const VcphipLssProblem P = probs[p];
   const int nrb = (P.n + T::R - 1) / T::R, q = (int)(blk - wb[p]);
-  if (q >= nrb) return;   // one block per row block serves every right-hand side
-  LssFinal<false> op(P);
-  T::run(op, lds, P.n, VCPHIP_THIN_CL, P.n, q * T::R, 0, (int)((blockIdx.x >> 8) % T::NW));
+  const int per = lss_final_group(P.n) / VCPHIP_THIN_CL;   // blocks of 8 right-hand sides to a group
+  if (q / nrb % per) return;   // the group's first block serves it
+  LssFinal<false> op(P, q / nrb / per);
+  T::run(op, lds, P.n, VCPHIP_THIN_CL, P.n, q % nrb * T::R, 0, (int)((blockIdx.x >> 8) % T::NW));
 }
 
 }  // namespace
@@ -448,9 +467,10 @@ int vcphip_lss_launch_abs(int rows, int cols, double* X, long ldx, hipStream_t s
 }
 
 namespace {
-// columns per workgroup as the single products choose them: 8 up to 8
-// right-hand sides, 64 above (2 MB of R or IA per row block and column group
-// are then read once per 64 right-hand sides)
+// columns per workgroup: 8 up to 8 right-hand sides, 64 above, so that a row
+// block of R or IA (64 n or 128 n bytes) is read once per 64 right-hand sides.
+// (The single products narrow the 64 until about 150 workgroups run; here the
+// step is a small part of the solve.)
 template <class Op, bool UP>
 void lss_step(const VcphipLssProblem& P, hipStream_t s) {
   const unsigned rb = (unsigned)((P.n + VCPHIP_THIN_R - 1) / VCPHIP_THIN_R);
@@ -478,10 +498,12 @@ int vcphip_lss_launch_ry(const VcphipLssProblem& P, hipStream_t s) {
 }
 
 int vcphip_lss_launch_bound(const VcphipLssProblem& P, double* rows, hipStream_t s) {
-  const dim3 rb((unsigned)((P.n + VCPHIP_THIN_R - 1) / VCPHIP_THIN_R));
-  hipLaunchKernelGGL(k_lss_rowsum, rb, dim3(VcphipThin<LssRowSum, 1>::NT), 0, s, P, rows);
+  const unsigned rb = (unsigned)((P.n + VCPHIP_THIN_R - 1) / VCPHIP_THIN_R);
+  hipLaunchKernelGGL(k_lss_rowsum, dim3(2 * rb), dim3(VcphipThin<LssRowSum<true>, 1>::NT), 0, s, P, rows);
   hipLaunchKernelGGL(k_lss_g, dim3(1), dim3(NT), 0, s, P, rows);
-  hipLaunchKernelGGL(k_lss_final<true>, rb, dim3(VcphipThin<LssFinal<true>, 1>::NT), 0, s, P);
+  const int group = lss_final_group(P.n);
+  hipLaunchKernelGGL(k_lss_final<true>, dim3(rb, (unsigned)(((long)P.nrhs + group - 1) / group)),
+                     dim3(VcphipThin<LssFinal<true>, 1>::NT), 0, s, P);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 

@@ -82,13 +82,6 @@ VCPHIP_DEVINL void vcphip_mode_round_up() {
   asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 4), 5" ::: "memory");
 }
 
-// back to round-to-nearest; what the code after it computes must come from
-// values loaded after it, and what it computed before it must be stored
-// before it (the memory clobber orders both)
-VCPHIP_DEVINL void vcphip_mode_nearest() {
-  asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 4), 0" ::: "memory");
-}
-
 // The reference's maximum (vcp/mats.hpp:1593-1598) over a workgroup of NT
 // threads: best = in[0], then in[i] where in[i] > best, so NaN exactly when
 // in[0] is (first) and otherwise the largest non-NaN.  best: each thread's

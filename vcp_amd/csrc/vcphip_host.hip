@@ -2052,7 +2052,7 @@ extern "C" int vcphip_lss_dev(vcphip_ctx* c, int n, int nrhs, const double* IA, 
   const size_t o_mx = 0, o_x = o_mx + up(nr), o_y = o_x + up(2 * nr), o_c = o_y + up(2 * nr);
   const size_t o_r = o_c + up(2 * (size_t)n * n);
   const size_t np = (size_t)inv_order(n);
-  const size_t o_s = o_r + up((size_t)n), o_ri = o_s + al, total = o_ri + (R ? 0 : up(inv_work_doubles(n)));
+  const size_t o_s = o_r + up(2 * (size_t)n), o_ri = o_s + al, total = o_ri + (R ? 0 : up(inv_work_doubles(n)));
   void* base;
   const int wrc = ws_get(c, vcphip_ctx::WS_LSS, total * sizeof(double), &base);
   if (wrc) return wrc;
