@@ -22,19 +22,27 @@ typedef unsigned __int128 u128;
 // stats: per row (or column) the exponent of max |hi| + |lo| (round-up sum)
 // ---------------------------------------------------------------------------
 // rows of a column-major operand: a workgroup takes 8 rows (128-byte runs of a
-// column) over the whole of len, 8 loads in flight per thread.  The maximum
-// does not depend on the order.
+// column) over k0 .. len, 8 loads in flight per thread.  The maximum does not
+// depend on the order, so few long rows are split over workgroups, whose maxima
+// and non-finite marks (part) k_dd_stats_merge joins.
 constexpr int ST_NT = 512, ST_ROWS = 8, ST_KL = ST_NT / ST_ROWS;
 
-VCPHIP_DEVINL void dd_stats_rows(const double* __restrict__ X, long ldx, int rows, int len, int* __restrict__ e,
-                                 int* __restrict__ flags, int block, double* __restrict__ s_mem) {
+// flags: 1 = zero row, 2 = a non-finite element
+VCPHIP_DEVINL void dd_stats_row(int* __restrict__ e, int* __restrict__ flags, int r, double mu, int nonfinite) {
+  e[r] = (nonfinite || !(mu > 0.0)) ? 0 : vcphip_fexp(mu);
+  flags[r] = nonfinite ? 2 : (mu > 0.0 ? 0 : 1);
+}
+
+VCPHIP_DEVINL void dd_stats_rows(const double* __restrict__ X, long ldx, int rows, int k0, int len, int* __restrict__ e,
+                                 int* __restrict__ flags, int block, double* __restrict__ s_mem,
+                                 double* __restrict__ part, int split, int nsplit) {
   constexpr int PT = 8;
   const int tid = threadIdx.x, lr = tid % ST_ROWS, lk = tid / ST_ROWS;
   const int r = block * ST_ROWS + lr;
   const double* x = X + 2 * (long)(r < rows ? r : rows - 1);
   double mu = 0.0;
   int nonfinite = 0;
-  for (int k0 = 0; k0 < len; k0 += ST_KL * PT) {
+  for (; k0 < len; k0 += ST_KL * PT) {
     double2 v[PT];
 #pragma unroll
     for (int q = 0; q < PT; ++q) {
@@ -67,9 +75,12 @@ VCPHIP_DEVINL void dd_stats_rows(const double* __restrict__ X, long ldx, int row
     mu = o > mu ? o : mu;
     nonfinite |= s_mem[64 + w * ST_ROWS + tid] != 0.0;
   }
-  // flags: 1 = zero row, 2 = a non-finite element
-  e[r] = (nonfinite || !(mu > 0.0)) ? 0 : vcphip_fexp(mu);
-  flags[r] = nonfinite ? 2 : (mu > 0.0 ? 0 : 1);
+  if (part) {
+    part[(long)split * rows + r] = mu;
+    part[(long)(nsplit + split) * rows + r] = nonfinite ? 1.0 : 0.0;
+    return;
+  }
+  dd_stats_row(e, flags, r, mu, nonfinite);
 }
 
 // the same statistics for lines whose elements are contiguous (columns of B,
@@ -110,18 +121,40 @@ VCPHIP_DEVINL void dd_stats_lines(const double* __restrict__ X, long rs, int row
   }
 }
 
-// both operands in one launch: blocks [0, na) A (its rows, or its columns of a
-// transposed A: a_lines), the rest the columns of B.  Against three launches
-// (chunk maxima, their merge, columns): 600 19 -> 7 us, 4096 136 -> 109 us.
+// both operands in one launch: blocks [0, na nsplit) A (its rows, or its columns
+// of a transposed A: a_lines, never split), the rest the columns of B.  Against
+// three launches (chunk maxima, their merge, columns): 600 19 -> 7 us, 4096
+// 136 -> 109 us.
 __global__ __launch_bounds__(ST_NT) void k_dd_stats(const double* __restrict__ A, long lda, int m, int a_lines, int na,
                                                   int* __restrict__ ea, int* __restrict__ fa,
                                                   const double* __restrict__ B, long ldb, int n, int* __restrict__ eb,
-                                                  int* __restrict__ fb, int k) {
+                                                  int* __restrict__ fb, int k, double* __restrict__ part, int nsplit,
+                                                  int kper) {
   vcphip_mode_round_up();
   __shared__ double s_mem[128];
-  if ((int)blockIdx.x >= na) dd_stats_lines(B, ldb, n, k, eb, fb, blockIdx.x - na);
-  else if (a_lines) dd_stats_lines(A, lda, m, k, ea, fa, blockIdx.x);
-  else dd_stats_rows(A, lda, m, k, ea, fa, blockIdx.x, s_mem);
+  if ((int)blockIdx.x >= na * nsplit) {
+    dd_stats_lines(B, ldb, n, k, eb, fb, blockIdx.x - na * nsplit);
+  } else if (a_lines) {
+    dd_stats_lines(A, lda, m, k, ea, fa, blockIdx.x);
+  } else {
+    const int split = blockIdx.x / na, k0 = split * kper, left = k - k0;
+    dd_stats_rows(A, lda, m, k0, k0 + (left < kper ? left : kper), ea, fa, blockIdx.x - split * na, s_mem,
+                  nsplit > 1 ? part : nullptr, split, nsplit);
+  }
+}
+
+__global__ __launch_bounds__(64) void k_dd_stats_merge(int rows, int nsplit, const double* __restrict__ part,
+                                                       int* __restrict__ e, int* __restrict__ flags) {
+  const int r = blockIdx.x * 64 + threadIdx.x;
+  if (r >= rows) return;
+  double mu = 0.0, nf = 0.0;
+#pragma unroll 8
+  for (int q = 0; q < nsplit; ++q) {
+    const double v = part[(long)q * rows + r], f = part[(long)(nsplit + q) * rows + r];
+    mu = v > mu ? v : mu;
+    nf = f > nf ? f : nf;
+  }
+  dd_stats_row(e, flags, r, mu, nf != 0.0);
 }
 
 // ---------------------------------------------------------------------------
@@ -769,11 +802,16 @@ int vcphip_dd_add_d(int m, int n, const double* d, double* X, long ldx, double* 
 
 // A == nullptr: B alone (A^T A)
 int vcphip_dd_stats(const double* A, long lda, int m, int a_lines, int* ea, int* fa, const double* B, long ldb, int n,
-                    int* eb, int* fb, int k, hipStream_t s) {
+                    int* eb, int* fb, int k, int cus, void* scratch, hipStream_t s) {
   const int W = ST_NT / 64;
   const int na = !A ? 0 : a_lines ? (m + W - 1) / W : (m + ST_ROWS - 1) / ST_ROWS, nb = (n + W - 1) / W;
   if (na + nb <= 0) return 0;
-  hipLaunchKernelGGL(k_dd_stats, dim3(na + nb), dim3(ST_NT), 0, s, A, lda, m, a_lines, na, ea, fa, B, ldb, n, eb, fb, k);
+  int nsplit, kper;
+  vcphip_stats_split(a_lines ? 0 : na, k, cus, nsplit, kper);
+  double* part = (double*)scratch;
+  hipLaunchKernelGGL(k_dd_stats, dim3(na * nsplit + nb), dim3(ST_NT), 0, s, A, lda, m, a_lines, na, ea, fa, B, ldb, n,
+                     eb, fb, k, part, nsplit, kper);
+  if (nsplit > 1) hipLaunchKernelGGL(k_dd_stats_merge, dim3((m + 63) / 64), dim3(64), 0, s, m, nsplit, part, ea, fa);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 

@@ -48,15 +48,27 @@ constexpr int ST_ROWS = 8;                  // its rows of A: 128-byte runs of a
 constexpr int ST_KL = ST_NT / ST_ROWS;      // k in flight per load of each thread
 constexpr int ST_CG = 2;                    // chunks whose 1-norms are summed together
 
-// rows of A (m x k, column-major): a workgroup takes 8 rows over the whole of
-// k.  The maxima are taken by every thread over its own elements; the upward
-// 1-norm is the sequential upward sum of each 256-k chunk (8 lanes per chunk,
-// two chunks at a time, over the magnitudes in LDS, while the next chunk's
-// loads are in flight) and then of the chunk sums in order.  One read of A, no partial results in
-// memory and no second launch (a thread per row and chunk, then a merging
-// launch: 28 + 5 us at 500 x 500, 215 + 16 us at 8192 x 8192).
-VCPHIP_DEVINL void oz_stats_rows(const double* __restrict__ X, long ldx, int rows, int len, const VcphipOzSide& side,
-                                 int block, double* __restrict__ s_mem) {
+// rows of A (m x k, column-major): a workgroup takes 8 rows over k0 .. k1.  The
+// maxima are taken by every thread over its own elements; the upward 1-norm is
+// the sequential upward sum of each 256-k chunk (8 lanes per chunk, two chunks
+// at a time, over the magnitudes in LDS, while the next chunk's loads are in
+// flight) and then of the chunk sums in order.  Over the whole of k that is one
+// read of A, no partial results in memory and no second launch (a thread per
+// row and chunk, then a merging launch: 28 + 5 us at 500 x 500, 215 + 16 us at
+// 8192 x 8192).  A workgroup's 512 k take about 4.4 us, so few long rows are
+// split over workgroups: each leaves its chunk sums and its maxima in `part`
+// (one of nsplit), and k_oz_stats_merge adds and compares them.
+VCPHIP_DEVINL void oz_stats_row(const VcphipOzSide& side, int r, double mu, double smax, double rmax, int nf, double n1) {
+  side.flags[r] = side_flags(mu, smax, rmax, nf);
+  side.e[r] = (!nf && mu > 0.0) ? vcphip_fexp(mu) : 0;
+  side.g[r] = (!nf && smax > 0.0) ? vcphip_fexp(smax) : 0;
+  side.h[r] = (!nf && rmax > 0.0) ? vcphip_fexp(rmax) : 0;
+  side.n1[r] = nf ? 0.0 : n1;
+}
+
+VCPHIP_DEVINL void oz_stats_rows(const double* __restrict__ X, long ldx, int rows, int k0, int len,
+                                 const VcphipOzSide& side, int block, double* __restrict__ s_mem,
+                                 double* __restrict__ part, long nchunk, int split, int nsplit) {
   constexpr int PT = VCPHIP_OZ_CHUNK / ST_KL;   // elements of a chunk per thread
   const int tid = threadIdx.x, lr = tid % ST_ROWS, lk = tid / ST_ROWS;
   const int r = block * ST_ROWS + lr;
@@ -72,8 +84,8 @@ VCPHIP_DEVINL void oz_stats_rows(const double* __restrict__ X, long ldx, int row
   };
   double mu = 0.0, smax = 0.0, rmax = 0.0, tot = 0.0;
   int nf = 0;
-  load(0);
-  for (int c0 = 0; c0 < len; c0 += ST_CG * VCPHIP_OZ_CHUNK) {
+  load(k0);
+  for (int c0 = k0; c0 < len; c0 += ST_CG * VCPHIP_OZ_CHUNK) {
 #pragma unroll
     for (int g = 0; g < ST_CG; ++g) {
 #pragma unroll
@@ -109,8 +121,12 @@ VCPHIP_DEVINL void oz_stats_rows(const double* __restrict__ X, long ldx, int row
       }
 #pragma unroll 1
       for (; kk < cnt; ++kk) sum = sum + am[kk * ST_ROWS];
+      if (part) {
+        if (cnt > 0 && r < rows) part[(c0 / VCPHIP_OZ_CHUNK + g) * (long)rows + r] = sum;
+      } else {
 #pragma unroll
-      for (int h = 0; h < ST_CG; ++h) tot = tot + __shfl(sum, h * ST_ROWS + lr, 64);   // an empty chunk adds 0
+        for (int h = 0; h < ST_CG; ++h) tot = tot + __shfl(sum, h * ST_ROWS + lr, 64);   // an empty chunk adds 0
+      }
     }
     __syncthreads();
   }
@@ -136,11 +152,16 @@ VCPHIP_DEVINL void oz_stats_rows(const double* __restrict__ X, long ldx, int row
   smax = s_mem[ST_NT + tid];
   rmax = s_mem[2 * ST_NT + tid];
   nf = (int)s_mem[3 * ST_NT + tid];
-  side.flags[r] = side_flags(mu, smax, rmax, nf);
-  side.e[r] = (!nf && mu > 0.0) ? vcphip_fexp(mu) : 0;
-  side.g[r] = (!nf && smax > 0.0) ? vcphip_fexp(smax) : 0;
-  side.h[r] = (!nf && rmax > 0.0) ? vcphip_fexp(rmax) : 0;
-  side.n1[r] = nf ? 0.0 : tot;
+  if (part) {
+    double* mx = part + nchunk * rows + (long)split * rows + r;
+    const long stride = (long)nsplit * rows;
+    mx[0] = mu;
+    mx[stride] = smax;
+    mx[2 * stride] = rmax;
+    mx[3 * stride] = (double)nf;
+    return;
+  }
+  oz_stats_row(side, r, mu, smax, rmax, nf, tot);
 }
 
 // columns of B (k x n, column k-contiguous): one wave per column.  Lane l
@@ -197,17 +218,52 @@ VCPHIP_DEVINL void oz_stats_cols(const double* __restrict__ X, long ldx, int col
   }
 }
 
-// both operands in one launch: blocks [0, na) the rows of A, the rest the
-// columns of B.  Bound by launches and the load latency of each row group's
+// both operands in one launch: blocks [0, na nsplit) the rows of A, the rest
+// the columns of B.  Bound by launches and the load latency of each row group's
 // serial chunks at small sizes, by HBM at large ones; against three launches:
 // 500 39 -> 10 us, 2000 65 -> 42 us, 8192 420 -> 403 us.
 __global__ __launch_bounds__(ST_NT) void k_oz_stats(const double* __restrict__ A, long lda, int m, VcphipOzSide sa, int na,
                                                   const double* __restrict__ B, long ldb, int n, VcphipOzSide sb,
-                                                  int k) {
+                                                  int k, double* __restrict__ part, int nsplit, int kper) {
   vcphip_mode_round_up();
   __shared__ double s_mem[ST_CG * VCPHIP_OZ_CHUNK * ST_ROWS];
-  if ((int)blockIdx.x < na) oz_stats_rows(A, lda, m, k, sa, blockIdx.x, s_mem);
-  else oz_stats_cols(B, ldb, n, k, sb, blockIdx.x - na, s_mem);
+  if ((int)blockIdx.x < na * nsplit) {
+    const int split = blockIdx.x / na, k0 = split * kper, left = k - k0;
+    oz_stats_rows(A, lda, m, k0, k0 + (left < kper ? left : kper), sa, blockIdx.x - split * na, s_mem,
+                  nsplit > 1 ? part : nullptr, (k + VCPHIP_OZ_CHUNK - 1) / VCPHIP_OZ_CHUNK, split, nsplit);
+  } else {
+    oz_stats_cols(B, ldb, n, k, sb, blockIdx.x - na * nsplit, s_mem);
+  }
+}
+
+// a row's statistics from its chunk sums, in order, and the maxima of its splits
+__global__ __launch_bounds__(64) void k_oz_stats_merge(int rows, int nchunk, int nsplit, const double* __restrict__ part,
+                                                       VcphipOzSide side) {
+  vcphip_mode_round_up();
+  const int r = blockIdx.x * 64 + threadIdx.x;
+  if (r >= rows) return;
+  double tot = 0.0, mx[3] = {0.0, 0.0, 0.0};
+  int nf = 0, c = 0;
+  for (; c + 32 <= nchunk; c += 32) {
+    double v[32];
+#pragma unroll
+    for (int u = 0; u < 32; ++u) v[u] = part[(long)(c + u) * rows + r];
+#pragma unroll
+    for (int u = 0; u < 32; ++u) tot = tot + v[u];
+  }
+  for (; c < nchunk; ++c) tot = tot + part[(long)c * rows + r];
+  const double* p = part + (long)nchunk * rows + r;
+  const long stride = (long)nsplit * rows;
+#pragma unroll 4
+  for (int q = 0; q < nsplit; ++q) {
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const double v = p[j * stride + (long)q * rows];
+      mx[j] = v > mx[j] ? v : mx[j];
+    }
+    nf |= (int)p[3 * stride + (long)q * rows];
+  }
+  oz_stats_row(side, r, mx[0], mx[1], mx[2], nf, tot);
 }
 
 // ---------------------------------------------------------------------------
@@ -1290,10 +1346,17 @@ __global__ __launch_bounds__(256) void k_oz_recon(int m, int n, int k, int mpad,
 // launchers
 // ---------------------------------------------------------------------------
 int vcphip_oz_stats(const double* A, long lda, int m, VcphipOzSide sa, const double* B, long ldb, int n,
-                    VcphipOzSide sb, int k, hipStream_t s) {
+                    VcphipOzSide sb, int k, int cus, void* scratch, hipStream_t s) {
   const int na = (m + ST_ROWS - 1) / ST_ROWS, nb = (n + ST_NT / 64 - 1) / (ST_NT / 64);
   if (na + nb <= 0) return 0;
-  hipLaunchKernelGGL(k_oz_stats, dim3(na + nb), dim3(ST_NT), 0, s, A, lda, m, sa, na, B, ldb, n, sb, k);
+  int nsplit, kper;
+  vcphip_stats_split(na, k, cus, nsplit, kper);
+  double* part = (double*)scratch;
+  hipLaunchKernelGGL(k_oz_stats, dim3(na * nsplit + nb), dim3(ST_NT), 0, s, A, lda, m, sa, na, B, ldb, n, sb, k, part,
+                     nsplit, kper);
+  if (nsplit > 1)
+    hipLaunchKernelGGL(k_oz_stats_merge, dim3((m + 63) / 64), dim3(64), 0, s, m,
+                       (k + VCPHIP_OZ_CHUNK - 1) / VCPHIP_OZ_CHUNK, nsplit, part, sa);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 

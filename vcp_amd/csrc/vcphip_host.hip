@@ -801,7 +801,7 @@ static int oz_run(vcphip_ctx* c, const OzPlan& p, int m, int n, int k, const dou
   const int mpad = p.tile.mpad, npad = p.tile.npad, kpad = p.kpad;
   int rc;
   StageTimer T(c, timed);
-  if ((rc = check_launch(vcphip_oz_stats(A, lda, m, SA, B, ldb, n, SB, k, c->stream)))) return rc;
+  if ((rc = check_launch(vcphip_oz_stats(A, lda, m, SA, B, ldb, n, SB, k, c->num_cu, pa, c->stream)))) return rc;
   T.mark("stats");
   if ((rc = check_launch(vcphip_oz_split(A, lda, m, mpad, SA, (int8_t*)pa, B, ldb, n, npad, SB, (int8_t*)pb, k, kpad, p.P,
                                          c->stream))))
@@ -1116,7 +1116,8 @@ static int dd_gemm_dev(vcphip_ctx* c, bool tn, int m, int n, int k, const double
   int* fb = eb + n;
   StageTimer T(c);
   const double* Aop = tn ? nullptr : A;   // A^T A: the columns of B = A serve both sides
-  if ((rc = check_launch(vcphip_dd_stats(Aop, lda, m, ta ? 1 : 0, ea, fa, B, ldb, n, eb, fb, k, c->stream)))) return rc;
+  if ((rc = check_launch(vcphip_dd_stats(Aop, lda, m, ta ? 1 : 0, ea, fa, B, ldb, n, eb, fb, k, c->num_cu, pa, c->stream))))
+    return rc;
   T.mark("stats");
   if ((rc = check_launch(vcphip_dd_split(Aop, lda, m, mpad, ta ? 1 : 0, ea, fa, (int8_t*)pa, B, ldb, n, npad, eb, fb,
                                          (int8_t*)pb, k, kpad, P, c->stream))))

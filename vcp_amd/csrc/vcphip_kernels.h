@@ -172,9 +172,29 @@ struct VcphipOzSide {
   double* n1;   // upward 1-norm of |mid|
 };
 
-// statistics of the rows of A (m x k) and the columns of B (k x n), one launch
+// How the statistics of m = 8 na rows are split over k: nsplit workgroups of
+// kper k (a multiple of 512) for every 8 rows.  A workgroup takes about 4.4 us
+// (interval) or 4.1 us (dd) for 512 k, and a split costs a merging launch, so
+// k is split where the row blocks are at most one per CU and k spans at least
+// six of those steps, into about two workgroups per CU.  Statistics of both
+// operands, one workgroup against split (interval / dd): 100 x 100 x 65000 591
+// against 229 us / 531 against 185, 512 x 512 x 30000 280 against 156 / 266
+// against 132, 200 x 200 x 8192 72 against 30 / 50 against 21.
+inline void vcphip_stats_split(int na, int k, int cus, int& nsplit, int& kper) {
+  const int steps = k / 512 + (k % 512 != 0);
+  nsplit = 1;
+  kper = k;
+  if (na <= 0 || na > cus || steps < 6) return;
+  const int want = 2 * cus / na, per = steps <= want ? 1 : (steps + want - 1) / want;
+  nsplit = (steps + per - 1) / per;
+  kper = per * 512;
+}
+
+// statistics of the rows of A (m x k) and the columns of B (k x n).  scratch:
+// m (k / 256 + 1 + 4 nsplit) doubles for rows split over k (the planes of A,
+// which are written afterwards, hold that many)
 int vcphip_oz_stats(const double* A, long lda, int m, VcphipOzSide sa, const double* B, long ldb, int n,
-                    VcphipOzSide sb, int k, hipStream_t s);
+                    VcphipOzSide sb, int k, int cus, void* scratch, hipStream_t s);
 // planes of both operands, one launch: N residue planes followed by the
 // radius-digit planes (VCPHIP_OZ_NDIGIT_A for A, _B for B), each
 // [rows_pad][kpad] int8 with k contiguous
@@ -193,9 +213,10 @@ int vcphip_oz_recon(int m, int n, int k, int mpad, int npad, const VcphipOzParam
 // ---- double-double product, Ozaki scheme II (kern_dd.hip) -------------------
 // rows of A (m x k; its columns if a_lines / a_cols: A^T with A k x m) and
 // columns of B (k x n): e with max |hi|+|lo| < 2^e; flags 1: zero, 2: not
-// finite; then the residue planes, each one launch.  A == nullptr: B alone
+// finite; then the residue planes.  A == nullptr: B alone.  scratch: 2 m nsplit
+// doubles for rows split over k (vcphip_stats_split)
 int vcphip_dd_stats(const double* A, long lda, int m, int a_lines, int* ea, int* fa, const double* B, long ldb, int n,
-                    int* eb, int* fb, int k, hipStream_t s);
+                    int* eb, int* fb, int k, int cus, void* scratch, hipStream_t s);
 int vcphip_dd_split(const double* A, long lda, int m, int mpad, int a_cols, const int* ea, const int* fa, int8_t* pa,
                     const double* B, long ldb, int n, int npad, const int* eb, const int* fb, int8_t* pb, int k,
                     int kpad, const VcphipOzParams& P, hipStream_t s);
