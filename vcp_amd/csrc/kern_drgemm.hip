@@ -406,26 +406,30 @@ struct PointBlock {
                                  int row0, int col0, int m, int n) {
     const int lc = lane & 31, h = lane >> 5, r = lane % R;
     double* l = reinterpret_cast<double*>(L);
-    double x[RPL];   // 32 / NC passes of T
 #pragma unroll
-    for (int q = 0; q < RPL; ++q) {
-      const int c = col0 + q / T * NC + lane / R + 64 / R * (q % T);
-      x[q] = row0 + r < m && c < n ? X[row0 + r + ldx * c] : 0.0;
-    }
+    for (int g = 0; g < 2; ++g) {   // half of the columns' loads in flight
+      double x[RPL / 2];
 #pragma unroll
-    for (int c0 = 0; c0 < 32; c0 += NC) {
-#pragma unroll
-      for (int t = 0; t < T; ++t) l[elem(lane / R + 64 / R * t, r)] = x[c0 / NC * T + t];
-      vcphip_wave_sync();
-      if (lc / NC == c0 / NC) {
-#pragma unroll
-        for (int i = 0; i < RPL; i += 2) {
-          const double2 p = L[pair(lc % NC, (h * RPL + i) / 2)];
-          v[i] = p.x;
-          v[i + 1] = p.y;
-        }
+      for (int q = 0; q < RPL / 2; ++q) {
+        const int c = col0 + 16 * g + q / T * NC + lane / R + 64 / R * (q % T);
+        x[q] = 0.0;
+        if (row0 + r < m && c < n) x[q] = X[row0 + r + ldx * c];
       }
-      vcphip_wave_sync();
+#pragma unroll
+      for (int c0 = 16 * g; c0 < 16 * g + 16; c0 += NC) {
+#pragma unroll
+        for (int t = 0; t < T; ++t) l[elem(lane / R + 64 / R * t, r)] = x[(c0 - 16 * g) / NC * T + t];
+        vcphip_wave_sync();
+        if (lc / NC == c0 / NC) {
+#pragma unroll
+          for (int i = 0; i < RPL; i += 2) {
+            const double2 p = L[pair(lc % NC, (h * RPL + i) / 2)];
+            v[i] = p.x;
+            v[i + 1] = p.y;
+          }
+        }
+        vcphip_wave_sync();
+      }
     }
   }
 };
