@@ -44,11 +44,15 @@ VCPHIP_DEVINL bool sign_definite(double lo, double hi) {
 // once per point instead of per element, a point's operands read during the
 // arithmetic of the one before, and marks per point, so that a point where
 // some operand holds zero does not send its whole stage through the general
-// form.  Against two barriers and a mark per stage (three contexts in turn /
-// one): m = 900 at 3600 points 514 / 770 against 560 / 870 us, 400 at 1600 250
-// against 280, 400 at 1681 (a zero at x = 0 and y = 0) 315 against 360, 3025
-// at 3600 5.57 against 6.26 ms.  Wider thread tiles (4 x 2, 4 x 4) leave the
-// chip short of waves up to m = 1600 (3.3 against 3.0 ms) and tie at 3025.
+// form.  The next stage's loads must be global ones (a zero by address, in place
+// of a value, in the bounds checks made them FLAT, which the arithmetic then
+// waited for: 400 at 1600 points 249 against 232 us, 100 at 400 63 against 58,
+// one context).  Against two barriers and a mark per stage, 64 x 64 tiles from
+// m = 2817 on (three contexts in turn / one): m = 400 at 1600 points 103 / 232
+// against 118 / 276 us, 400 at 1681 109 / 245 against 125 / 292, 900 at 3600
+// 522 / 717 against 570 / 827, 3025 at 3600 5.70 / 5.68 against 5.56 / 6.42 ms.
+// Wider thread tiles (4 x 2, 4 x 4) leave the chip short of waves up to m =
+// 1600 (3.3 against 3.0 ms) and tie at 3025.
 __global__ __launch_bounds__(NT, 2) void k_uhphiphi(int m, int npts, const double* __restrict__ phi, long ldp,
                                                     const double* __restrict__ w, const double* __restrict__ u,
                                                     double* __restrict__ A, long lda) {
@@ -81,13 +85,12 @@ __global__ __launch_bounds__(NT, 2) void k_uhphiphi(int m, int npts, const doubl
   // stage k0 in registers: the global loads of the next stage are issued
   // before the current stage's arithmetic and stored to LDS after it
   double2 ga[NQ], gb[NQ];
-  const double2 zero2 = make_double2(0.0, 0.0);
   auto load_stage = [&](int k0) {
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
       const int e = tid + NT * q, r = e % BM, k = k0 + e / BM;
-      ga[q] = (k < npts && row0 + r < m) ? *reinterpret_cast<const double2*>(phi + 2 * (row0 + r + ldp * k)) : zero2;
-      gb[q] = (k < npts && col0 + r < m) ? *reinterpret_cast<const double2*>(phi + 2 * (col0 + r + ldp * k)) : zero2;
+      ga[q] = (k < npts && row0 + r < m) ? *reinterpret_cast<const double2*>(phi + 2 * (row0 + r + ldp * k)) : make_double2(0.0, 0.0);
+      gb[q] = (k < npts && col0 + r < m) ? *reinterpret_cast<const double2*>(phi + 2 * (col0 + r + ldp * k)) : make_double2(0.0, 0.0);
     }
   };
   auto store_v = [&](int k0, int st) {

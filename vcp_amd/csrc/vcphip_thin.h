@@ -12,9 +12,12 @@
 // B into LDS, one stage ahead of the chains and with the next stage's loads in
 // flight; the chain waves carry the chains: lane = row (8) x column lane (8),
 // CPT columns per lane.  Loading by separate waves keeps conversions and
-// global waits out of the chains' way.  m = 4000 rows give 500 workgroups, two
-// per CU; consecutive row blocks run on one XCD, so that cache lines that
-// straddle two row blocks are fetched once per L2.
+// global waits out of the chains' way.  (The batched forms take their pointers
+// from descriptors in memory.  Their loads are then FLAT ones, which count as
+// LDS operations too: the next barrier waits for them, so a stage lasts at
+// least as long as the loads issued in it.)  m = 4000 rows give 500
+// workgroups, two per CU; consecutive row blocks run on one XCD, so that cache
+// lines that straddle two row blocks are fetched once per L2.
 //
 // The operation is a policy Op:
 //   A2, B2      global elements of A / B are pairs (else doubles)
