@@ -15,7 +15,10 @@
 //
 // Each block of multiply-adds is one asm statement: the factors' last VALU
 // writes and the first DPP read of them need two wait states, which the
-// leading s_nop gives whatever the compiler put before it.
+// leading s_nop gives whatever the compiler put before it.  The statement
+// writes accumulators before it has read its last factor, so they are early
+// clobbers: without that an accumulator whose value equals a factor's may share
+// its registers.
 #pragma once
 
 #include "vcphip_device.h"
@@ -31,7 +34,7 @@
   VCPHIP_DPP_1(acc, 8, a, b) VCPHIP_DPP_1(acc, 9, a, b) VCPHIP_DPP_1(acc, 10, a, b)                     \
   VCPHIP_DPP_1(acc, 11, a, b) VCPHIP_DPP_1(acc, 12, a, b) VCPHIP_DPP_1(acc, 13, a, b)                   \
   VCPHIP_DPP_1(acc, 14, a, b) VCPHIP_DPP_1(acc, 15, a, b)
-#define VCPHIP_DPP_O1(acc, i) [acc##i] "+v"(acc[i])
+#define VCPHIP_DPP_O1(acc, i) [acc##i] "+&v"(acc[i])
 #define VCPHIP_DPP_O8(acc)                                                                              \
   VCPHIP_DPP_O1(acc, 0), VCPHIP_DPP_O1(acc, 1), VCPHIP_DPP_O1(acc, 2), VCPHIP_DPP_O1(acc, 3),           \
       VCPHIP_DPP_O1(acc, 4), VCPHIP_DPP_O1(acc, 5), VCPHIP_DPP_O1(acc, 6), VCPHIP_DPP_O1(acc, 7)
