@@ -1,6 +1,6 @@
 // Plain FP64 directed-rounding GEMM family (vector FMA, LDS-tiled, gfx950).
 //
-// One kernel template covers the four products of the pidblas policy:
+// The four products of the pidblas policy:
 //   II  C = IA*IB        pidblas::mulmm     vcp/pidblas.hpp:239-294
 //   IP  C = IA*B         pidblas::mul_im_m  vcp/pidblas.hpp:90-140
 //   PI  C = B*IA         pidblas::mul_m_im  vcp/pidblas.hpp:142-196
@@ -16,11 +16,11 @@
 //   t = RU(r1 + r2); upper = RU(up + t); lower = RD(-dn - t) = -RU(dn + t).
 // Three implementations share these chains: k_drgemm_planes (the single
 // products), fed from midpoint-radius planes made once per operand; the tile
-// function dr_tile (the batched launches, and k = 0), which reads the AoS
-// {inf, sup} operands and converts them to midpoint-radius on their way into
-// LDS (pidblas_assist::midrad, :43-60); and the row-serial k_drgemm_thin for
-// few columns and small sizes (vcphip_thin.h).  The two tiled ones carry them
-// as DPP multiply-adds (vcphip_dpp.h).
+// function dr_tile (the batched launches), which reads the AoS {inf, sup}
+// operands and converts them to midpoint-radius on their way into LDS
+// (pidblas_assist::midrad, :43-60); and the row-serial k_drgemm_thin for few
+// columns and small sizes (vcphip_thin.h).  The two tiled ones carry them as
+// DPP multiply-adds (vcphip_dpp.h).  A single product of k = 0 is a fill.
 //
 // The whole kernel runs in round-toward-+inf (see vcphip_device.h).
 #include "vcphip_device.h"
@@ -32,8 +32,8 @@ namespace {
 
 constexpr int BM = 64, BN = 64, BK = 16;
 constexpr int NT = 256;          // 4 waves
-// the k = 0 syrk and the inf-sup tiles: thread (tx, ty) of 16 x 16 holds rows
-// 4 ty .. 4 ty + 3 and columns tx + 16 j
+// the inf-sup tiles: thread (tx, ty) of 16 x 16 holds rows 4 ty .. 4 ty + 3 and
+// columns tx + 16 j
 constexpr int TM = 4, TN = 4;
 constexpr int PAD = 2;           // doubles of row padding (keeps 16-byte alignment)
 constexpr int LA = BM + PAD;     // LDS row length of an A k-slice
@@ -73,7 +73,8 @@ constexpr long DR_LDMAX = VCPHIP_TILE_LDMAX;
 template <bool AI, bool BI, bool RESID, int TMR = 4, bool BIG = false, class Lds = DrLds<AI, BI>>
 __device__ __forceinline__ void dr_tile(Lds& L, int m, int n, int k, const double* __restrict__ A,
                                         long lda, const double* __restrict__ B, long ldb, double* __restrict__ C,
-                                        long ldc, double* __restrict__ C2, int accumulate, int row0, int col0) {
+                                        long ldc, int row0, int col0) {
+  static_assert(AI || BI, "an interval product");
   constexpr bool II = AI && BI;
   constexpr int RPL = 4 * TMR, TBM = 4 * RPL;   // rows per lane, tile rows
   constexpr int BKT = Lds::BKT, AE = Lds::AE, BE = Lds::BE, LDR = Lds::LDR;
@@ -166,16 +167,6 @@ __device__ __forceinline__ void dr_tile(Lds& L, int m, int n, int k, const doubl
     r2[i] = 0.0;
   }
 
-  if (!AI && !BI && accumulate) {
-    // udmatmul form: the chains continue from the values already in CU / CD
-#pragma unroll
-    for (int i = 0; i < RPL; ++i)
-      if (orow + i < m && ocol < n) {
-        up[i] = C[orow + i + ldc * ocol];
-        dn[i] = -C2[orow + i + ldc * ocol];
-      }
-  }
-
   // slices up to k rounded up to 16 (as the planes pad)
   const int nt = (k + 15) / 16 * 16 / BKT;
   if (nt > 0) {
@@ -206,33 +197,32 @@ __device__ __forceinline__ void dr_tile(Lds& L, int m, int n, int k, const doubl
   for (int i = 0; i < RPL; ++i) {
     const int r = orow + i;
     if (r >= m) break;
-    if (AI || BI) {
-      const double t = II ? r1[i] + r2[i] : r1[i];   // temp = (|mA|+rA) rB + rA |mB|   (:283)
-      double hi = up[i] + t;                         // uC += temp, RU                  (:284)
-      double nlo = dn[i] + t;                        // lC -= temp, RD = -(RU(-lC + t)) (:285-286)
-      if (RESID && r == ocol) {                      // b(i,i) -= 1 in interval arithmetic
-        hi = hi - 1.0;
-        nlo = nlo + 1.0;
-      }
-      *reinterpret_cast<double2*>(C + 2 * (r + ldc * ocol)) = make_double2(-nlo, hi);
-    } else {
-      C[r + ldc * ocol] = up[i];
-      C2[r + ldc * ocol] = -dn[i];
+    const double t = II ? r1[i] + r2[i] : r1[i];   // temp = (|mA|+rA) rB + rA |mB|   (:283)
+    double hi = up[i] + t;                         // uC += temp, RU                  (:284)
+    double nlo = dn[i] + t;                        // lC -= temp, RD = -(RU(-lC + t)) (:285-286)
+    if (RESID && r == ocol) {                      // b(i,i) -= 1 in interval arithmetic
+      hi = hi - 1.0;
+      nlo = nlo + 1.0;
     }
+    *reinterpret_cast<double2*>(C + 2 * (r + ldc * ocol)) = make_double2(-nlo, hi);
   }
 }
 
-template <bool AI, bool BI>
-__global__ __launch_bounds__(NT, 2) void k_drgemm(int m, int n, int k, const double* __restrict__ A, long lda,
-                                                   const double* __restrict__ B, long ldb, double* __restrict__ C,
-                                                   long ldc, double* __restrict__ C2, int accumulate) {
-  vcphip_mode_round_up();
-  const int ntm = (m + BM - 1) / BM, ntn = (n + BN - 1) / BN;
-  const int tile = vcphip_xcd_remap(blockIdx.x, ntm * ntn);
-  int tm, tn;
-  vcphip_tile_coords(tile, ntm, ntn, 16, tm, tn);
-  __shared__ __attribute__((aligned(16))) DrLds<AI, BI> lds;
-  dr_tile<AI, BI, false, 4, true>(lds, m, n, k, A, lda, B, ldb, C, ldc, C2, accumulate, tm * BM, tn * BN);
+// The products of k = 0: every chain is 0, so the round-up and round-down
+// results are +0 and -0 (an interval's ends: {-0, +0}).  C2 null: C holds
+// intervals.
+__global__ __launch_bounds__(NT) void k_empty_product(int m, int n, double* __restrict__ C, long ldc,
+                                                      double* __restrict__ C2) {
+  const int r = blockIdx.x * NT + threadIdx.x;
+  if (r >= m) return;
+  for (long c = blockIdx.y; c < n; c += gridDim.y) {
+    if (C2) {
+      C[r + ldc * c] = 0.0;
+      C2[r + ldc * c] = -0.0;
+    } else {
+      *reinterpret_cast<double2*>(C + 2 * (r + ldc * c)) = make_double2(-0.0, 0.0);
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -557,18 +547,17 @@ __global__ __launch_bounds__(NT, BIG ? 2 : 3) void k_resid_tiles(int ntiles, con
   for (int t = next_tile(queue, slot); t < ntiles; t = next_tile(queue, slot)) {
     const VcphipResidTile tl = tiles[t];
     const VcphipResidProblem p = probs[tl.problem];
-    dr_tile<false, true, true, TMR, BIG>(lds, p.n, p.n, p.n, p.R, p.ldr, p.A, p.lda, p.C, p.ldc, nullptr, 0, tl.row0,
-                                    tl.col0);
+    dr_tile<false, true, true, TMR, BIG>(lds, p.n, p.n, p.n, p.R, p.ldr, p.A, p.lda, p.C, p.ldc, tl.row0, tl.col0);
   }
 }
 
 // Many interval products C_p = IA_p * IB_p of uneven (m, n, k) in one
 // persistent launch per tile shape (pidblas::mulmm, vcp/pidblas.hpp:239-294,
 // per problem): workgroups take the tiles of a list sorted by problem size
-// from a work queue, each tile the interval x interval form of k_drgemm, so
+// from a work queue, each tile the interval x interval form above, so
 // every C_p is bit-identical to the single product's.
 template <int TMR, bool BIG>
-__global__ __launch_bounds__(NT, BIG ? 2 : 2) void k_igemm_tiles(int ntiles, const VcphipResidTile* __restrict__ tiles,
+__global__ __launch_bounds__(NT, 2) void k_igemm_tiles(int ntiles, const VcphipResidTile* __restrict__ tiles,
                                                         const VcphipIgemmProblem* __restrict__ probs,
                                                         unsigned* __restrict__ queue) {
   vcphip_mode_round_up();
@@ -577,8 +566,7 @@ __global__ __launch_bounds__(NT, BIG ? 2 : 2) void k_igemm_tiles(int ntiles, con
   for (int t = next_tile(queue, slot); t < ntiles; t = next_tile(queue, slot)) {
     const VcphipResidTile tl = tiles[t];
     const VcphipIgemmProblem p = probs[tl.problem];
-    dr_tile<true, true, false, TMR, BIG>(lds, p.m, p.n, p.k, p.A, p.lda, p.B, p.ldb, p.C, p.ldc, nullptr, 0, tl.row0,
-                                    tl.col0);
+    dr_tile<true, true, false, TMR, BIG>(lds, p.m, p.n, p.k, p.A, p.lda, p.B, p.ldb, p.C, p.ldc, tl.row0, tl.col0);
   }
 }
 
@@ -704,130 +692,10 @@ __global__ __launch_bounds__(256) void k_resid_max(int count, const VcphipResidP
 //   point (pidblas::vmulmm, :198-236): upper = RU chain, lower = RD chain.
 // Element (i, j), i <= j, is written to (i, j) and (j, i).
 // ---------------------------------------------------------------------------
-template <bool INTV>
-__global__ __launch_bounds__(NT, 2) void k_drsyrk(int k, int n, const double* __restrict__ A, long lda,
-                                                  double* __restrict__ C, long ldc) {
-  vcphip_mode_round_up();
-  __shared__ __attribute__((aligned(16))) double sIm[BK][LA];
-  __shared__ __attribute__((aligned(16))) double sIr[INTV ? BK : 1][LA];
-  __shared__ __attribute__((aligned(16))) double sJm[BK][LB];
-  __shared__ __attribute__((aligned(16))) double sJr[INTV ? BK : 1][LB];
-
-  const int tid = threadIdx.x;
-  const int nt = (n + BM - 1) / BM;
-  // decode upper-triangle tile index b -> (tm, tn), tm <= tn, row-major over tm
-  int b = blockIdx.x, tm = 0;
-  while (b >= nt - tm) { b -= nt - tm; ++tm; }
-  const int tn = tm + b;
-  const int i0 = tm * BM, j0 = tn * BN;
-
-  const int l_k = tid % BK, l_c = tid / BK;   // k-contiguous loads, 16 columns per pass
-  double im[A_PER_T], ir[A_PER_T], jm[B_PER_T], jr[B_PER_T];
-  auto load_tile = [&](int k0) {
-#pragma unroll
-    for (int q = 0; q < A_PER_T; ++q) {
-      const int kk = k0 + l_k;
-      const int ci = i0 + l_c + 16 * q, cj = j0 + l_c + 16 * q;
-      if (INTV) {
-        const double2 vi = (kk < k && ci < n) ? *reinterpret_cast<const double2*>(A + 2 * (kk + lda * ci)) : make_double2(0.0, 0.0);
-        const double2 vj = (kk < k && cj < n) ? *reinterpret_cast<const double2*>(A + 2 * (kk + lda * cj)) : make_double2(0.0, 0.0);
-        im[q] = vi.x; ir[q] = vi.y; jm[q] = vj.x; jr[q] = vj.y;
-      } else {
-        im[q] = (kk < k && ci < n) ? A[kk + lda * ci] : 0.0;
-        jm[q] = (kk < k && cj < n) ? A[kk + lda * cj] : 0.0;
-      }
-    }
-  };
-  auto store_tile = [&]() {
-#pragma unroll
-    for (int q = 0; q < A_PER_T; ++q) {
-      if (INTV) {
-        double mm, rr;
-        vcphip_midrad_ru(im[q], ir[q], mm, rr);
-        sIm[l_k][l_c + 16 * q] = mm;
-        sIr[l_k][l_c + 16 * q] = rr;
-        vcphip_midrad_ru(jm[q], jr[q], mm, rr);
-        sJm[l_k][l_c + 16 * q] = mm;
-        sJr[l_k][l_c + 16 * q] = rr;
-      } else {
-        sIm[l_k][l_c + 16 * q] = im[q];
-        sJm[l_k][l_c + 16 * q] = jm[q];
-      }
-    }
-  };
-
-  const int tx = tid % 16, ty = tid / 16;
-  double up[TM][TN], dn[TM][TN], tij[TM][TN], tji[TM][TN], sij[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) { up[i][j] = 0.0; dn[i][j] = 0.0; tij[i][j] = 0.0; tji[i][j] = 0.0; sij[i][j] = 0.0; }
-
-  const int ntiles = (k + BK - 1) / BK;
-  load_tile(0);
-  store_tile();
-  __syncthreads();
-  for (int t = 0; t < ntiles; ++t) {
-    if (t + 1 < ntiles) load_tile((t + 1) * BK);
-#pragma unroll(INTV ? 1 : 2)
-    for (int kk = 0; kk < BK; ++kk) {
-      double a[TM], ar[TM], bb[TN], br[TN];
-      {
-        const double2 x0 = *reinterpret_cast<const double2*>(&sIm[kk][ty * TM]);
-        const double2 x1 = *reinterpret_cast<const double2*>(&sIm[kk][ty * TM + 2]);
-        a[0] = x0.x; a[1] = x0.y; a[2] = x1.x; a[3] = x1.y;
-      }
-      if (INTV) {
-        const double2 x0 = *reinterpret_cast<const double2*>(&sIr[kk][ty * TM]);
-        const double2 x1 = *reinterpret_cast<const double2*>(&sIr[kk][ty * TM + 2]);
-        ar[0] = x0.x; ar[1] = x0.y; ar[2] = x1.x; ar[3] = x1.y;
-      }
-#pragma unroll
-      for (int j = 0; j < TN; ++j) { bb[j] = sJm[kk][tx + 16 * j]; if (INTV) br[j] = sJr[kk][tx + 16 * j]; }
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          up[i][j] = __builtin_fma(a[i], bb[j], up[i][j]);
-          dn[i][j] = __builtin_fma(-a[i], bb[j], dn[i][j]);
-          if (INTV) {
-            tij[i][j] = __builtin_fma(__builtin_fabs(a[i]), br[j], tij[i][j]);
-            tji[i][j] = __builtin_fma(__builtin_fabs(bb[j]), ar[i], tji[i][j]);
-            sij[i][j] = __builtin_fma(ar[i], br[j], sij[i][j]);
-          }
-        }
-    }
-    __syncthreads();
-    if (t + 1 < ntiles) {
-      store_tile();
-      __syncthreads();
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int r = i0 + ty * TM + i, c = j0 + tx + 16 * j;
-      if (r >= n || c >= n || r > c) continue;
-      double lo, hi;
-      if (INTV) {
-        const double T = tij[i][j] + (tji[i][j] + sij[i][j]);
-        hi = up[i][j] + T;
-        lo = -(dn[i][j] + T);
-      } else {
-        hi = up[i][j];
-        lo = -dn[i][j];
-      }
-      *reinterpret_cast<double2*>(C + 2 * (r + ldc * c)) = make_double2(lo, hi);
-      *reinterpret_cast<double2*>(C + 2 * (c + ldc * r)) = make_double2(lo, hi);
-    }
-}
-
-// The same A^T A forms from the planes of A (k x n) made by k_planes's B part:
-// (mid, rad) pairs (or A), kpad x npad, columns contiguous, zero-padded.
-// Column i of A is then the contiguous run at i of every k-row, so one plane
-// set feeds both operands.  Tiles of 4 RPL rows x 64 columns that meet the
-// upper triangle; the chains and their order are k_drsyrk's.
+// From the planes of A (k x n) made by k_planes's B part: (mid, rad) pairs (or
+// A), kpad x npad, columns contiguous, zero-padded.  Column i of A is then the
+// contiguous run at i of every k-row, so one plane set feeds both operands.
+// Tiles of 4 RPL rows x 64 columns that meet the upper triangle.
 template <bool INTV, int RPL>
 __global__ __launch_bounds__(NT, RPL == 16 ? (INTV ? 2 : 4) : 4) void k_drsyrk_planes(int n, int npad, int kpad,
                                                                                       const double* __restrict__ P,
@@ -1080,25 +948,17 @@ int vcphip_launch_isgemm(int m, int n, int k, const double* A, long lda, const d
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
-int vcphip_launch_drgemm(int kind, int m, int n, int k, const double* A, long lda, const double* B,
-                         long ldb, double* C, long ldc, double* C2, int accumulate, hipStream_t s) {
+int vcphip_launch_empty_product(int m, int n, double* C, long ldc, double* C2, hipStream_t s) {
   if (m <= 0 || n <= 0) return 0;
-  const int ntiles = ((m + BM - 1) / BM) * ((n + BN - 1) / BN);
-  dim3 grid(ntiles), block(NT);
-  switch (kind) {
-    case VCPHIP_DR_II: hipLaunchKernelGGL((k_drgemm<true, true>), grid, block, 0, s, m, n, k, A, lda, B, ldb, C, ldc, C2, accumulate); break;
-    case VCPHIP_DR_IP: hipLaunchKernelGGL((k_drgemm<true, false>), grid, block, 0, s, m, n, k, A, lda, B, ldb, C, ldc, C2, accumulate); break;
-    case VCPHIP_DR_PI: hipLaunchKernelGGL((k_drgemm<false, true>), grid, block, 0, s, m, n, k, A, lda, B, ldb, C, ldc, C2, accumulate); break;
-    case VCPHIP_DR_PP: hipLaunchKernelGGL((k_drgemm<false, false>), grid, block, 0, s, m, n, k, A, lda, B, ldb, C, ldc, C2, accumulate); break;
-    default: return -1;
-  }
+  const dim3 grid((unsigned)((m + NT - 1) / NT), (unsigned)(n < 65535 ? n : 65535));
+  hipLaunchKernelGGL(k_empty_product, grid, dim3(NT), 0, s, m, n, C, ldc, C2);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
 int vcphip_launch_drgemm_thin(int kind, int m, int n, int k, const double* A, long lda, const double* B, long ldb,
                               double* C, long ldc, double* C2, int accumulate, hipStream_t s) {
   if (m <= 0 || n <= 0) return 0;
-  if (k <= 0) return -1;   // k = 0 takes the tile path
+  if (k <= 0) return -1;   // k = 0 is a fill
   // columns of a workgroup: few right-hand sides take the narrow shapes; else
   // the widest (64, the fewest LDS reads per multiply-add) that still gives
   // about 150 workgroups (n = k = m = 300: 19 us with 64, 24 with 32, 30 with
@@ -1158,7 +1018,7 @@ int vcphip_launch_drgemm_planes(int kind, int m, int n, int k, const double* PA,
                                 double* C2, int accumulate, int rows, hipStream_t s) {
   const int mpad = (m + BM - 1) / BM * BM, npad = (n + BN - 1) / BN * BN, kpad = (k + BK - 1) / BK * BK;
   if (m <= 0 || n <= 0) return 0;
-  if (kpad == 0 || (rows != 64 && rows != 32)) return -1;   // k = 0 takes the tile path
+  if (kpad == 0 || (rows != 64 && rows != 32)) return -1;   // k = 0 is a fill
   const dim3 grid((mpad / rows) * (npad / BN)), block(NT);
 #define VCPHIP_PLANES_CASE(KIND, AI, BI)                                                                            \
   case KIND:                                                                                                        \
@@ -1184,7 +1044,7 @@ int vcphip_launch_drsyrk_planes(int interval, int k, int n, const double* A, lon
                                 int rows, hipStream_t s) {
   if (n <= 0) return 0;
   const int npad = (n + BN - 1) / BN * BN, kpad = (k + BK - 1) / BK * BK;
-  if (kpad == 0 || (rows != 64 && rows != 32)) return -1;   // k = 0 takes the tile path
+  if (kpad == 0 || (rows != 64 && rows != 32)) return -1;   // k = 0 is a fill
   const size_t nb = (size_t)((kpad + 31) / 32) * (npad / 32);
   if (nb > 0x7FFFFFFFu) return -7;
   const dim3 gb((unsigned)nb);
@@ -1199,16 +1059,6 @@ int vcphip_launch_drsyrk_planes(int interval, int k, int n, const double* A, lon
     if (rows == 64) hipLaunchKernelGGL((k_drsyrk_planes<false, 16>), grid, dim3(NT), 0, s, n, npad, kpad, P, C, ldc);
     else hipLaunchKernelGGL((k_drsyrk_planes<false, 8>), grid, dim3(NT), 0, s, n, npad, kpad, P, C, ldc);
   }
-  return hipGetLastError() == hipSuccess ? 0 : -3;
-}
-
-int vcphip_launch_drsyrk(int interval, int k, int n, const double* A, long lda, double* C, long ldc,
-                         hipStream_t s) {
-  if (n <= 0) return 0;
-  const int nt = (n + BM - 1) / BM;
-  dim3 grid(nt * (nt + 1) / 2), block(NT);
-  if (interval) hipLaunchKernelGGL((k_drsyrk<true>), grid, block, 0, s, k, n, A, lda, C, ldc);
-  else hipLaunchKernelGGL((k_drsyrk<false>), grid, block, 0, s, k, n, A, lda, C, ldc);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 

@@ -150,7 +150,7 @@ inline dim3 grid_of(long count) { return dim3((unsigned)((count + NT - 1) / NT))
 
 // ===========================================================================
 // The steps of one system (P), as row-serial products: the chains and
-// epilogues are those of the k_drgemm tiles (k ascending, midrad on load, the
+// epilogues are those of the product tiles (k ascending, midrad on load, the
 // same fused operations in the same order), so the single and the batched
 // form give the same bits.
 // ===========================================================================

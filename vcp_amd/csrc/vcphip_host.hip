@@ -965,16 +965,15 @@ struct Extent {
 
 // A single product of kind VCPHIP_DR_*: the operand planes (midpoint and
 // radius of an interval operand, the point operand itself), padded and laid
-// out for whole k-slices, then the product from them.  k = 0 (an all-zero or,
-// accumulating, unchanged product) takes the tile kernel.  The planes are
+// out for whole k-slices, then the product from them.  k = 0 fills in zeros or,
+// accumulating, leaves the results as they are.  The planes are
 // copies, so a result may lie over an operand (A <- A B, X <- R X); the
 // row-serial form reads the operands while it stores, and is not taken then.
 int planes_product(vcphip_ctx* c, int kind, int m, int n, int k, const double* A, int lda, const double* B, int ldb,
                    double* C, int ldc, double* C2 = nullptr, int accumulate = 0) {
   StageTimer T(c);
   if (k == 0) {
-    const int rc =
-        check_launch(vcphip_launch_drgemm(kind, m, n, k, A, lda, B, ldb, C, ldc, C2, accumulate, c->stream));
+    const int rc = accumulate ? VCPHIP_OK : check_launch(vcphip_launch_empty_product(m, n, C, ldc, C2, c->stream));
     T.mark("drgemm");
     return rc;
   }
@@ -1009,7 +1008,7 @@ int planes_product(vcphip_ctx* c, int kind, int m, int n, int k, const double* A
 int syrk_planes(vcphip_ctx* c, int interval, int k, int n, const double* A, int lda, double* C, int ldc) {
   StageTimer T(c);
   if (k == 0) {
-    const int rc = check_launch(vcphip_launch_drsyrk(interval, k, n, A, lda, C, ldc, c->stream));
+    const int rc = check_launch(vcphip_launch_empty_product(n, n, C, ldc, nullptr, c->stream));
     T.mark("drsyrk");
     return rc;
   }

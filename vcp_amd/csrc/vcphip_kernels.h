@@ -29,11 +29,8 @@ int vcphip_launch_drgemm_thin(int kind, int m, int n, int k, const double* A, lo
 // kpad x npad pairs or doubles); k > 0, tiles of `rows` (64 or 32) x 64
 int vcphip_launch_drsyrk_planes(int interval, int k, int n, const double* A, long lda, double* P, double* C, long ldc,
                                 int rows, hipStream_t s);
-int vcphip_launch_drgemm(int kind, int m, int n, int k, const double* A, long lda, const double* B,
-                         long ldb, double* C, long ldc, double* C2, int accumulate, hipStream_t s);
-// C = A^T A forms (pidblas::mulltmm / vmulmm), kern_drgemm.hip
-int vcphip_launch_drsyrk(int interval, int k, int n, const double* A, long lda, double* C, long ldc,
-                         hipStream_t s);
+// the products of k = 0 (C2 null: interval results, else the RU and RD ones)
+int vcphip_launch_empty_product(int m, int n, double* C, long ldc, double* C2, hipStream_t s);
 
 // batched verified residual R_p * IA_p - I (kern_drgemm.hip)
 struct VcphipResidProblem {

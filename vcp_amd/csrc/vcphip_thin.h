@@ -186,7 +186,7 @@ struct VcphipThin {
   }
 };
 
-// the chains of the plain products (k_drgemm's: the same operations in the
+// the chains of the plain products (the tiles': the same operations in the
 // same order, so the same bits); round-up mode
 template <bool AI, bool BI>
 struct VcphipThinDr {
