@@ -308,8 +308,7 @@ __global__ __launch_bounds__(256) void k_planes(int m, int n, int k, int mpad, i
 // The k-slices of a (4 RPL) x 64 tile in LDS and their loads: a stage is BKS
 // k of A's rows, then of B's columns, elements of AE / BE doubles.  A
 // wave-wide load moves 1 KB: 1024 / (row bytes) k-rows; the workgroup's four
-// waves take the stage's 1 KB pieces in turn, G each (a piece past the last
-// repeats the last one).  Two stages: the next one's loads are in flight
+// waves take the stage's 1 KB pieces in turn, G each.  Two stages: the next one's loads are in flight
 // under the multiply-adds of the current one.  8 k for 64-row tiles, so that
 // three workgroups' stages fit a CU; 16 k for 32-row ones, whose 8 k take
 // about a load's latency.  (Three or four stages of 8 k measured 0 - 3% slower
@@ -319,8 +318,8 @@ struct PlaneStage {
   static constexpr int BKS = RPL == 16 ? 8 : 16, NST = 2;
   static constexpr int ROWS = 4 * RPL, ARB = ROWS * AE * 8, BRB = 64 * BE * 8;   // bytes of a k-row
   static constexpr int ABYTES = BKS * ARB, BBYTES = BKS * BRB, BYTES = ABYTES + BBYTES;
-  static constexpr int NA = ABYTES / 1024, NB = BBYTES / 1024, G = (NA + NB + 3) / 4;
-  static_assert(ABYTES % 1024 == 0 && BBYTES % 1024 == 0 && 16 % BKS == 0, "stage shape");
+  static constexpr int NA = ABYTES / 1024, NB = BBYTES / 1024, G = (NA + NB) / 4;
+  static_assert(ABYTES % 4096 == 0 && BBYTES % 4096 == 0 && 16 % BKS == 0, "stage shape");
   const char *a, *b;
   long lda, ldb;   // bytes of a k-row of the planes
   uint32_t lds;
@@ -340,9 +339,8 @@ struct PlaneStage {
     const char* gb = b + (long)t * BKS * ldb;
 #pragma unroll
     for (int q = 0; q < G; ++q) {
-      int c = 4 * q + w;   // wave-uniform
-      if (c > NA + NB - 1) c = NA + NB - 1;
-      if (c < NA) vcphip_lds_dma16(ga + (long)c * (1024 / ARB) * lda, d + (uint32_t)c * 1024);
+      const int c = 4 * q + w;   // wave-uniform; the four waves' pieces are all A's or all B's
+      if (4 * q < NA) vcphip_lds_dma16(ga + (long)c * (1024 / ARB) * lda, d + (uint32_t)c * 1024);
       else vcphip_lds_dma16(gb + (long)(c - NA) * (1024 / BRB) * ldb, d + (uint32_t)c * 1024);
     }
   }
@@ -424,13 +422,47 @@ struct PointBlock {
   }
 };
 
+// The same for a block of interval results: a lane holds the pairs v(0) ..
+// v(RPL - 1) of its column, written D pairs at a time.  2048 x 2048 x 16, a pair
+// per lane and column against through LDS: interval x interval 24.1 against 15.8
+// us (three contexts in turn; 32 against 23 one), 1500 x 1500 x 100 39.2 against
+// 37.7 (55 against 51).
+template <int RPL, int D>
+struct IntervalBlock {
+  static constexpr int R = 2 * RPL, NC = D / R, T = D / 64;
+  static VCPHIP_DEVINL int slot(int c, int r) { return c * R + (r ^ (c & (R - 1))); }
+  template <class F>
+  static VCPHIP_DEVINL void store(double2* L, const F& v, int lane, double* __restrict__ X, long ldx, int row0, int col0,
+                                  int m, int n) {
+    const int lc = lane & 31, h = lane >> 5, r = lane % R;
+#pragma unroll
+    for (int c0 = 0; c0 < 32; c0 += NC) {
+      if (col0 + c0 >= n) break;   // wave-uniform
+      if (lc / NC == c0 / NC) {
+#pragma unroll
+        for (int i = 0; i < RPL; ++i) L[slot(lc % NC, h * RPL + i)] = v(i);
+      }
+      vcphip_wave_sync();
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        const int c = lane / R + 64 / R * t;
+        if (row0 + r < m && col0 + c0 + c < n)
+          *reinterpret_cast<double2*>(X + 2 * (row0 + r + ldx * (col0 + c0 + c))) = L[slot(c, r)];
+      }
+      vcphip_wave_sync();
+    }
+  }
+};
+
 // Tiles of 4 RPL x 64 outputs, four waves of 2 RPL rows x 32 columns, RPL
 // outputs of one column per lane (vcphip_dpp.h): RPL = 16 (64 rows) for grids
 // that fill the device, RPL = 8 (32 rows) for small ones.  Bound by the FP64
 // multiply-adds, at n = 4096 by the clock that they leave (61 TFLOP/s is 0.93
-// of the rate at 2.0 GHz).  Interval x interval, planes included, against 4 x 4
-// outputs per lane read from LDS: n = 1024 205 -> 203 us, 2048 1432 -> 1153,
-// 4096 11.0 -> 9.1 ms; point x interval at 4096 7.5 -> 6.5 - 7.2 ms.
+// of the rate at 2.0 GHz).  A wave whose block is all padding keeps the loads
+// and barriers in a loop of its own (20000 x 32 x 2000 548 against 502 us).
+// Interval x interval, planes included, against 4 x 4 outputs per lane read
+// from LDS: n = 1024 205 -> 161 us, 2048 1432 -> 1107, 4096 11.0 -> 9.1 ms;
+// point x interval at 2048 981 -> 817 us, at 4096 7.5 -> 6.5 - 7.2 ms.
 template <bool AI, bool BI, int RPL>
 __global__ __launch_bounds__(NT, RPL == 16 ? ((AI && BI) ? 3 : 4) : 4)
 void k_drgemm_planes(int m, int n, int mpad, int npad, int kpad, const double* __restrict__ PA,
@@ -448,10 +480,9 @@ void k_drgemm_planes(int m, int n, int mpad, int npad, int kpad, const double* _
   const int row0 = tm * Stage::ROWS, col0 = tn * 64;
   const Stage st(PA, mpad, row0, PB, npad, col0, sL);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  // this lane's outputs: rows orow .. orow + RPL - 1 of column ocol; lane i
-  // of its DPP row of 16 holds A's row orow + i
+  // this lane's outputs: rows lrow .. lrow + RPL - 1 of column lcol of the tile;
+  // lane i of its DPP row of 16 holds A's row lrow + i
   const int lrow = (w & 1) * 2 * RPL + (lane >> 5) * RPL, lcol = (w >> 1) * 32 + (lane & 31);
-  const int orow = row0 + lrow, ocol = col0 + lcol;
   const int aoff = (lrow + (lane & (RPL - 1))) * AE * 8, boff = Stage::ABYTES + lcol * BE * 8;
 
   double up[RPL], dn[RPL], r1[RPL], r2[RPL];
@@ -463,7 +494,6 @@ void k_drgemm_planes(int m, int n, int mpad, int npad, int kpad, const double* _
     r2[i] = 0.0;
   }
   const int wrow = row0 + (w & 1) * 2 * RPL, wcol = col0 + (w >> 1) * 32;   // the wave's block
-  const bool work = __builtin_amdgcn_readfirstlane(wrow < m && wcol < n);   // else it only loads and waits
   const int nt = kpad / Stage::BKS;
   st.issue(0);
   if (!AI && !BI && accumulate) {
@@ -476,9 +506,13 @@ void k_drgemm_planes(int m, int n, int mpad, int npad, int kpad, const double* _
 #pragma unroll
     for (int i = 0; i < RPL; ++i) dn[i] = -dn[i];
   }
+  if (__builtin_amdgcn_readfirstlane(wrow >= m || wcol >= n)) {   // a block of padding: load and keep the barriers
+    for (int t = 0; t < nt; ++t) st.next(t, nt);
+    __syncthreads();
+    return;
+  }
   for (int t = 0; t < nt; ++t) {
     st.next(t, nt);
-    if (!work) continue;
     const char* s0 = sL + (t % Stage::NST) * Stage::BYTES;
     auto rd = [&](int kk, double2& a, double2& b) {
       if (AI) a = *reinterpret_cast<const double2*>(s0 + aoff + kk * Stage::ARB);
@@ -491,25 +525,25 @@ void k_drgemm_planes(int m, int n, int mpad, int npad, int kpad, const double* _
     });
   }
 
-  if (!AI && !BI) {
-    __syncthreads();   // every wave has read the last stage
-    if (!work) return;
-    double2* L = reinterpret_cast<double2*>(sL) + 256 * w;
-    PointBlock<RPL, 512>::store(L, up, lane, C, ldc, wrow, wcol, m, n);
+  __syncthreads();   // every wave has read the last stage
+  // the wave's own quarter of the stages takes D = 2^n pairs (or pairs of rows)
+  constexpr int D = Stage::NST * Stage::BYTES / 64 >= 512 ? 512 : 256;
+  double2* L = reinterpret_cast<double2*>(sL) + D * w;
+  if (AI || BI) {
+    IntervalBlock<RPL, D>::store(
+        L,
+        [&](int i) {
+          const double tt = II ? r1[i] + r2[i] : r1[i];   // temp (:283, :129, :185)
+          const double hi = up[i] + tt;                   // uC += temp, RU (:284)
+          const double nlo = dn[i] + tt;                  // lC -= temp, RD = -(RU(-lC + t)) (:285-286)
+          return make_double2(-nlo, hi);
+        },
+        lane, C, ldc, wrow, wcol, m, n);
+  } else {
+    PointBlock<RPL, 2 * D>::store(L, up, lane, C, ldc, wrow, wcol, m, n);
 #pragma unroll
     for (int i = 0; i < RPL; ++i) dn[i] = -dn[i];
-    PointBlock<RPL, 512>::store(L, dn, lane, C2, ldc, wrow, wcol, m, n);
-    return;
-  }
-  if (ocol >= n) return;
-#pragma unroll
-  for (int i = 0; i < RPL; ++i) {
-    const int r = orow + i;
-    if (r >= m) break;
-    const double tt = II ? r1[i] + r2[i] : r1[i];   // temp (:283, :129, :185)
-    const double hi = up[i] + tt;                   // uC += temp, RU (:284)
-    const double nlo = dn[i] + tt;                  // lC -= temp, RD = -(RU(-lC + t)) (:285-286)
-    *reinterpret_cast<double2*>(C + 2 * (r + ldc * ocol)) = make_double2(-nlo, hi);
+    PointBlock<RPL, 2 * D>::store(L, dn, lane, C2, ldc, wrow, wcol, m, n);
   }
 }
 
