@@ -903,11 +903,14 @@ namespace {
 
 // Tile rows of a plane-fed product.  Both heights keep a wave's multiply-adds
 // at the same LDS reads per k; the 32-row tiles give twice the workgroups, the
-// 64-row ones twice the multiply-adds per read and barrier.  Measured on
-// MI355X (interval x interval / point RU-RD, 32 against 64 rows): n = 512 60
-// against 96 us / 58 against 80, 1024 204 against 203 / 129 against 161, 1536
-// 594 against 631 / 371 against 402, 2048 (4 64-row tiles per CU) 1218 against
-// 1153 / 708 against 689, 3072 4181 against 3900: 32 rows up to 3 per CU.
+// 64-row ones twice the multiply-adds per read and barrier.  Whole products on
+// MI355X, 32 against 64 rows, one context (us): interval x interval, interval x
+// point, point x interval, RU / RD: n = 1024 (one 64-row tile per CU) 163, 129,
+// 122, 97 against 179, 149, 138, 111; 1536 (2.25) 541, 419, 399, 296 against
+// 611, 480, 458, 336; 2000 (4) 1117, 860, 820, 607 against 1075, 841, 796, 586;
+// 3072 3816, 2927, 2771, 2030 against 3665, 2870, 2661, 1948: 32 rows up to 3
+// per CU in every form.  (With other products beside it the 64-row tile is 3 -
+// 6% faster from 1024 on, where the last round of tiles costs nothing.)
 int plane_rows(const vcphip_ctx* c, size_t mpad, size_t npad) {
   if (c->plane_rows) return (int)c->plane_rows;
   const size_t cus = c->num_cu > 0 ? (size_t)c->num_cu : 256;
@@ -916,8 +919,8 @@ int plane_rows(const vcphip_ctx* c, size_t mpad, size_t npad) {
 
 // the same choice for the upper-triangle tiles of A^T A, whose 64-row interval
 // form holds five chains (192 registers, two waves per SIMD, against three
-// waves with 32 rows): n = 1500 775 against 952 us, 3000 (4.4 64-row tiles per
-// CU) 1512 against 1641
+// waves with 32 rows).  Interval, 32 against 64 rows, one context: n = 1500
+// 700 against 913 us, 3000 (4.4 64-row tiles per CU) 2085 against 2309
 int syrk_rows(const vcphip_ctx* c, size_t npad) {
   if (c->plane_rows) return (int)c->plane_rows;
   const size_t cus = c->num_cu > 0 ? (size_t)c->num_cu : 256, nt = npad / 64;
