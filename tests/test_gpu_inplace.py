@@ -72,3 +72,23 @@ def test_result_one_element_into_operand(ctx, shift):
         "igemm_pi_dev")
     ctx.synchronize()
     assert np.array_equal(_read_iv(C[:n], m), O.pidblas_mul_m_im(A, B))
+
+
+@pytest.mark.parametrize("ka", [40, 39])
+def test_row_blocks_of_one_matrix(ka):
+    # B (rows 0 .. k) and C (the rows after them, or from B's last row on) in one matrix's columns
+    m, n, k = 50, 6, 40
+    rng = np.random.default_rng(6)
+    A, B = _wide(rng, m, k), W.wide_exponent_intervals(rng, k, n, rad_exp=-20)
+    ld = 100
+    buf = torch.zeros((n, ld, 2), dtype=torch.float64, device="cuda")
+    buf[:, :k] = _dev_iv(B, k)
+    dA = _dev_pt(A, m)
+    with vcp_amd.Context(0) as c:
+        c.set_param(vcp_amd.PARAM_STAGE_TIMING, 1)
+        torch.cuda.synchronize()
+        C = buf.data_ptr() + 16 * ka
+        _ok(vcp_amd.lib().vcphip_igemm_pi_dev(c.handle, m, n, k, dA.data_ptr(), m, buf.data_ptr(), ld, C, ld), "pi")
+        c.synchronize()
+        assert ("planes" in c.stage_times()) == (ka < k)   # apart: the row-serial form; overlapping: the planes
+    assert np.array_equal(buf[:, ka:ka + m].cpu().numpy().transpose(1, 0, 2), O.pidblas_mul_m_im(A, B))

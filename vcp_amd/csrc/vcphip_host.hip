@@ -957,13 +957,22 @@ bool thin_product(const vcphip_ctx* c, size_t m, size_t n, size_t k, bool bi) {
   return blocks <= (n > 8 ? 8 : 16) * cus || k >= 64;
 }
 
-// the bytes from the first to the last element of a column-major rows x cols
-// matrix (rows, cols > 0) of e doubles per element
+// the bytes of a column-major rows x cols matrix (rows, cols > 0) of e doubles
+// per element
 struct Extent {
   uintptr_t first, last;
+  size_t col, stride;   // bytes of a column, from column to column
   Extent(const double* p, int e, int rows, int ld, int cols)
-      : first((uintptr_t)p), last(first + sizeof(double) * e * ((size_t)(cols - 1) * ld + rows) - 1) {}
-  bool meets(const Extent& o) const { return first <= o.last && o.first <= last; }
+      : first((uintptr_t)p), col(sizeof(double) * e * rows), stride(sizeof(double) * e * ld) {
+    last = first + (size_t)(cols - 1) * stride + col - 1;
+  }
+  bool meets(const Extent& o) const {
+    if (first > o.last || o.first > last) return false;
+    if (stride != o.stride) return true;
+    // row blocks of one larger matrix: apart if the other's columns lie between this one's
+    const size_t d = o.first >= first ? (o.first - first) % stride : (stride - (first - o.first) % stride) % stride;
+    return d < col || d + o.col > stride;
+  }
 };
 
 // A single product of kind VCPHIP_DR_*: the operand planes (midpoint and
