@@ -800,11 +800,11 @@ int vcphip_dd_add_d(int m, int n, const double* d, double* X, long ldx, double* 
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
-// A == nullptr: B alone (A^T A)
+// m = 0: B alone (A^T A)
 int vcphip_dd_stats(const double* A, long lda, int m, int a_lines, int* ea, int* fa, const double* B, long ldb, int n,
                     int* eb, int* fb, int k, int cus, void* scratch, hipStream_t s) {
   const int W = ST_NT / 64;
-  const int na = !A ? 0 : a_lines ? (m + W - 1) / W : (m + ST_ROWS - 1) / ST_ROWS, nb = (n + W - 1) / W;
+  const int na = a_lines ? (m + W - 1) / W : (m + ST_ROWS - 1) / ST_ROWS, nb = (n + W - 1) / W;
   if (na + nb <= 0) return 0;
   int nsplit, kper;
   vcphip_stats_split(a_lines ? 0 : na, k, cus, nsplit, kper);
@@ -818,7 +818,7 @@ int vcphip_dd_stats(const double* A, long lda, int m, int a_lines, int* ea, int*
 int vcphip_dd_split(const double* A, long lda, int m, int mpad, int a_cols, const int* ea, const int* fa, int8_t* pa,
                     const double* B, long ldb, int n, int npad, const int* eb, const int* fb, int8_t* pb, int k,
                     int kpad, const VcphipOzParams& P, hipStream_t s) {
-  const long na = A ? (long)(mpad / 16) * (kpad / 64) : 0, nb = (long)(npad / 16) * (kpad / 64);
+  const long na = m > 0 ? (long)(mpad / 16) * (kpad / 64) : 0, nb = (long)(npad / 16) * (kpad / 64);
   if (na + nb > 0x7FFFFFFFL) return -7;
   switch (P.nmod) {
 #define VCPHIP_DD_SPLIT(NN)                                                                                        \

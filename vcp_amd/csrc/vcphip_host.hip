@@ -1126,11 +1126,11 @@ static int dd_gemm_dev(vcphip_ctx* c, bool tn, int m, int n, int k, const double
   int* eb = fa + m;
   int* fb = eb + n;
   StageTimer T(c);
-  const double* Aop = tn ? nullptr : A;   // A^T A: the columns of B = A serve both sides
-  if ((rc = check_launch(vcphip_dd_stats(Aop, lda, m, ta ? 1 : 0, ea, fa, B, ldb, n, eb, fb, k, c->num_cu, pa, c->stream))))
+  const int ma = tn ? 0 : m;   // A^T A: the columns of B = A serve both sides
+  if ((rc = check_launch(vcphip_dd_stats(A, lda, ma, ta ? 1 : 0, ea, fa, B, ldb, n, eb, fb, k, c->num_cu, pa, c->stream))))
     return rc;
   T.mark("stats");
-  if ((rc = check_launch(vcphip_dd_split(Aop, lda, m, mpad, ta ? 1 : 0, ea, fa, (int8_t*)pa, B, ldb, n, npad, eb, fb,
+  if ((rc = check_launch(vcphip_dd_split(A, lda, ma, mpad, ta ? 1 : 0, ea, fa, (int8_t*)pa, B, ldb, n, npad, eb, fb,
                                          (int8_t*)pb, k, kpad, P, c->stream))))
     return rc;
   T.mark("split");

@@ -210,7 +210,7 @@ int vcphip_oz_recon(int m, int n, int k, int mpad, int npad, const VcphipOzParam
 // ---- double-double product, Ozaki scheme II (kern_dd.hip) -------------------
 // rows of A (m x k; its columns if a_lines / a_cols: A^T with A k x m) and
 // columns of B (k x n): e with max |hi|+|lo| < 2^e; flags 1: zero, 2: not
-// finite; then the residue planes.  A == nullptr: B alone.  scratch: 2 m nsplit
+// finite; then the residue planes.  m = 0: B alone.  scratch: 2 m nsplit
 // doubles for rows split over k (vcphip_stats_split)
 int vcphip_dd_stats(const double* A, long lda, int m, int a_lines, int* ea, int* fa, const double* B, long ldb, int n,
                     int* eb, int* fb, int k, int cus, void* scratch, hipStream_t s);
