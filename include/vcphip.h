@@ -436,7 +436,9 @@ int vcphip_tune_igemm_batched_dev(vcphip_ctx* ctx, int count, const int* m, cons
                                   double* padded);
 /* Writes / reads the context's tuning table (text: a "vcphip-tune 2" line,
  * then "igemm|ddgemm lm ln lk variant nmod radius" and "residual per_cu"
- * lines; version 1 tables, without the radius field, still load). */
+ * lines; version 1 tables, without the radius field, still load).  Lines of
+ * variant 7 end in 128, the columns of its tiles; without it they load as
+ * variant 10, the 128 x 256 tiles that 7 stood for in older tables. */
 int vcphip_tune_save(vcphip_ctx* ctx, const char* path);
 int vcphip_tune_load(vcphip_ctx* ctx, const char* path);
 

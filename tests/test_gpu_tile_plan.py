@@ -46,6 +46,22 @@ def test_tuner_finds_the_small_tile(ctx, tmp_path):
         assert c2.ozaki_plan(m, n, k)["variant"] == v
 
 
+@pytest.mark.parametrize("line,variant", [("igemm 11 11 11 7 16 1", 10), ("igemm 11 11 11 7 16 1 128", 7),
+                                          ("igemm 11 11 11 7 16 1 256", 10), ("igemm 11 11 11 9 16 1", 9),
+                                          ("igemm 11 11 11 7 16", 10)])
+def test_tables_of_the_older_seven(ctx, tmp_path, line, variant):
+    # 7 stood for 128 x 256 tiles, which are variant 10's, before it was the 128 x 128 tile
+    path = tmp_path / "tune.txt"
+    path.write_text("vcphip-tune %d\n%s\n" % (1 if len(line.split()) == 6 else 2, line))
+    ctx.tune_load(str(path))
+    assert ctx.ozaki_plan(2000, 2000, 2000)["variant"] == variant
+    again = tmp_path / "again.txt"
+    ctx.tune_save(str(again))
+    with vcp_amd.Context(0) as c2:
+        c2.tune_load(str(again))
+        assert c2.ozaki_plan(2000, 2000, 2000)["variant"] == variant
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 1, 1), (130, 257, 65), (300, 511, 200)])
 def test_set_small_tile_bits(ctx, m, n, k):
     rng = np.random.default_rng(m + n + k)

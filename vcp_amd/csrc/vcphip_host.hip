@@ -1016,7 +1016,7 @@ int planes_product(vcphip_ctx* c, int kind, int m, int n, int k, const double* A
   return rc;
 }
 
-// A^T A (mulltmm / vmulmm) from the planes of A; k = 0 takes the tile kernel
+// A^T A (mulltmm / vmulmm) from the planes of A; k = 0 is a fill
 int syrk_planes(vcphip_ctx* c, int interval, int k, int n, const double* A, int lda, double* C, int ldc) {
   StageTimer T(c);
   if (k == 0) {
@@ -3408,8 +3408,8 @@ extern "C" int vcphip_tune_save(vcphip_ctx* c, const char* path) {
   if (!f) return VCPHIP_ERR_ARGUMENT;
   fprintf(f, "vcphip-tune 2\n");
   for (const auto& t : c->tune)
-    fprintf(f, "%s %d %d %d %d %d %d\n", t.kind == TUNE_IGEMM ? "igemm" : "ddgemm", t.lm, t.ln, t.lk, t.variant,
-            t.nmod, t.radius);
+    fprintf(f, "%s %d %d %d %d %d %d%s\n", t.kind == TUNE_IGEMM ? "igemm" : "ddgemm", t.lm, t.ln, t.lk, t.variant,
+            t.nmod, t.radius, t.variant == VCPHIP_OZ_TILE128 ? " 128" : "");
   fprintf(f, "residual %d\n", c->resid_per_cu);
   for (int kind = 0; kind < 2; ++kind)
     for (int l = 0; l < 32; ++l)
@@ -3437,9 +3437,11 @@ extern "C" int vcphip_tune_load(vcphip_ctx* c, const char* path) {
   int rc = VCPHIP_OK;
   while (fgets(line, sizeof line, f)) {
     char kind[32];
-    int lm, ln, lk, v, nm, p, rad = 0;
-    const int nf = sscanf(line, "%31s %d %d %d %d %d %d", kind, &lm, &ln, &lk, &v, &nm, &rad);
-    if (nf == 6 + (version >= 2 ? 1 : 0)) {   // version 1 lines carry no radius scheme
+    int lm, ln, lk, v, nm, p, rad = 0, cols = 0;
+    const int nf = sscanf(line, "%31s %d %d %d %d %d %d %d", kind, &lm, &ln, &lk, &v, &nm, &rad, &cols);
+    if (version == 1 ? nf == 6 : nf >= 7) {   // version 1 lines carry no radius scheme
+      // a 7 without its tile's columns was tuned when 7 had 128 x 256 tiles, as 10 has
+      if (v == VCPHIP_OZ_TILE128 && cols != 128) v = 10;
       const bool iv = strcmp(kind, "igemm") == 0, dd = strcmp(kind, "ddgemm") == 0;
       const bool ok = (iv || dd) && lm >= 0 && lm <= 31 && ln >= 0 && ln <= 31 && lk >= 0 && lk <= 31 &&
                       (v == 0 || (v >= 6 && v <= 18)) && (nm == 0 || (iv && nm >= 8 && nm <= VCPHIP_OZ_MAXMOD_IV) ||
